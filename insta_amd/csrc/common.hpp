@@ -186,9 +186,28 @@ struct TraversalCount {
 // triangle distances, list queries, list entries scanned
 constexpr int kTravCounters = 6;
 
-template <bool kCount>
+// Where a second pass takes what is left (kBudget), a per-lane query gives up
+// after kLeafMost leaves or kListMost list entries, and already after
+// kLeafFew / kListFew when at most kLeafFewLanes / kListFewLanes lanes of its
+// wave are still at it: a wave runs as long as its longest query, and a few long ones
+// (sub-cells around a mesh pole, whose lists hold hundreds of entries or
+// overflow to the BVH; points near the medial axis, which visit most leaves)
+// would otherwise set the kernel's time.  Waves whose lanes all walk the BVH
+// keep walking: their coherent walk is cheaper than a wave per query.  A
+// 301 x 257 frame of the 9,976-triangle head (1.2 M samples): 928 us without
+// budgets, 244 + 36 us (second pass) with; its 512^2 frame 702 -> 572 + 30.
+// Giving up earlier (24 or 12 entries) or with more lanes left costs more in
+// the second pass (410 us, 51 us) than it saves; later, the tail returns.
+constexpr uint32_t kLeafFewLanes = 16, kLeafFew = 8, kLeafMost = 64;
+constexpr uint32_t kListFewLanes = 4, kListFew = 72, kListMost = 192;
+
+INSTA_DEV bool few_lanes_left(uint32_t few) { return (uint32_t)__popcll(__ballot(true)) <= few; }
+
+enum Budget { kNoBudget, kMostBudget, kFewBudget };  // kMostBudget: without the few-lanes rule
+
+template <bool kCount, Budget kBudget = kNoBudget>
 INSTA_DEV Hit bvh_closest_impl(const MeshView& m, V3 p, uint32_t* stack, uint32_t stride, float max_dist_sq,
-                               TraversalCount* tc) {
+                               TraversalCount* tc, bool* unfinished = nullptr) {
     // max_dist_sq (bvh.cuh:48): only triangles closer than this are reported
     float best = max_dist_sq;
     int32_t best_idx = -1;
@@ -196,7 +215,7 @@ INSTA_DEV Hit bvh_closest_impl(const MeshView& m, V3 p, uint32_t* stack, uint32_
     float bound = prune_bound(best);
     const uint32_t shift = 2u * m.k;
     int sp = 0;
-    uint32_t node = 0;
+    uint32_t node = 0, leaves = 0;
     for (;;) {
         while (node < m.leaf_base) {
             if constexpr (kCount) ++tc->inner;
@@ -261,6 +280,13 @@ INSTA_DEV Hit bvh_closest_impl(const MeshView& m, V3 p, uint32_t* stack, uint32_
         bound = prune_bound(best);
         node = pop_live(stack, sp, stride, bound);
         if (node == kNoNode) break;
+        if constexpr (kBudget != kNoBudget) {
+            ++leaves;
+            if (leaves >= kLeafMost || (kBudget == kFewBudget && leaves >= kLeafFew && few_lanes_left(kLeafFewLanes))) {
+                *unfinished = true;
+                break;
+            }
+        }
     }
     Hit h;
     h.idx = best_idx;
@@ -342,12 +368,13 @@ INSTA_DEV bool cell_list_find(const CellListView& cl, V3 p, uint2& hd) {
 // the entry, then of its triangle), so entries go in batches of kListBatch:
 // the batch's triangles are loaded together, with the next batch's entry
 // words already in flight, then tested in order; loads past the stopping
-// entry are wasted, never used.
-constexpr uint32_t kListBatch = 3;
+// entry are wasted, never used.  (Batches of 2 at 7 waves per SIMD and of 3
+// at 5 measure the same; of 3 at 6 or more spill.)
+constexpr uint32_t kListBatch = 2;
 
-template <bool kCount>
+template <bool kCount, Budget kBudget = kNoBudget>
 INSTA_DEV Hit list_closest_impl(const MeshView& m, const uint32_t* __restrict__ ent, uint2 hd, V3 p,
-                                TraversalCount* tc) {
+                                TraversalCount* tc, bool* unfinished = nullptr) {
     float best = 3.40282347e38f;
     int32_t best_idx = -1;
     uint32_t best_orig = 0xffffffffu;
@@ -360,6 +387,12 @@ INSTA_DEV Hit list_closest_impl(const MeshView& m, const uint32_t* __restrict__ 
 #pragma unroll
     for (uint32_t j = 0; j < kListBatch; ++j) wn[j] = e[min(j, n - 1u)];
     for (uint32_t k = 0; k < n && !done; k += kListBatch) {
+        if constexpr (kBudget != kNoBudget) {
+            if (k >= kListMost || (kBudget == kFewBudget && k >= kListFew && few_lanes_left(kListFewLanes))) {
+                *unfinished = true;
+                break;
+            }
+        }
         uint32_t w[kListBatch];
         float4 R[kListBatch][3];
 #pragma unroll
@@ -411,17 +444,252 @@ INSTA_DEV Hit list_closest_impl(const MeshView& m, const uint32_t* __restrict__ 
 
 // Nearest triangle of a point: its sub-cell's list when there is one, else
 // the BVH (same result).
-template <bool kCount>
+template <bool kCount, Budget kBudget = kNoBudget>
 INSTA_DEV Hit closest_impl(const MeshView& m, const CellListView& cl, V3 p, uint32_t* stack, uint32_t stride,
-                           TraversalCount* tc) {
+                           TraversalCount* tc, bool* unfinished = nullptr) {
     uint2 hd;
     const bool in_box = p.x >= 0.0f && p.x <= 1.0f && p.y >= 0.0f && p.y <= 1.0f && p.z >= 0.0f && p.z <= 1.0f;
-    if (in_box && cell_list_find(cl, p, hd)) return list_closest_impl<kCount>(m, cl.ent, hd, p, tc);
-    return bvh_closest_impl<kCount>(m, p, stack, stride, 3.40282347e38f, tc);
+    if (in_box && cell_list_find(cl, p, hd)) return list_closest_impl<kCount, kBudget>(m, cl.ent, hd, p, tc, unfinished);
+    return bvh_closest_impl<kCount, kBudget>(m, p, stack, stride, 3.40282347e38f, tc, unfinished);
 }
 
 INSTA_DEV Hit closest(const MeshView& m, const CellListView& cl, V3 p, uint32_t* stack, uint32_t stride) {
     return closest_impl<false>(m, cl, p, stack, stride, nullptr);
+}
+
+// ---------------------------------------------------------------------------
+// Group queries: kGroup consecutive lanes answer one query together, for the
+// same result under the same (dist_sq, original id) order and prune margin.
+// A list's entries, a node's four children and a leaf's triangles are tested
+// side by side, so a query's chain of dependent loads is up to kGroup times
+// shorter and queries of different length share a wave with only
+// 64 / kGroup - 1 others.  Every lane of a group holds the same query and ends
+// with the same Hit.  For points in no particular order (the geometry entry
+// points) this takes 200,000 points anywhere in the cube from 956 to 582 us
+// and 100,000 near the skin from 209 to 88 us on the 9,976-triangle head; for
+// the samples of neighbouring rays, whose lanes walk together, one lane per
+// query is faster (1.95 against 2.8 ms per 18 M samples).
+// ---------------------------------------------------------------------------
+constexpr uint32_t kGroup = 8;
+
+template <int CTRL>
+INSTA_DEV uint32_t dpp(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, CTRL, 0xf, 0xf, false);
+}
+// smallest value over a group (as unsigned integers: also the order of
+// non-negative floats' bits), in every lane: exchanges within quads (xor 1,
+// xor 2), then with the other quad of eight lanes (half-row mirror)
+INSTA_DEV uint32_t group_min(uint32_t v) {
+    v = min(v, dpp<0xB1>(v));
+    v = min(v, dpp<0x4E>(v));
+    return min(v, dpp<0x141>(v));
+}
+// the group's bits of a wave ballot
+INSTA_DEV uint32_t group_ballot(bool b) {
+    const uint64_t w = __ballot(b);
+    return (uint32_t)(w >> (threadIdx.x & 63u & ~(kGroup - 1u))) & ((1u << kGroup) - 1u);
+}
+
+struct GroupBest {
+    uint32_t dist = 0x7f7fffffu;    // bits of the squared distance (starts at the largest float)
+    uint32_t key = 0xffffffffu;     // original id << 16 | BVH-order index (both < 2^14)
+    float bound = prune_bound(3.40282347e38f);
+    // this lane's candidate (dist 0xffffffff: none) into the group's best
+    INSTA_DEV void take(uint32_t d, uint32_t k) {
+        const uint32_t dm = group_min(d);
+        if (dm > dist) return;
+        const uint32_t km = group_min(d == dm ? k : 0xffffffffu);
+        if (dm < dist || km < key) {
+            dist = dm;
+            key = km;
+            bound = prune_bound(__uint_as_float(dm));
+        }
+    }
+    INSTA_DEV Hit hit() const {
+        Hit h;
+        const bool none = key == 0xffffffffu;
+        h.idx = none ? -1 : (int32_t)(key & 0xffffu);
+        h.orig = none ? 0xffffffffu : key >> 16;
+        h.dist_sq = none ? 0.0f : __uint_as_float(dist);
+        return h;
+    }
+};
+
+// exact squared distance to triangle t (bits) when its box (and, with kPlane,
+// its plane, as in list_closest_impl) lies within the bound, else 0xffffffff
+template <bool kPlane>
+INSTA_DEV uint32_t triangle_candidate(const MeshView& m, uint32_t t, V3 p, float bound, uint32_t& key) {
+    const float4 r0 = m.btris[3 * t + 0], r1 = m.btris[3 * t + 1], r2 = m.btris[3 * t + 2];
+    const V3 va = v3(r0.x, r0.y, r0.z), vb = v3(r0.w, r1.x, r1.y), vc = v3(r1.z, r1.w, r2.x);
+    const float4 lo = make_float4(fminf(fminf(va.x, vb.x), vc.x), fminf(fminf(va.y, vb.y), vc.y),
+                                  fminf(fminf(va.z, vb.z), vc.z), 0.0f);
+    const float4 hi = make_float4(fmaxf(fmaxf(va.x, vb.x), vc.x), fmaxf(fmaxf(va.y, vb.y), vc.y),
+                                  fmaxf(fmaxf(va.z, vb.z), vc.z), 0.0f);
+    if (box_distance_sq(lo, hi, p) > bound) return 0xffffffffu;
+    if constexpr (kPlane) {
+        const V3 nor = cross(vb - va, va - vc);
+        const float pd = dot(nor, p - va);
+        if (pd * pd > bound * sqnorm(nor) * (1.0f + 0x1p-8f)) return 0xffffffffu;
+    }
+    key = __float_as_uint(r2.y) << 16 | t;
+    return __float_as_uint(tri_distance_sq(va, vb, vc, p));
+}
+
+INSTA_DEV Hit group_list_closest(const MeshView& m, const uint32_t* __restrict__ ent, uint2 hd, V3 p) {
+    const uint32_t gl = threadIdx.x & (kGroup - 1u);
+    const uint32_t n = hd.y & 0xffffu;
+    const uint32_t* e = ent + hd.x;
+    GroupBest b;
+    uint32_t wn = e[min(gl, n - 1u)];
+    for (uint32_t k = 0; k < n; k += kGroup) {
+        const uint32_t w = wn;
+        const bool in = k + gl < n && __uint_as_float(w & 0xffff0000u) <= b.bound;
+        if (group_ballot(in) == 0u) break;  // entries ascend: no later one is within the bound either
+        wn = e[min(k + kGroup + gl, n - 1u)];  // next entries, in flight with this round's triangles
+        uint32_t d = 0xffffffffu, key = 0xffffffffu;
+        if (in) d = triangle_candidate<true>(m, w & 0xffffu, p, b.bound, key);
+        b.take(d, key);
+    }
+    return b.hit();
+}
+
+// `stack`: this group's [stack_depth(k)] uint32 in LDS (entries as in
+// bvh_closest_impl).  A node's four children go to the group's first quad of
+// lanes, a leaf's triangles to all kGroup of them.
+INSTA_DEV Hit group_bvh_closest(const MeshView& m, V3 p, uint32_t* stack) {
+    const uint32_t gl = threadIdx.x & (kGroup - 1u);
+    const uint32_t shift = 2u * m.k;
+    GroupBest b;
+    uint32_t sp = 0, node = 0;
+    for (;;) {
+        while (node < m.leaf_base) {
+            const uint32_t first = 4u * node + 1u, c = gl & 3u;
+            const float d = box_distance_sq(m.nodes[2 * (first + c)], m.nodes[2 * (first + c) + 1], p);
+            const bool live = gl < 4u && d <= b.bound;
+            const uint32_t bits = live ? __float_as_uint(d) : 0xffffffffu;
+            // nearer survivors (ties by child); a quad's lanes see each other's keys
+            uint32_t rank = 0;
+            const uint32_t o1 = dpp<0xB1>(bits), o2 = dpp<0x4E>(bits), o3 = dpp<0x1B>(bits);
+            rank += o1 < bits || (o1 == bits && (c ^ 1u) < c) ? 1u : 0u;
+            rank += o2 < bits || (o2 == bits && (c ^ 2u) < c) ? 1u : 0u;
+            rank += o3 < bits || (o3 == bits && (c ^ 3u) < c) ? 1u : 0u;
+            const uint32_t n_live = (uint32_t)__popc(group_ballot(live));
+            const uint32_t nearest = group_ballot(live && rank == 0u);
+            if (live && rank) stack[sp + n_live - 1u - rank] = (bits & 0xffff0000u) | (first + c);
+            if (nearest) {
+                sp += n_live - 1u;
+                node = first + (uint32_t)__builtin_ctz(nearest);
+            } else {
+                node = kNoNode;
+                while (sp > 0) {
+                    const uint32_t w = stack[--sp];
+                    if (__uint_as_float(w & 0xffff0000u) <= b.bound) {
+                        node = w & 0xffffu;
+                        break;
+                    }
+                }
+            }
+        }
+        if (node == kNoNode) break;
+        const uint32_t j = node - m.leaf_base;
+        const uint32_t t0 = (uint32_t)(((uint64_t)j * m.nf) >> shift);
+        const uint32_t t1 = (uint32_t)(((uint64_t)(j + 1) * m.nf) >> shift);
+        for (uint32_t t = t0; t < t1; t += kGroup) {
+            uint32_t d = 0xffffffffu, key = 0xffffffffu;
+            if (t + gl < t1) d = triangle_candidate<false>(m, t + gl, p, b.bound, key);
+            b.take(d, key);
+        }
+        node = kNoNode;
+        while (sp > 0) {
+            const uint32_t w = stack[--sp];
+            if (__uint_as_float(w & 0xffff0000u) <= b.bound) {
+                node = w & 0xffffu;
+                break;
+            }
+        }
+        if (node == kNoNode) break;
+    }
+    return b.hit();
+}
+
+// nearest triangle of the group's point (as closest_impl)
+INSTA_DEV Hit group_closest(const MeshView& m, const CellListView& cl, V3 p, uint32_t* stack) {
+    uint2 hd;
+    const bool in_box = p.x >= 0.0f && p.x <= 1.0f && p.y >= 0.0f && p.y <= 1.0f && p.z >= 0.0f && p.z <= 1.0f;
+    if (in_box && cell_list_find(cl, p, hd)) return group_list_closest(m, cl.ent, hd, p);
+    return group_bvh_closest(m, p, stack);
+}
+
+// ---------------------------------------------------------------------------
+// Wave queries: the second pass over the queries a budget left unfinished,
+// one wave each, starting from the first pass's best triangle (so_far, BVH
+// order, -1: none).  A list is read 64 entries a round; without one, all leaves are tested against the bound, 64 boxes a
+// round, and each lane measures its own leaf's triangles.
+// ---------------------------------------------------------------------------
+INSTA_DEV uint32_t wave_min_bits(uint32_t v) {
+    v = group_min(v);
+    v = min(v, dpp<0x140>(v));  // the other eight lanes of the row
+    v = min(v, (uint32_t)__shfl_xor((int)v, 16));
+    return min(v, (uint32_t)__shfl_xor((int)v, 32));
+}
+
+INSTA_DEV Hit wave_closest(const MeshView& m, const CellListView& cl, V3 p, int32_t so_far) {
+    const uint32_t lane = threadIdx.x & 63u;
+    uint32_t dist = 0x7f7fffffu, key = 0xffffffffu;  // this lane's best (as GroupBest)
+    float bound = prune_bound(3.40282347e38f);
+    if (so_far >= 0) {
+        uint32_t k = 0;
+        const uint32_t d = triangle_candidate<false>(m, (uint32_t)so_far, p, bound, k);
+        if (d <= dist) {
+            dist = d;
+            key = k;
+            bound = prune_bound(__uint_as_float(d));
+        }
+    }
+    const bool in_box = p.x >= 0.0f && p.x <= 1.0f && p.y >= 0.0f && p.y <= 1.0f && p.z >= 0.0f && p.z <= 1.0f;
+    uint2 hd;
+    if (in_box && cell_list_find(cl, p, hd)) {
+        const uint32_t n = hd.y & 0xffffu;
+        const uint32_t* e = cl.ent + hd.x;
+        for (uint32_t k = 0; k < n; k += 64u) {
+            const uint32_t w = e[min(k + lane, n - 1u)];
+            const bool in = k + lane < n && __uint_as_float(w & 0xffff0000u) <= bound;
+            if (__ballot(in) == 0ull) break;
+            uint32_t c = 0, d = 0xffffffffu;
+            if (in) d = triangle_candidate<true>(m, w & 0xffffu, p, bound, c);
+            if (d < dist || (d == dist && c < key)) {
+                dist = d;
+                key = c;
+            }
+            bound = prune_bound(__uint_as_float(wave_min_bits(dist)));
+        }
+    } else {
+        const uint32_t shift = 2u * m.k, n_leaves = 1u << shift;
+        for (uint32_t j0 = 0; j0 < n_leaves; j0 += 64u) {
+            const uint32_t j = j0 + lane, node = m.leaf_base + j;
+            if (j < n_leaves && box_distance_sq(m.nodes[2 * node], m.nodes[2 * node + 1], p) <= bound) {
+                const uint32_t t0 = (uint32_t)(((uint64_t)j * m.nf) >> shift);
+                const uint32_t t1 = (uint32_t)(((uint64_t)(j + 1) * m.nf) >> shift);
+                for (uint32_t t = t0; t < t1; ++t) {
+                    uint32_t c = 0;
+                    const uint32_t d = triangle_candidate<false>(m, t, p, bound, c);
+                    if (d < dist || (d == dist && c < key)) {
+                        dist = d;
+                        key = c;
+                        bound = prune_bound(__uint_as_float(d));
+                    }
+                }
+            }
+            bound = prune_bound(__uint_as_float(wave_min_bits(dist)));
+        }
+    }
+    const uint32_t dm = wave_min_bits(dist);
+    const uint32_t km = wave_min_bits(dist == dm ? key : 0xffffffffu);
+    Hit h;
+    h.idx = km == 0xffffffffu ? -1 : (int32_t)(km & 0xffffu);
+    h.orig = km == 0xffffffffu ? 0xffffffffu : km >> 16;
+    h.dist_sq = km == 0xffffffffu ? 0.0f : __uint_as_float(dm);
+    return h;
 }
 
 // Stack entries a query can hold: at most 3 pending siblings per inner level

@@ -211,16 +211,23 @@ insta_status launch_closest(insta_ctx* ctx, uint32_t slot, const float* pts, uin
 insta_status launch_deform_aos(insta_ctx* ctx, float* coords, uint32_t n, uint32_t stride, int32_t frame,
                                hipStream_t stream);
 insta_status launch_deform_soa(insta_ctx* ctx, RenderWS& ws, int32_t frame, const uint32_t* n_dev, uint32_t n_max,
-                               uint32_t* miss_counter, hipStream_t stream);
+                               uint32_t* miss_counter, uint32_t* queue_n, hipStream_t stream);
 // positions [n][3] in place, each through a random frame of 0..n_frames-2
 insta_status launch_deform_positions(insta_ctx* ctx, float* pos, uint32_t n, uint32_t n_frames, const Pcg32& rng,
                                      hipStream_t stream);
+// records (position, frame bits) in place, each through its frame; queue holds
+// up to n entries, *queue_n is 0
+insta_status launch_deform_records(insta_ctx* ctx, float4* rec, uint32_t n, uint2* queue, uint32_t* queue_n,
+                                   hipStream_t stream);
 // samples s_pos (xyz, ray id bits) with ray directions r_d; frame per ray
 // from ray_frame when non-null
-// miss_counter (nullable) counts in-box samples whose query found no triangle
+// miss_counter (nullable) counts in-box samples whose query found no triangle;
+// scratch (one float4 per sample; written by nothing else in the call) and
+// *queue_n = 0 hold the queries' second-pass queue
 insta_status launch_deform_samples(insta_ctx* ctx, int32_t frame, const int32_t* ray_frame, const uint32_t* n_dev,
                                    uint32_t n_max, const float4* s_pos, const float4* r_d, int32_t* s_hit,
-                                   float4* s_cpos, float4* s_cdir, uint32_t* miss_counter, hipStream_t stream);
+                                   float4* s_cpos, float4* s_cdir, uint32_t* miss_counter, float4* scratch,
+                                   uint32_t* queue_n, hipStream_t stream);
 insta_status launch_occupancy(insta_ctx* ctx, uint32_t slot, float threshold, hipStream_t stream);
 // candidate lists (celllist.hip): device buffers, the build over a slot's
 // current linear occupancy bits, and the invalidation when its mesh changes

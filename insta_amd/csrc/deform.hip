@@ -7,12 +7,20 @@
 // frames inverted per sample (include/rta/affine.cuh:45-100), followed by the
 // canonical triangle's (blended) frame.  Directions go through the 3x3 parts
 // and are renormalised.
+#include <algorithm>
+
 #include "context.hpp"
 
 namespace insta {
 namespace {
 
 constexpr uint32_t kDeformThreads = 256;
+// Coordinates of one call go to groups of lanes up to here: 200,000 random
+// points near a skin take 121 us in groups and 252 us one lane each (the
+// 9,976-triangle head; 89 and 101 us, the 2,048-triangle sphere), 1,000,000
+// take 432 and 477 us (352 and 270 us): beyond, the chip is full either way
+// and the groups' idle lanes cost more on the smaller mesh.
+constexpr uint32_t kGroupedCoords = 1u << 18;
 
 struct MeshSet {
     const float4* nodes;
@@ -188,38 +196,41 @@ INSTA_DEV void warp_from_hit(const MeshSet& ms, uint32_t frame, int32_t idx, V3 
     out_d = v3((dc.x + 1.0f) * 0.5f, (dc.y + 1.0f) * 0.5f, (dc.z + 1.0f) * 0.5f);
 }
 
-// Body of `warp` for one sample; false leaves the sample untouched.  A
-// sample in the unit box whose query finds no triangle is counted (the
-// reference prints it and returns, src/core.cu:482-485).
-INSTA_DEV bool warp_one(const MeshSet& ms, uint32_t frame, V3 p, V3 dir_w, V3& out_p, V3& out_d, uint32_t& mask,
-                        uint32_t* stack, uint32_t stride, uint32_t* misses) {
-    if (!in_unit_box(p)) return false;
-    const Hit h = closest(ms.view(frame + 1), ms.cells(frame + 1), p, stack, stride);
-    if (h.idx < 0) {
-        atomicAdd(misses, 1u);
-        return false;
-    }
-    warp_from_hit(ms, frame, h.idx, p, dir_w, out_p, out_d, mask);
-    return true;
-}
-
-// NerfCoordinate samples in place (stride floats per sample)
+// NerfCoordinate samples in place (stride floats per sample), one lane each
+// or, with kGrouped, one group of lanes each (its first lane transforms).  A
+// sample outside the unit box or of an unbuilt frame stays as it is; one in
+// the box whose query finds no triangle is counted (the reference prints it
+// and returns, src/core.cu:482-485).
+template <bool kGrouped>
 __global__ __launch_bounds__(kDeformThreads) void deform_aos_kernel(MeshSet ms, float* __restrict__ coords, uint32_t n,
                                                                     uint32_t stride, int32_t frame_arg,
                                                                     uint32_t n_extra, uint32_t* __restrict__ misses) {
-    extern __shared__ uint32_t stack[];  // [stack_depth(k)][kDeformThreads]
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    // [stack_depth(k)][kDeformThreads], grouped: [kDeformThreads / kGroup][stack_depth(k)]
+    extern __shared__ uint32_t stack[];
+    const uint32_t i = (blockIdx.x * blockDim.x + threadIdx.x) / (kGrouped ? kGroup : 1u);
     if (i >= n) return;
     float* c = coords + (size_t)i * stride;
     const float holder = c[4];
     if (holder < 0.0f) return;
     const uint32_t frame = frame_arg < 0 ? (uint32_t)holder : (uint32_t)frame_arg;
     if (frame >= ms.n_slots - 1 || !ms.built[frame + 1]) return;
+    const V3 p = v3(c[0], c[1], c[2]);
+    if (!in_unit_box(p)) return;
+    int32_t h;
+    if constexpr (kGrouped) {
+        h = group_closest(ms.view(frame + 1), ms.cells(frame + 1), p,
+                          stack + threadIdx.x / kGroup * stack_depth(ms.k)).idx;
+        if ((threadIdx.x & (kGroup - 1u)) != 0) return;
+    } else {
+        h = closest(ms.view(frame + 1), ms.cells(frame + 1), p, stack + threadIdx.x, kDeformThreads).idx;
+    }
+    if (h < 0) {
+        atomicAdd(misses, 1u);
+        return;
+    }
     V3 op, od;
     uint32_t mask = 0;
-    if (!warp_one(ms, frame, v3(c[0], c[1], c[2]), v3(c[8], c[9], c[10]), op, od, mask, stack + threadIdx.x,
-                  kDeformThreads, misses))
-        return;
+    warp_from_hit(ms, frame, h, p, v3(c[8], c[9], c[10]), op, od, mask);
     c[0] = op.x; c[1] = op.y; c[2] = op.z;
     c[8] = od.x; c[9] = od.y; c[10] = od.z;
     if (mask != 7u)
@@ -238,6 +249,8 @@ __global__ __launch_bounds__(kDeformThreads) void deform_aos_kernel(MeshSet ms, 
 //         triangle measured slower: the descent reaches a tight bound on its
 //         first leaf anyway, and chunking samples per lane breaks the
 //         coherence above.)
+//         Queries that exceed a lane's budget (common.hpp) go to a queue and
+//         get a wave each (in deform_apply_kernel).
 //  apply: per sample, the frame transforms of `warp` from the hit; writes
 //         canonical position (+ mask bits) to s_cpos and the warped
 //         direction to s_cdir, whose w selects the extra dims: all 1.0 when
@@ -252,16 +265,23 @@ INSTA_DEV int32_t sample_frame(int32_t frame, const int32_t* __restrict__ ray_fr
     return ray_frame ? ray_frame[__float_as_uint(sp.w)] : frame;
 }
 
+// The second pass's queue of a call holds up to one entry per sample:
+// (sample, best triangle so far); its samples' s_hit is kLongHit.
+constexpr int32_t kLongHit = -2;
+constexpr uint32_t kLongBlocks = 256;  // second pass: four waves per CU beside the first pass's samples
+
 // kCount: also sum the traversal work into counts[4] (queries, inner nodes,
 // leaves, triangles) -- a separate build for measurement runs
 template <bool kCount>
-__global__ __launch_bounds__(kDeformThreads) void deform_hits_kernel(MeshSet ms, int32_t frame,
+__global__ __launch_bounds__(kDeformThreads, 7) void deform_hits_kernel(MeshSet ms, int32_t frame,
                                                                      const int32_t* __restrict__ ray_frame,
                                                                      const uint32_t* __restrict__ n_dev,
                                                                      const float4* __restrict__ s_pos,
                                                                      int32_t* __restrict__ s_hit,
                                                                      unsigned long long* __restrict__ counts,
-                                                                     uint32_t* __restrict__ misses) {
+                                                                     uint32_t* __restrict__ misses,
+                                                                     uint2* __restrict__ queue,
+                                                                     uint32_t* __restrict__ queue_n) {
     extern __shared__ uint32_t stack[];  // [stack_depth(k)][kDeformThreads]
     const uint32_t n = *n_dev;
     TraversalCount tc;
@@ -272,11 +292,15 @@ __global__ __launch_bounds__(kDeformThreads) void deform_hits_kernel(MeshSet ms,
         const int32_t f = sample_frame(frame, ray_frame, sp);
         const bool q = f >= 0 && in_unit_box(p);
         if constexpr (kCount) queries += q ? 1u : 0u;
-        const int32_t h = q ? closest_impl<kCount>(ms.view((uint32_t)f + 1), ms.cells((uint32_t)f + 1), p,
-                                                   stack + threadIdx.x, kDeformThreads, &tc).idx
+        bool rest = false;  // left for the second pass
+        const int32_t h = q ? closest_impl<kCount, kCount ? kNoBudget : kFewBudget>(ms.view((uint32_t)f + 1), ms.cells((uint32_t)f + 1), p,
+                                                            stack + threadIdx.x, kDeformThreads, &tc, &rest).idx
                             : -1;
-        missed += (q && h < 0) ? 1u : 0u;
-        s_hit[i] = h;
+        missed += (q && h < 0 && !rest) ? 1u : 0u;
+        s_hit[i] = rest ? kLongHit : h;
+        if constexpr (!kCount) {
+            if (rest) queue[atomicAdd(queue_n, 1u)] = make_uint2(i, (uint32_t)h);
+        }
     }
     if (misses) {  // one atomic per wave, only when a lane missed
 #pragma unroll
@@ -294,37 +318,86 @@ __global__ __launch_bounds__(kDeformThreads) void deform_hits_kernel(MeshSet ms,
     }
 }
 
-__global__ __launch_bounds__(kDeformThreads) void deform_apply_kernel(MeshSet ms, int32_t frame,
+INSTA_DEV void apply_sample(const MeshSet& ms, int32_t f, int32_t h, float4 sp, float4 rd, uint32_t i,
+                            float4* __restrict__ s_cpos, float4* __restrict__ s_cdir) {
+    const V3 p = xyz(sp);
+    const V3 dir_w = v3((rd.x + 1.0f) * 0.5f, (rd.y + 1.0f) * 0.5f, (rd.z + 1.0f) * 0.5f);
+    V3 op = p, od = dir_w;
+    uint32_t mask = 0;
+    if (h >= 0) warp_from_hit(ms, (uint32_t)f, h, p, dir_w, op, od, mask);
+    const bool frame_values = ms.n_extra && f >= 0 && !(h >= 0 && mask != 7u);
+    const uint32_t sel = frame_values ? (uint32_t)f + 1u : kExtraOnes;
+    s_cpos[i] = make_float4(op.x, op.y, op.z, __uint_as_float(mask));
+    s_cdir[i] = make_float4(od.x, od.y, od.z, __uint_as_float(sel));
+}
+
+// The first long_blocks workgroups answer the queue, one wave per query, and
+// transform its samples; the others transform every sample the first pass
+// answered.  One launch for both: the queue is mostly empty, and a launch of
+// its own costs a small batch 4.5 us.
+__global__ __launch_bounds__(kDeformThreads, 6) void deform_apply_kernel(MeshSet ms, int32_t frame,
                                                                       const int32_t* __restrict__ ray_frame,
                                                                       const uint32_t* __restrict__ n_dev,
                                                                       const float4* __restrict__ s_pos,
                                                                       const float4* __restrict__ r_d,
                                                                       const int32_t* __restrict__ s_hit,
                                                                       float4* __restrict__ s_cpos,
-                                                                      float4* __restrict__ s_cdir) {
+                                                                      float4* __restrict__ s_cdir,
+                                                                      uint32_t long_blocks,
+                                                                      const uint2* __restrict__ queue,
+                                                                      const uint32_t* __restrict__ queue_n,
+                                                                      uint32_t* __restrict__ misses) {
+    if (blockIdx.x < long_blocks) {
+        const uint32_t n = *queue_n;
+        for (uint32_t q = (blockIdx.x * kDeformThreads + threadIdx.x) >> 6; q < n;
+             q += long_blocks * (kDeformThreads / 64u)) {
+            const uint2 e = queue[q];
+            const float4 sp = s_pos[e.x];
+            const int32_t f = sample_frame(frame, ray_frame, sp);
+            const int32_t h = wave_closest(ms.view((uint32_t)f + 1u), ms.cells((uint32_t)f + 1u), xyz(sp),
+                                           (int32_t)e.y).idx;
+            if ((threadIdx.x & 63u) == 0) {
+                if (h < 0 && misses) atomicAdd(misses, 1u);
+                apply_sample(ms, f, h, sp, r_d[__float_as_uint(sp.w)], e.x, s_cpos, s_cdir);
+            }
+        }
+        return;
+    }
     const uint32_t n = *n_dev;
-    for (uint32_t i = blockIdx.x * kDeformThreads + threadIdx.x; i < n; i += gridDim.x * kDeformThreads) {
+    for (uint32_t i = (blockIdx.x - long_blocks) * kDeformThreads + threadIdx.x; i < n;
+         i += (gridDim.x - long_blocks) * kDeformThreads) {
         const float4 sp = s_pos[i];
-        const float4 rd = r_d[__float_as_uint(sp.w)];
-        const V3 p = v3(sp.x, sp.y, sp.z);
-        const V3 dir_w = v3((rd.x + 1.0f) * 0.5f, (rd.y + 1.0f) * 0.5f, (rd.z + 1.0f) * 0.5f);
-        V3 op = p, od = dir_w;
-        uint32_t mask = 0;
         const int32_t f = sample_frame(frame, ray_frame, sp);
         const int32_t h = f >= 0 ? s_hit[i] : -1;
-        if (h >= 0) warp_from_hit(ms, (uint32_t)f, h, p, dir_w, op, od, mask);
-        const bool frame_values = ms.n_extra && f >= 0 && !(h >= 0 && mask != 7u);
-        const uint32_t sel = frame_values ? (uint32_t)f + 1u : kExtraOnes;
-        s_cpos[i] = make_float4(op.x, op.y, op.z, __uint_as_float(mask));
-        s_cdir[i] = make_float4(od.x, od.y, od.z, __uint_as_float(sel));
+        if (h != kLongHit) apply_sample(ms, f, h, sp, r_d[__float_as_uint(sp.w)], i, s_cpos, s_cdir);
     }
+}
+
+// The transform of a position whose nearest triangle is `hit` (no unit-box
+// test, as in the reference).
+INSTA_DEV V3 warp_position(const MeshSet& ms, uint32_t frame, int32_t hit, V3 p) {
+    float W[12], C[12];
+    uint32_t mask;
+    frames_for_hit(ms, frame, hit, p, W, C, mask);
+    return apply_point(C, apply_point(W, p));
+}
+
+INSTA_DEV void apply_record(const MeshSet& ms, float4* __restrict__ rec, uint32_t i, int32_t hit,
+                            uint32_t* __restrict__ misses) {
+    if (hit < 0) {  // src/core.cu:554-557
+        atomicAdd(misses, 1u);
+        return;
+    }
+    const float4 r = rec[i];
+    const V3 c = warp_position(ms, __float_as_uint(r.w), hit, xyz(r));
+    rec[i] = make_float4(c.x, c.y, c.z, r.w);
 }
 
 // warp_random_samples (src/core.cu:528-579): positions (stride 3) of
 // occupancy-grid samples mapped to canonical space through a random posed
 // frame each: the PCG32 stream advanced by i * (n_frames - 1) draws gives
 // frame = floor(u * (n_frames - 1)), so the last frame is never chosen (the
-// reference's own off-by-one, kept).  No unit-box test, as in the reference.
+// reference's own off-by-one, kept).
 __global__ __launch_bounds__(kDeformThreads) void deform_positions_kernel(MeshSet ms, float* __restrict__ pos,
                                                                          uint32_t n, uint32_t n_meshes, Pcg32 rng,
                                                                          uint32_t* __restrict__ misses) {
@@ -339,13 +412,50 @@ __global__ __launch_bounds__(kDeformThreads) void deform_positions_kernel(MeshSe
         atomicAdd(misses, 1u);
         return;
     }
-    float W[12], C[12];
-    uint32_t mask;
-    frames_for_hit(ms, frame, h, p, W, C, mask);
-    const V3 c = apply_point(C, apply_point(W, p));
+    const V3 c = warp_position(ms, frame, h, p);
     pos[3 * i] = c.x;
     pos[3 * i + 1] = c.y;
     pos[3 * i + 2] = c.z;
+}
+
+// The same for the density grid's samples, whose frames are drawn with them
+// (rec.w), ordered by frame and cell so that a wave's walks visit the same
+// nodes and triangles.  Bound by the walk's arithmetic (far points: 35 leaves
+// and 130 exact distances each) over the union of a wave's visits: 1,048,576
+// samples of three 9,976-triangle frames take 2,410 us, in drawing order
+// 3,390 us, and 2,740 us with a group of lanes per sample; without the budget
+// (the second pass takes 170 us) the few samples near the medial axis alone
+// set 4,500 us.
+__global__ __launch_bounds__(kDeformThreads) void deform_records_kernel(MeshSet ms, float4* __restrict__ rec,
+                                                                       uint32_t n, uint32_t* __restrict__ misses,
+                                                                       uint2* __restrict__ queue,
+                                                                       uint32_t* __restrict__ queue_n) {
+    extern __shared__ uint32_t stack[];  // [stack_depth(k)][kDeformThreads]
+    const uint32_t i = blockIdx.x * kDeformThreads + threadIdx.x;
+    if (i >= n) return;
+    const float4 r = rec[i];
+    const uint32_t frame = __float_as_uint(r.w);
+    bool rest = false;
+    const int32_t h = closest_impl<false, kMostBudget>(ms.view(frame + 1), ms.cells(frame + 1), xyz(r),
+                                                       stack + threadIdx.x, kDeformThreads, nullptr, &rest).idx;
+    if (rest)
+        queue[atomicAdd(queue_n, 1u)] = make_uint2(i, (uint32_t)h);
+    else
+        apply_record(ms, rec, i, h, misses);
+}
+
+__global__ __launch_bounds__(kDeformThreads) void deform_records_long_kernel(MeshSet ms, float4* __restrict__ rec,
+                                                                            uint32_t* __restrict__ misses,
+                                                                            const uint2* __restrict__ queue,
+                                                                            const uint32_t* __restrict__ queue_n) {
+    const uint32_t n = *queue_n;
+    for (uint32_t q = (blockIdx.x * kDeformThreads + threadIdx.x) >> 6; q < n; q += gridDim.x * (kDeformThreads / 64u)) {
+        const uint2 e = queue[q];
+        const float4 r = rec[e.x];
+        const uint32_t frame = __float_as_uint(r.w);
+        const int32_t h = wave_closest(ms.view(frame + 1), ms.cells(frame + 1), xyz(r), (int32_t)e.y).idx;
+        if ((threadIdx.x & 63u) == 0) apply_record(ms, rec, e.x, h, misses);
+    }
 }
 
 uint32_t blocks_for(uint64_t items) {
@@ -359,30 +469,43 @@ insta_status launch_deform_aos(insta_ctx* ctx, float* coords, uint32_t n, uint32
                                hipStream_t stream) {
     if (n == 0) return INSTA_OK;
     const size_t shmem = (size_t)stack_depth(ctx->bvh_k) * kDeformThreads * sizeof(uint32_t);
-    hipLaunchKernelGGL(deform_aos_kernel, dim3((n + kDeformThreads - 1) / kDeformThreads), dim3(kDeformThreads), shmem,
-                       stream, mesh_set(ctx, ctx->d_built), coords, n, stride, frame, ctx->cfg.n_extra_dims,
-                       ctx->d_misses);
+    const MeshSet ms = mesh_set(ctx, ctx->d_built);
+    if (n <= kGroupedCoords)
+        hipLaunchKernelGGL(deform_aos_kernel<true>, dim3((n * kGroup + kDeformThreads - 1) / kDeformThreads),
+                           dim3(kDeformThreads), shmem / kGroup, stream, ms, coords, n, stride, frame,
+                           ctx->cfg.n_extra_dims, ctx->d_misses);
+    else
+        hipLaunchKernelGGL(deform_aos_kernel<false>, dim3((n + kDeformThreads - 1) / kDeformThreads),
+                           dim3(kDeformThreads), shmem, stream, ms, coords, n, stride, frame, ctx->cfg.n_extra_dims,
+                           ctx->d_misses);
     INSTA_HIP(hipGetLastError());
     return INSTA_OK;
 }
 
 insta_status launch_deform_samples(insta_ctx* ctx, int32_t frame, const int32_t* ray_frame, const uint32_t* n_dev,
                                    uint32_t n_max, const float4* s_pos, const float4* r_d, int32_t* s_hit,
-                                   float4* s_cpos, float4* s_cdir, uint32_t* miss_counter, hipStream_t stream) {
+                                   float4* s_cpos, float4* s_cdir, uint32_t* miss_counter, float4* scratch,
+                                   uint32_t* queue_n, hipStream_t stream) {
     if (n_max == 0) return INSTA_OK;
     const MeshSet ms = mesh_set(ctx, ctx->d_built);
+    uint2* queue = reinterpret_cast<uint2*>(scratch);
+    uint32_t long_blocks = 0;
     if (frame >= 0 || ray_frame) {
         const size_t shmem = (size_t)stack_depth(ctx->bvh_k) * kDeformThreads * sizeof(uint32_t);
-        if (ctx->d_trav_counts)
+        if (ctx->d_trav_counts) {
             hipLaunchKernelGGL(deform_hits_kernel<true>, dim3(blocks_for(n_max)), dim3(kDeformThreads), shmem, stream,
-                               ms, frame, ray_frame, n_dev, s_pos, s_hit, ctx->d_trav_counts, miss_counter);
-        else
+                               ms, frame, ray_frame, n_dev, s_pos, s_hit, ctx->d_trav_counts, miss_counter, nullptr,
+                               nullptr);
+        } else {
             hipLaunchKernelGGL(deform_hits_kernel<false>, dim3(blocks_for(n_max)), dim3(kDeformThreads), shmem,
-                               stream, ms, frame, ray_frame, n_dev, s_pos, s_hit, nullptr, miss_counter);
+                               stream, ms, frame, ray_frame, n_dev, s_pos, s_hit, nullptr, miss_counter, queue, queue_n);
+            long_blocks = kLongBlocks;
+        }
         INSTA_HIP(hipGetLastError());
     }
-    hipLaunchKernelGGL(deform_apply_kernel, dim3(blocks_for(n_max)), dim3(kDeformThreads), 0, stream, ms, frame,
-                       ray_frame, n_dev, s_pos, r_d, s_hit, s_cpos, s_cdir);
+    hipLaunchKernelGGL(deform_apply_kernel, dim3(long_blocks + blocks_for(n_max)), dim3(kDeformThreads), 0, stream, ms,
+                       frame, ray_frame, n_dev, s_pos, r_d, s_hit, s_cpos, s_cdir, long_blocks, queue, queue_n,
+                       miss_counter);
     INSTA_HIP(hipGetLastError());
     return INSTA_OK;
 }
@@ -397,10 +520,23 @@ insta_status launch_deform_positions(insta_ctx* ctx, float* pos, uint32_t n, uin
     return INSTA_OK;
 }
 
+insta_status launch_deform_records(insta_ctx* ctx, float4* rec, uint32_t n, uint2* queue, uint32_t* queue_n,
+                                   hipStream_t stream) {
+    if (n == 0) return INSTA_OK;
+    const size_t shmem = (size_t)stack_depth(ctx->bvh_k) * kDeformThreads * sizeof(uint32_t);
+    const MeshSet ms = mesh_set(ctx, ctx->d_built);
+    hipLaunchKernelGGL(deform_records_kernel, dim3((n + kDeformThreads - 1) / kDeformThreads), dim3(kDeformThreads),
+                       shmem, stream, ms, rec, n, ctx->d_misses, queue, queue_n);
+    hipLaunchKernelGGL(deform_records_long_kernel, dim3(kLongBlocks), dim3(kDeformThreads), 0, stream, ms, rec,
+                       ctx->d_misses, queue, queue_n);
+    INSTA_HIP(hipGetLastError());
+    return INSTA_OK;
+}
+
 insta_status launch_deform_soa(insta_ctx* ctx, RenderWS& ws, int32_t frame, const uint32_t* n_dev, uint32_t n_max,
-                               uint32_t* miss_counter, hipStream_t stream) {
+                               uint32_t* miss_counter, uint32_t* queue_n, hipStream_t stream) {
     return launch_deform_samples(ctx, frame, nullptr, n_dev, n_max, ws.s_pos, ws.r_d, ws.s_hit, ws.s_cpos, ws.s_cdir,
-                                 miss_counter, stream);
+                                 miss_counter, ws.s_out, queue_n, stream);
 }
 
 }  // namespace insta

@@ -6,7 +6,11 @@
 //             10 probes of a multiplicative-hash cell sequence), a random
 //             position inside each cell; both sets read the same PCG32 state,
 //             which then advances by 2^32 (pcg32's default jump)
-//   warp      each position to canonical space through a random posed frame
+//   order     counting sort of the samples by (posed frame, Morton cell): the
+//             cells come from a multiplicative sequence and the frames from a
+//             random stream, so in drawing order a wave's 64 nearest-triangle
+//             walks would share nothing
+//   warp      each position to canonical space through its random posed frame
 //             (warp_random_samples, src/core.cu:528-579)
 //   splat     density MLP at the canonical position (extra dims all 1.0, as
 //             extract_expressions_random writes, nerf_network.h:107-127),
@@ -20,6 +24,8 @@
 //             2863-2878, 585-609), written into an occupancy slot
 // The mean is a two-stage fixed-order reduction, so the bitfield is a
 // deterministic function of the grid.
+#include <algorithm>
+
 #include "context.hpp"
 #include "encoding.hpp"
 
@@ -28,8 +34,12 @@ namespace insta {
 struct DensityGridState {
     float* grid = nullptr;      // [G^3] Morton order
     float* tmp = nullptr;       // [G^3] this update's splats
-    float* pos = nullptr;       // [cap][3]
-    uint32_t* idx = nullptr;    // [cap]
+    float4* rec = nullptr;      // [cap] drawn samples: position, posed frame (bits)
+    uint32_t* idx = nullptr;    // [cap] their cells
+    float4* srec = nullptr;     // [cap] the samples by (frame, cell)
+    uint32_t* sidx = nullptr;   // [cap]
+    uint32_t* bins = nullptr;   // [kMaxBins] samples per bin, then each bin's next slot
+    uint32_t* bin_sums = nullptr;  // [kMaxBins / kScanBins]
     float* partial = nullptr;   // [G^3 / kReduce] block sums
     float* mean = nullptr;      // [1]
     float* h_mean = nullptr;    // pinned mirror
@@ -43,6 +53,11 @@ namespace {
 
 constexpr uint32_t kThreads = 256;
 constexpr uint32_t kReduce = 1024;    // cells per first-stage block
+// Sort bins: at most 2^20 (and about one per sample), the frames times equal
+// runs of the Morton order.  At 2^20 samples of three frames a bin is a box
+// of 2 x 2 x 2 cells of the 128^3 grid.
+constexpr uint32_t kMaxBins = 1u << 20;
+constexpr uint32_t kScanBins = 1024;  // bins per workgroup of the scan
 constexpr float kMinOpticalThickness = 0.01f;  // NERF_MIN_OPTICAL_THICKNESS (testbed_nerf.cu:63)
 
 __global__ void dg_fill_kernel(float* p, uint32_t n) {
@@ -76,8 +91,13 @@ __global__ void dg_mark_kernel(float* __restrict__ grid, uint32_t G, const Train
     if (clear || (g < 0.0f) != !seen) grid[i] = seen ? 0.0f : -1.0f;
 }
 
+// The sample's posed frame is the warp's draw (warp_random_samples): the
+// stream `frames` advanced by (first + i) * n_meshes gives
+// floor(u * n_meshes), so the last frame is never chosen.
 __global__ void dg_samples_kernel(uint32_t n, uint32_t step, float thresh, uint32_t G, const float* __restrict__ grid,
-                                  Pcg32 rng, float* __restrict__ pos, uint32_t* __restrict__ idx_out) {
+                                  Pcg32 rng, Pcg32 frames, uint32_t first, uint32_t n_meshes, uint32_t bin_shift,
+                                  uint32_t frame_bins, float4* __restrict__ rec, uint32_t* __restrict__ idx_out,
+                                  uint32_t* __restrict__ bins) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const uint32_t cells = G * G * G;
@@ -91,36 +111,142 @@ __global__ void dg_samples_kernel(uint32_t n, uint32_t step, float thresh, uint3
     const uint32_t x = compact3(idx), y = compact3(idx >> 1), z = compact3(idx >> 2);
     const float rx = rng.next_float(), ry = rng.next_float(), rz = rng.next_float();
     const float g = (float)G;
-    pos[3 * i] = (((float)x + rx) / g - 0.5f) * 1.0f + 0.5f;
-    pos[3 * i + 1] = (((float)y + ry) / g - 0.5f) * 1.0f + 0.5f;
-    pos[3 * i + 2] = (((float)z + rz) / g - 0.5f) * 1.0f + 0.5f;
-    idx_out[i] = idx;
+    frames.advance((uint64_t)(first + i) * n_meshes);
+    const uint32_t frame = (uint32_t)(frames.next_float() * (float)n_meshes);
+    rec[first + i] = make_float4((((float)x + rx) / g - 0.5f) * 1.0f + 0.5f, (((float)y + ry) / g - 0.5f) * 1.0f + 0.5f,
+                                 (((float)z + rz) / g - 0.5f) * 1.0f + 0.5f, __uint_as_float(frame));
+    idx_out[first + i] = idx;
+    atomicAdd(bins + frame * frame_bins + (idx >> bin_shift), 1u);
 }
 
-// density MLP output 0 at a canonical position (the FMA chains of the plain
-// inference kernel), optical thickness max-splatted into the sample's cell
-template <int L, int X>
-__global__ __launch_bounds__(128) void dg_splat_kernel(const float* __restrict__ params,
-                                                       const float* __restrict__ table, GridParams gp,
-                                                       const float* __restrict__ pos,
-                                                       const uint32_t* __restrict__ idx, uint32_t n, float dt,
-                                                       float bias, float* __restrict__ tmp) {
-    constexpr int E = 2 * L + X;
-    constexpr int W = 64;
+// sum over the workgroup's kScanBins threads' values, in every thread
+__device__ inline uint32_t block_sum(uint32_t v, uint32_t* s) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+    if ((threadIdx.x & 63u) == 0) s[threadIdx.x >> 6] = v;
+    __syncthreads();
+    uint32_t t = 0;
+    for (uint32_t w = 0; w < kScanBins / 64; ++w) t += s[w];
+    __syncthreads();
+    return t;
+}
+
+__global__ __launch_bounds__(kScanBins) void dg_bin_sums_kernel(const uint32_t* __restrict__ bins, uint32_t n_bins,
+                                                                uint32_t* __restrict__ sums) {
+    __shared__ uint32_t s[kScanBins / 64];
+    const uint32_t i = blockIdx.x * kScanBins + threadIdx.x;
+    const uint32_t t = block_sum(i < n_bins ? bins[i] : 0u, s);
+    if (threadIdx.x == 0) sums[blockIdx.x] = t;
+}
+
+// bins[i] <- samples in the bins before i (at most kScanBins workgroups)
+__global__ __launch_bounds__(kScanBins) void dg_bin_scan_kernel(uint32_t* __restrict__ bins, uint32_t n_bins,
+                                                                const uint32_t* __restrict__ sums) {
+    __shared__ uint32_t s[kScanBins / 64];
+    const uint32_t t = threadIdx.x, lane = t & 63u, wave = t >> 6;
+    const uint32_t i = blockIdx.x * kScanBins + t;
+    uint32_t run = block_sum(t < blockIdx.x ? sums[t] : 0u, s);
+    const uint32_t v = i < n_bins ? bins[i] : 0u;
+    uint32_t incl = v;
+#pragma unroll
+    for (uint32_t o = 1; o < 64u; o <<= 1) {
+        const uint32_t up = __shfl_up(incl, o);
+        if (lane >= o) incl += up;
+    }
+    if (lane == 63u) s[wave] = incl;
+    __syncthreads();
+    for (uint32_t w = 0; w < wave; ++w) run += s[w];
+    if (i < n_bins) bins[i] = run + incl - v;
+}
+
+// the drawn samples into their bins (their order inside a bin varies; every
+// use of a sample is its own)
+__global__ void dg_order_kernel(uint32_t n, uint32_t bin_shift, uint32_t frame_bins, const float4* __restrict__ rec,
+                                const uint32_t* __restrict__ idx, uint32_t* __restrict__ bins,
+                                float4* __restrict__ srec, uint32_t* __restrict__ sidx) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    const V3 x = v3(pos[3 * i], pos[3 * i + 1], pos[3 * i + 2]);
-    float enc[E];
+    const float4 r = rec[i];
+    const uint32_t c = idx[i];
+    const uint32_t slot = atomicAdd(bins + __float_as_uint(r.w) * frame_bins + (c >> bin_shift), 1u);
+    srec[slot] = r;
+    sidx[slot] = c;
+}
+
+// Density logit (output 0 of the density MLP) at canonical positions, optical
+// thickness max-splatted into the sample's cell.  The hidden layer is a
+// contraction over the batch, so it runs on v_mfma_f32_16x16x4f32: phase A,
+// one thread per sample, encodes into LDS; phase B, a wave's 64 samples in
+// four blocks of 16 columns, weights as A operands held in registers (lane l:
+// row l % 16, k l / 16) and the extra dims' columns (all 1.0) as the starting
+// accumulator; the one output row needed is a dot product on the vector ALUs
+// (16 terms per lane, then the four lane groups), not a padded MFMA tile.
+// Bound by the table gathers of phase A: 1,048,576 samples at L = 16, T =
+// 2^19 take 547 us; with one thread per sample running the MLP as FMA
+// chains on scalar weights, and the samples in drawing order, 894 us.
+typedef float dg_f4 __attribute__((ext_vector_type(4)));
+constexpr uint32_t kSplatTile = 256;
+template <int L, int X>
+__global__ __launch_bounds__(kSplatTile) void dg_splat_kernel(const float* __restrict__ params,
+                                                              const float* __restrict__ table, GridParams gp,
+                                                              const float4* __restrict__ pos,
+                                                              const uint32_t* __restrict__ idx, uint32_t n, float dt,
+                                                              float bias, float* __restrict__ tmp) {
+    constexpr int E = 2 * L, DIN = E + X, KB = E / 4, S = E + 1;
+    constexpr int W = 64;
+    __shared__ float s_x[kSplatTile * S];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+    const uint32_t m = lane & 15u, g = lane >> 4;
+    const uint32_t base = blockIdx.x * kSplatTile;
+    {
+        const uint32_t i = min(base + tid, n - 1u);  // lanes past the end repeat the last sample
+        const V3 x = xyz(pos[i]);
+        float* row = s_x + tid * S;
+#pragma unroll 2
+        for (int l = 0; l < L; ++l) {
+            float f[2];
+            encode_level<2>(table, gp, (uint32_t)l, x, f);
+            row[2 * l] = f[0];
+            row[2 * l + 1] = f[1];
+        }
+    }
+    float a[4][KB];
+    dg_f4 first[4], w1[4];
 #pragma unroll
-    for (int l = 0; l < L; ++l) encode_level<2>(table, gp, (uint32_t)l, x, enc + 2 * l);
+    for (int t = 0; t < 4; ++t) {
 #pragma unroll
-    for (int e = 2 * L; e < E; ++e) enc[e] = 1.0f;
-    float h[W];
-    dense<E, W, true>(params, enc, h);
-    float logit;
-    dense<W, 1, false>(params + W * E, h, &logit);
-    const float thickness = expf(logit + bias) * dt;
-    atomicMax(reinterpret_cast<uint32_t*>(tmp) + idx[i], __float_as_uint(thickness));
+        for (int kb = 0; kb < KB; ++kb) a[t][kb] = params[(16 * t + m) * DIN + 4 * kb + g];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const uint32_t r = 16 * t + 4 * g + q;
+            float sum = 0.0f;
+#pragma unroll
+            for (int e = 0; e < X; ++e) sum = sum + params[r * DIN + E + e];
+            first[t][q] = sum;
+            w1[t][q] = params[W * DIN + r];
+        }
+    }
+    __syncthreads();
+    for (uint32_t nb = 0; nb < 4; ++nb) {
+        const uint32_t s = wave * 64 + nb * 16 + m;  // sample (column) of this lane
+        const float* xr = s_x + s * S;
+        float logit = 0.0f;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            dg_f4 h = first[t];
+#pragma unroll
+            for (int kb = 0; kb < KB; ++kb)
+                h = __builtin_amdgcn_mfma_f32_16x16x4f32(a[t][kb], xr[4 * kb + g], h, 0, 0, 0);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) logit = __builtin_fmaf(w1[t][q], fmaxf(h[q], 0.0f), logit);
+        }
+        logit += __shfl_xor(logit, 16);
+        logit += __shfl_xor(logit, 32);
+        if (g == 0 && base + s < n) {
+            const float thickness = expf(logit + bias) * dt;
+            atomicMax(reinterpret_cast<uint32_t*>(tmp) + idx[base + s], __float_as_uint(thickness));
+        }
+    }
 }
 
 // NerfNetwork::density (nerf_network.h:385-414): the density MLP's 16
@@ -209,7 +335,8 @@ bool dg_alloc(void* p, size_t bytes) { return hipMalloc(reinterpret_cast<void**>
 void free_density_grid(insta_ctx* ctx) {
     DensityGridState* d = ctx->density;
     if (!d) return;
-    dev_free(d->grid); dev_free(d->tmp); dev_free(d->pos); dev_free(d->idx); dev_free(d->partial); dev_free(d->mean);
+    dev_free(d->grid); dev_free(d->tmp); dev_free(d->partial); dev_free(d->mean);
+    dev_free(d->rec); dev_free(d->idx); dev_free(d->srec); dev_free(d->sidx); dev_free(d->bins); dev_free(d->bin_sums);
     if (d->h_mean) (void)hipHostFree(d->h_mean);
     delete d;
     ctx->density = nullptr;
@@ -237,10 +364,15 @@ insta_status update_density_grid(insta_ctx* ctx, uint32_t slot, uint32_t n_frame
     }
     DensityGridState* d = ctx->density;
     if (n > d->cap) {
-        dev_free(d->pos);
+        dev_free(d->rec);
         dev_free(d->idx);
+        dev_free(d->srec);
+        dev_free(d->sidx);
         d->cap = 0;
-        if (!dg_alloc(&d->pos, (size_t)n * 12) || !dg_alloc(&d->idx, (size_t)n * 4)) {
+        if ((!d->bins && !dg_alloc(&d->bins, kMaxBins * 4)) ||
+            (!d->bin_sums && !dg_alloc(&d->bin_sums, kMaxBins / kScanBins * 4)) ||
+            !dg_alloc(&d->rec, (size_t)n * 16) || !dg_alloc(&d->idx, (size_t)n * 4) ||
+            !dg_alloc(&d->srec, (size_t)n * 16) || !dg_alloc(&d->sidx, (size_t)n * 4)) {
             set_error("density grid sample allocation failed");
             return INSTA_ERR_OOM;
         }
@@ -261,26 +393,45 @@ insta_status update_density_grid(insta_ctx* ctx, uint32_t slot, uint32_t n_frame
         d->marked_n = tv.n_images;
     }
     hipLaunchKernelGGL(dg_fill_kernel, cgrid, block, 0, stream, d->tmp, cells);
-    if (c.n_uniform)
-        hipLaunchKernelGGL(dg_samples_kernel, dim3((c.n_uniform + kThreads - 1) / kThreads), block, 0, stream,
-                           c.n_uniform, d->step, -0.01f, G, d->grid, d->rng, d->pos, d->idx);
-    if (c.n_nonuniform)
-        hipLaunchKernelGGL(dg_samples_kernel, dim3((c.n_nonuniform + kThreads - 1) / kThreads), block, 0, stream,
-                           c.n_nonuniform, d->step, kMinOpticalThickness, G, d->grid, d->rng,
-                           d->pos + 3 * (size_t)c.n_uniform, d->idx + c.n_uniform);
-    INSTA_HIP(hipGetLastError());
-    d->rng.advance(1ull << 32);
     // frames for the warp: a second stream, advanced per update
     Pcg32 wr = Pcg32::seeded(c.seed ^ 0x9e3779b9u);
     wr.advance((uint64_t)d->step << 32);
-    insta_status st = launch_deform_positions(ctx, d->pos, n, n_frames, wr, stream);
+    // bins: frames 0 .. n_frames - 2 (one at least) times runs of 2^bin_shift
+    // Morton cells, at most kMaxBins and about one per sample
+    const uint32_t n_meshes = n_frames - 1, bin_frames = std::max(n_meshes, 1u);
+    uint32_t max_bins = kScanBins;
+    while (max_bins < n && max_bins < kMaxBins) max_bins <<= 1;
+    uint32_t bin_shift = 0;
+    while (((uint64_t)bin_frames * (cells >> bin_shift)) > max_bins && (cells >> bin_shift) > 1) ++bin_shift;
+    const uint32_t frame_bins = cells >> bin_shift, n_bins = bin_frames * frame_bins;
+    const uint32_t scan_blocks = (n_bins + kScanBins - 1) / kScanBins;
+    hipLaunchKernelGGL(dg_fill_kernel, dim3((n_bins + kThreads - 1) / kThreads), block, 0, stream,
+                       reinterpret_cast<float*>(d->bins), n_bins);
+    if (c.n_uniform)
+        hipLaunchKernelGGL(dg_samples_kernel, dim3((c.n_uniform + kThreads - 1) / kThreads), block, 0, stream,
+                           c.n_uniform, d->step, -0.01f, G, d->grid, d->rng, wr, 0u, n_meshes, bin_shift, frame_bins,
+                           d->rec, d->idx, d->bins);
+    if (c.n_nonuniform)
+        hipLaunchKernelGGL(dg_samples_kernel, dim3((c.n_nonuniform + kThreads - 1) / kThreads), block, 0, stream,
+                           c.n_nonuniform, d->step, kMinOpticalThickness, G, d->grid, d->rng, wr, c.n_uniform,
+                           n_meshes, bin_shift, frame_bins, d->rec, d->idx, d->bins);
+    hipLaunchKernelGGL(dg_bin_sums_kernel, dim3(scan_blocks), dim3(kScanBins), 0, stream, d->bins, n_bins, d->bin_sums);
+    hipLaunchKernelGGL(dg_bin_scan_kernel, dim3(scan_blocks), dim3(kScanBins), 0, stream, d->bins, n_bins, d->bin_sums);
+    hipLaunchKernelGGL(dg_order_kernel, dim3((n + kThreads - 1) / kThreads), block, 0, stream, n, bin_shift, frame_bins,
+                       d->rec, d->idx, d->bins, d->srec, d->sidx);
+    INSTA_HIP(hipGetLastError());
+    d->rng.advance(1ull << 32);
+    // the drawn records and the first bin's counter are done with: the warp's
+    // queue and its length
+    hipLaunchKernelGGL(dg_fill_kernel, dim3(1), block, 0, stream, reinterpret_cast<float*>(d->bins), 1u);
+    insta_status st = launch_deform_records(ctx, d->srec, n, reinterpret_cast<uint2*>(d->rec), d->bins, stream);
     if (st != INSTA_OK) return st;
     const float* table = ctx->d_params + ctx->layout.n_mlp_params;
     const GridParams gp = grid_params(ctx);
-    const dim3 sgrid((n + 127) / 128);
+    const dim3 sgrid((n + kSplatTile - 1) / kSplatTile);
 #define INSTA_SPLAT(L_, X_)                                                                                     \
-    hipLaunchKernelGGL((dg_splat_kernel<L_, X_>), sgrid, dim3(128), 0, stream, ctx->d_params, table, gp, d->pos,    \
-                       d->idx, n, ctx->cfg.dt, ctx->cfg.density_logit_bias, d->tmp)
+    hipLaunchKernelGGL((dg_splat_kernel<L_, X_>), sgrid, dim3(kSplatTile), 0, stream, ctx->d_params, table, gp, d->srec,   \
+                       d->sidx, n, ctx->cfg.dt, ctx->cfg.density_logit_bias, d->tmp)
     const bool x16 = ctx->cfg.n_extra_dims != 0;
     if (ctx->cfg.n_levels == 8) {
         if (x16) INSTA_SPLAT(8, 16);

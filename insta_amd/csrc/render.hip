@@ -43,6 +43,7 @@ enum : uint32_t {
     kCntEmitted = 5,
     kCntRounds = 6,
     kCntMisses = 7,   // in-box samples whose nearest-triangle query found nothing
+    kCntQueue = 8,    // queries left for the deformation's second pass
     kNumCounters = 16
 };
 
@@ -327,13 +328,14 @@ __global__ void clear_counters_kernel(uint32_t* counters, uint32_t first, uint32
     if (i < n) counters[first + i] = 0;
 }
 
-// Before a round: clear the next live list's count and the round's sample
-// count; the first round also keeps the initial live count.
+// Before a round: clear the next live list's count and the round's sample and
+// queue counts; the first round also keeps the initial live count.
 __global__ void round_begin_kernel(uint32_t* counters, uint32_t next_slot, uint32_t first) {
     if (threadIdx.x != 0) return;
     if (first) counters[kCntAlive0] = counters[kCntAliveA];
     counters[next_slot] = 0;
     counters[kCntSamples] = 0;
+    counters[kCntQueue] = 0;
 }
 
 // ---- host side of the Sobol pixel offset (random_val.cuh:272-322) --------
@@ -584,7 +586,7 @@ insta_status enqueue_round(insta_ctx* ctx, RenderWS& ws, const RenderArgs& a, in
     // at most max_alive * K <= sample capacity samples this round
     const uint32_t n_max = (uint32_t)ws.samples;
     prof_begin(ctx, prof, INSTA_KERNEL_DEFORM, stream);
-    insta_status st = launch_deform_soa(ctx, ws, frame, cnt + kCntSamples, n_max, cnt + kCntMisses, stream);
+    insta_status st = launch_deform_soa(ctx, ws, frame, cnt + kCntSamples, n_max, cnt + kCntMisses, cnt + kCntQueue, stream);
     if (st != INSTA_OK) return st;
     prof_end(ctx, prof, INSTA_KERNEL_DEFORM, 0, stream);
     prof_begin(ctx, prof, INSTA_KERNEL_NETWORK, stream);

@@ -63,7 +63,8 @@ enum : uint32_t {
     kTCompactRes = 6,  // compacted samples reserved
     kTCompactN = 7,    // compacted samples kept (<= compact capacity)
     kTRound0 = 8,      // samples evaluated in each window (kRounds counters)
-    kTCounters = 12
+    kTQueue = 12,      // queries left for the deformation's second pass
+    kTCounters = 13
 };
 
 // Evaluation windows over each ray's marched samples: samples [kWin[w],
@@ -470,6 +471,7 @@ __global__ __launch_bounds__(256) void train_gather_kernel(uint32_t lo, uint32_t
                                                            float4* __restrict__ r_pos,
                                                            uint32_t* __restrict__ counters, uint32_t round_slot) {
     const uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
+    if (r == 0) counters[kTQueue] = 0u;  // this round's
     uint32_t n = 0;
     if (r < counters[kTRays] && ray_alive[r]) {
         const uint32_t cnt = ray_cnt[r];
@@ -1681,7 +1683,7 @@ insta_status train_step(insta_ctx* ctx, const insta_train_config& tc, insta_trai
         const uint32_t round_grid =
             (uint32_t)std::min<uint64_t>(std::min<uint64_t>(cap, (uint64_t)n_rays * (hi - lo)), 1u << 20);
         st = launch_deform_samples(ctx, -1, ts->ray_frame, n_round, round_grid, ts->r_pos, ts->ray_d, ts->s_hit,
-                                   ts->r_cpos, ts->r_cdir, ctx->d_misses, stream);
+                                   ts->r_cpos, ts->r_cdir, ctx->d_misses, ts->r_out, ts->counters + kTQueue, stream);
         if (st != INSTA_OK) return st;
         st = launch_network_samples(ctx, n_round, cap, ts->r_cpos, ts->r_cdir, ts->r_out, stream);
         if (st != INSTA_OK) return st;
