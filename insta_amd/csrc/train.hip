@@ -137,11 +137,10 @@ struct TrainState {
     float* t_buf = nullptr;        // march t values, step-major [max_steps][rays of the step]: the rounds and the loss read them
     // optimizer
     float *grad = nullptr, *adam_m = nullptr, *adam_v = nullptr;
-    // hash-table gradients during the backward: one copy per XCD (FP32 or
-    // packed FP16), summed into grad afterwards
-    float* grad_x = nullptr;
-    __half2* grad_xh = nullptr;
-    float* denc = nullptr;         // dL/dencoding of the batch [32][batch cap], for the LDS scatter
+    // hash-table gradients under FP16 accumulation: kHalfCopies partial tables
+    // of the levels beyond the LDS-scattered ones, summed into grad afterwards
+    __half2* grad_h = nullptr;
+    float* denc = nullptr;         // dL/dencoding of the batch [32][batch cap], for the scatters
     // LDS-scattered levels (a prefix of the levels, entries [0, lds_end)):
     // one partial table per chunk of the batch, [kScatterMaxChunks][2 lds_end]
     float* grad_p = nullptr;
@@ -663,48 +662,20 @@ __global__ __launch_bounds__(256) void train_loss_kernel(LossArgs a, Pcg32 rng0,
     }
 }
 
-// The XCD (accelerator complex die) this wave runs on, 0 .. kXcds - 1: the
-// hardware register XCC_ID (s_getreg_b32, register 20).
-INSTA_DEV uint32_t xcd_id() { return (uint32_t)__builtin_amdgcn_s_getreg((31 << 11) | 20) % kXcds; }
-
-// Table gradients into grad_tab (FP32): entries below lds_end are the sum of
-// the LDS scatter's chunk partials (chunk order), the others the sum of the
-// per-XCD copies (a fixed order, the FP32 ones then the FP16 ones, each set
-// when in use; the copies are cleared before each backward).
-__global__ void grad_copies_reduce_kernel(const float* __restrict__ grad_x, const __half2* __restrict__ grad_xh,
-                                          uint64_t entries, uint32_t use_x, uint32_t use_xh,
-                                          const float* __restrict__ grad_p, uint32_t lds_end, uint32_t chunks,
-                                          float* __restrict__ grad_tab, uint32_t accumulate) {
-    for (uint64_t e = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; e < entries;
-         e += (uint64_t)gridDim.x * blockDim.x) {
-        float a = 0.0f, b = 0.0f;
-        if (e < lds_end) {
-            for (uint32_t c = 0; c < chunks; ++c) {
-                const float2 v = *reinterpret_cast<const float2*>(grad_p + 2 * ((uint64_t)c * lds_end + e));
-                a = a + v.x;
-                b = b + v.y;
-            }
-        } else if (use_x)
-#pragma unroll
-            for (uint32_t x = 0; x < kXcds; ++x) {
-                const float2 v = *reinterpret_cast<const float2*>(grad_x + 2 * (x * entries + e));
-                a = a + v.x;
-                b = b + v.y;
-            }
-        if (use_xh)
-#pragma unroll
-            for (uint32_t x = 0; x < kXcds; ++x) {
-                const __half2 h = grad_xh[x * entries + e];
-                a = a + __low2float(h);
-                b = b + __high2float(h);
-            }
-        if (accumulate) {
-            a = a + grad_tab[2 * e];
-            b = b + grad_tab[2 * e + 1];
-        }
-        grad_tab[2 * e] = a;
-        grad_tab[2 * e + 1] = b;
+// Gradients of the LDS-scattered entries into grad_tab: the sum of the
+// scatter's chunk partials in chunk order.
+__global__ void grad_partials_reduce_kernel(const float* __restrict__ grad_p, uint32_t lds_end, uint32_t chunks,
+                                            float* __restrict__ grad_tab) {
+    const uint32_t e = blockIdx.x * blockDim.x + threadIdx.x;
+    if (e >= lds_end) return;
+    float a = 0.0f, b = 0.0f;
+    for (uint32_t c = 0; c < chunks; ++c) {
+        const float2 v = *reinterpret_cast<const float2*>(grad_p + 2 * ((uint64_t)c * lds_end + e));
+        a = a + v.x;
+        b = b + v.y;
     }
+    grad_tab[2 * e] = a;
+    grad_tab[2 * e + 1] = b;
 }
 
 // Sum of v over the run of equal keys that starts at this lane, in the run's
@@ -715,6 +686,7 @@ INSTA_DEV float2 run_sum(uint32_t key, float2 v, bool& head) {
     const uint32_t prev = __shfl_up(key, 1u);
     head = lane == 0u || prev != key;
     const uint64_t heads = __ballot(head);
+    if (heads == ~0ull) return v;  // no two neighbours share a key
     const uint64_t later = lane == 63u ? 0ull : heads & (~0ull << (lane + 1u));
     const uint32_t end = later ? (uint32_t)__builtin_ctzll(later) - 1u : 63u;
 #pragma unroll
@@ -735,7 +707,7 @@ INSTA_DEV float2 run_sum(uint32_t key, float2 v, bool& head) {
 // instead of two; on levels in run_mask a wave first sums runs of
 // consecutive samples with one corner, as the per-sample scatter does), then
 // stores the whole table as its chunk's partial (plain coalesced stores, no
-// global atomics); grad_copies_reduce_kernel sums the partials in chunk
+// global atomics); grad_partials_reduce_kernel sums the partials in chunk
 // order.  Same corner and weight arithmetic as the per-sample scatter.
 constexpr uint32_t kLdsEntries = 16384;
 constexpr uint32_t kScatterThreads = 1024;
@@ -850,30 +822,129 @@ __global__ __launch_bounds__(kScatterThreads) void scatter_lds_kernel(GridParams
     }
 }
 
-// Backward over a block of 256 compacted samples, in two phases.
-// Phase 1 (FP32 MFMA, the forward kernel's layout, 16 samples per step of a
-// wave): the deltas of both MLPs through the transposed weights (held in
-// LDS), the ReLU masks from the stored activations, each delta's rows stored
-// for the weight gradients, and dL/dencoding into LDS.  Phase 2 (one thread
-// per sample): the hash-grid scatter; on the levels of run_mask the corner
-// gradients of consecutive samples that land on one table entry (coarse
-// levels along one ray) are summed across the wave first and added by one
-// lane.  (A split into a delta kernel and a low-register scatter kernel
-// measured slower: the scatter's extra occupancy does not repay the round
-// trip of dL/dencoding through memory.)
-template <int L, bool H16, int X>
-__global__ __launch_bounds__(kMlpThreads) void train_backward_kernel(const float* __restrict__ params, GridParams gp,
+// Hash-grid scatter of the levels whose tables exceed LDS, one level's
+// samples after the other on one XCD.  Workgroups are dispatched round-robin
+// over the eight XCDs (block b on XCD b % 8), each with a 4 MB L2, so block b
+// takes the levels b % 8, b % 8 + 8, ... of the list, a level's samples before
+// the next level's: a table of 2^19 entries (4 MB) is added to from one L2
+// while it is resident, instead of every table's lines moving between eight
+// L2s and HBM.  On the levels of run_mask the corner gradients of consecutive
+// samples that land on one entry (coarse levels along one ray) are summed
+// across the wave first and added by one lane.
+// FP32: atomics straight into the gradients; neighbouring lanes first pair
+// up, so that an entry's two adds are neighbours in one memory request.
+// H16: one packed FP16 atomic per corner, into one of kHalfCopies partial
+// tables (by block of kLevelThreads samples; a level's first copy before its
+// second), which keep the rounding of many small adds in check and are summed
+// in a fixed order afterwards.
+// Bound by the L2's atomics.  LEVELS_FIGURES
+constexpr uint32_t kLevelThreads = 256;
+constexpr uint32_t kHalfCopies = 8;
+template <bool H16>
+__global__ __launch_bounds__(kLevelThreads) void scatter_levels_kernel(GridParams gp, uint32_t level_mask,
+                                                                       uint32_t run_mask, uint32_t blocks,
                                                                        const uint32_t* __restrict__ n_dev,
                                                                        const uint32_t* __restrict__ c_idx,
                                                                        const float4* __restrict__ cpos,
+                                                                       const float* __restrict__ denc_g, uint32_t ld,
+                                                                       float* __restrict__ grad_tab,
+                                                                       __half2* __restrict__ grad_h,
+                                                                       uint64_t entries) {
+    // blocks: sample blocks per level, a multiple of kHalfCopies
+    const uint32_t k = blockIdx.x / kXcds, li = (k / blocks) * kXcds + blockIdx.x % kXcds;
+    uint32_t b = k % blocks, copy = 0;
+    if constexpr (H16) {
+        const uint32_t per_copy = blocks / kHalfCopies;
+        copy = b / per_copy;
+        b = (b % per_copy) * kHalfCopies + copy;
+    }
+    const uint32_t n = *n_dev, s0 = b * kLevelThreads;
+    if (li >= (uint32_t)__popc(level_mask) || (s0 + (threadIdx.x & ~63u)) >= n) return;  // whole waves
+    uint32_t rest = level_mask;
+    for (uint32_t j = 0; j < li; ++j) rest &= rest - 1u;  // drop the li lowest levels of the list
+    const uint32_t l = (uint32_t)__builtin_ctz(rest);
+    const uint32_t size = gp.size[l], res = gp.res[l], off = gp.offset[l];
+    const bool dense_l = (gp.dense_mask >> l) & 1u, runs = (run_mask >> l) & 1u;
+    const float sc = gp.scale[l];
+    const bool valid = s0 + threadIdx.x < n, odd = threadIdx.x & 1u;
+    const uint32_t i = valid ? s0 + threadIdx.x : n - 1u;  // tail lanes repeat the last sample and add nothing
+    const float4 p4 = cpos[c_idx[i]];
+    const float e0 = valid ? denc_g[(size_t)(2u * l) * ld + i] : 0.0f;
+    const float e1 = valid ? denc_g[(size_t)(2u * l + 1u) * ld + i] : 0.0f;
+    const float xs[3] = {p4.x, p4.y, p4.z};
+    float frac[3];
+    uint32_t g[3];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        const float pp = xs[d] * sc + 0.5f;
+        const float fl = floorf(pp);
+        frac[d] = pp - fl;
+        g[d] = (uint32_t)(int32_t)fl;
+    }
+#pragma unroll
+    for (uint32_t c = 0; c < 8; ++c) {
+        float w = 1.0f;
+        uint32_t cg[3];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            const bool up = (c >> q) & 1u;
+            w = w * (up ? frac[q] : 1.0f - frac[q]);
+            cg[q] = g[q] + (up ? 1u : 0u);
+        }
+        uint32_t idx = off + grid_index(cg, dense_l, res, size);
+        float2 v = make_float2(w * e0, w * e1);
+        bool lead = valid;
+        if (runs) {
+            bool head;
+            v = run_sum(valid ? idx : ~0u, v, head);
+            lead = valid && head;
+        }
+        if constexpr (H16) {
+            if (lead) unsafeAtomicAdd(grad_h + copy * entries + idx, __floats2half2_rn(v.x, v.y));
+        } else {
+            if (!lead) idx = ~0u;
+            // quad_perm 0,0,2,2 and 1,1,3,3: the even, then the odd lane's
+            // sample of each pair, its features on the pair's two lanes
+            const uint32_t ie = dpp<0xA0>(idx), io = dpp<0xF5>(idx);
+            const float ye = __uint_as_float(dpp<0xA0>(__float_as_uint(v.y)));
+            const float xo = __uint_as_float(dpp<0xF5>(__float_as_uint(v.x)));
+            const float ve = odd ? ye : v.x, vo = odd ? v.y : xo;
+            if (ie != ~0u) atomicAdd(grad_tab + 2u * (size_t)ie + (odd ? 1u : 0u), ve);
+            if (io != ~0u) atomicAdd(grad_tab + 2u * (size_t)io + (odd ? 1u : 0u), vo);
+        }
+    }
+}
+
+// Gradients of the entries [first, entries) into grad_tab: the sum of the
+// FP16 copies in copy order.
+__global__ void grad_copies_reduce_kernel(const __half2* __restrict__ grad_h, uint64_t first, uint64_t entries,
+                                          float* __restrict__ grad_tab) {
+    for (uint64_t e = first + blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; e < entries;
+         e += (uint64_t)gridDim.x * blockDim.x) {
+        float a = 0.0f, b = 0.0f;
+#pragma unroll
+        for (uint32_t x = 0; x < kHalfCopies; ++x) {
+            const __half2 h = grad_h[x * entries + e];
+            a = a + __low2float(h);
+            b = b + __high2float(h);
+        }
+        grad_tab[2 * e] = a;
+        grad_tab[2 * e + 1] = b;
+    }
+}
+
+// Backward of both MLPs over a block of 256 compacted samples, on FP32 MFMA
+// in the forward kernel's layout (16 samples per step of a wave): the deltas
+// through the transposed weights (held in LDS), the ReLU masks from the
+// stored activations, each delta's rows stored for the weight gradients, and
+// dL/dencoding through LDS to memory for the hash-grid scatters.
+template <int L, int X>
+__global__ __launch_bounds__(kMlpThreads) void train_backward_kernel(const float* __restrict__ params,
+                                                                       const uint32_t* __restrict__ n_dev,
                                                                        const float* __restrict__ act,
                                                                        const float4* __restrict__ dout,
                                                                        float* __restrict__ dact, uint32_t ld,
-                                                                       float* __restrict__ grad_x,
-                                                                       __half2* __restrict__ grad_xh,
-                                                                       uint64_t entries, uint32_t run_mask,
-                                                                       float* __restrict__ denc_g,
-                                                                       uint32_t lds_mask) {
+                                                                       float* __restrict__ denc_g) {
     constexpr int E = 2 * L, DIN = E + X;  // encoding, density input (+ extra dims)
     using A = Act<DIN>;
     using O = Off<DIN>;
@@ -979,75 +1050,16 @@ __global__ __launch_bounds__(kMlpThreads) void train_backward_kernel(const float
     const uint32_t i = base + tid;
     if ((i & ~63u) >= n) return;  // whole wave past the batch (no barrier follows)
     const bool valid = i < n;
-    const uint32_t ic = valid ? i : n - 1u;  // tail lanes recompute the last sample and store nothing
     if (valid) {
         const float4 d4 = dout[i];
         dact[(size_t)(Dact::DRGB + 0) * ld + i] = d4.x;
         dact[(size_t)(Dact::DRGB + 1) * ld + i] = d4.y;
         dact[(size_t)(Dact::DRGB + 2) * ld + i] = d4.z;
     }
-    // hash-grid scatter (the corner/weight arithmetic of encode_level) into
-    // this XCD's copy of the table gradients: a copy's lines stay in one
-    // XCD's L2, instead of moving between the L2s of the eight XCDs that
-    // would otherwise add to the same entries
-    const uint32_t xcd = xcd_id();
-    float* __restrict__ grad_tab = grad_x + (size_t)xcd * 2u * entries;
-    __half2* __restrict__ grad_tab_h = grad_xh + (size_t)xcd * entries;
-    const float4 p4 = cpos[c_idx[ic]];
-    const float xs[3] = {p4.x, p4.y, p4.z};
-#pragma unroll 1
-    for (int l = 0; l < L; ++l) {
-        if ((lds_mask >> l) & 1u) {
-            // scattered by scatter_lds_kernel, which reads dL/dencoding from memory
-            if (valid) {
-                denc_g[(size_t)(2 * l) * ld + i] = s_denc[2 * l][threadIdx.x];
-                denc_g[(size_t)(2 * l + 1) * ld + i] = s_denc[2 * l + 1][threadIdx.x];
-            }
-            continue;
-        }
-        const float sc = gp.scale[l];
-        float frac[3];
-        uint32_t g[3];
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            const float pp = xs[d] * sc + 0.5f;
-            const float fl = floorf(pp);
-            frac[d] = pp - fl;
-            g[d] = (uint32_t)(int32_t)fl;
-        }
-        const bool dense_l = (gp.dense_mask >> l) & 1u;
-        const bool runs = (run_mask >> l) & 1u;
-        const uint32_t res = gp.res[l], size = gp.size[l], off = gp.offset[l];
-        const float e0 = valid ? s_denc[2 * l][threadIdx.x] : 0.0f;
-        const float e1 = valid ? s_denc[2 * l + 1][threadIdx.x] : 0.0f;
-#pragma unroll
-        for (uint32_t c = 0; c < 8; ++c) {
-            float w = 1.0f;
-            uint32_t cg[3];
-#pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                const bool up = (c >> k) & 1u;
-                w = w * (up ? frac[k] : 1.0f - frac[k]);
-                cg[k] = g[k] + (up ? 1u : 0u);
-            }
-            const uint32_t idx = off + grid_index(cg, dense_l, res, size);
-            float2 v = make_float2(w * e0, w * e1);
-            bool lead = valid;
-            if (runs) {
-                bool head;
-                v = run_sum(valid ? idx : ~0u, v, head);
-                lead = valid && head;
-            }
-            if (lead) {
-                if constexpr (H16) {
-                    unsafeAtomicAdd(grad_tab_h + idx, __floats2half2_rn(v.x, v.y));
-                } else {
-                    atomicAdd(grad_tab + 2 * (size_t)idx, v.x);
-                    atomicAdd(grad_tab + 2 * (size_t)idx + 1, v.y);
-                }
-            }
-        }
-    }
+    // dL/dencoding for the scatter kernels
+    if (valid)
+#pragma unroll 4
+        for (int e = 0; e < E; ++e) denc_g[(size_t)e * ld + i] = s_denc[e][tid];
 }
 
 
@@ -1309,32 +1321,16 @@ insta_status launch_train_backward(insta_ctx* ctx, TrainState* ts, const insta_t
     const uint32_t n_mlp = (uint32_t)ctx->layout.n_mlp_params;
     const dim3 sgrid((cap + kMlpThreads - 1) / kMlpThreads);
     float* grad_tab = ts->grad + n_mlp;
-    const uint64_t entries = ctx->layout.n_grid_params / 2;
-    // levels whose tables fit in LDS are scattered by scatter_lds_kernel,
-    // the others per sample (FP32, or packed FP16 copies)
+    // levels whose tables fit in LDS are scattered by scatter_lds_kernel (FP32
+    // or packed FP16), the others by scatter_levels_kernel (FP32)
     const uint32_t lds_mask = ts->lds_levels, lds_end = ts->lds_end;
-    const bool per_sample = lds_mask != (1u << L) - 1u;
-    const bool use_xh = tc.grid_grad_fp16 && per_sample;
-    const bool use_x = !tc.grid_grad_fp16 && per_sample;
-    // clear this backward's copies (fill kernels: capturable)
-    if (use_xh)
-        hipLaunchKernelGGL(fill_zero_kernel, dim3(2048), dim3(256), 0, stream, reinterpret_cast<uint32_t*>(ts->grad_xh),
-                           kXcds * entries);
-    if (use_x)
-        hipLaunchKernelGGL(fill_zero_kernel, dim3(2048), dim3(256), 0, stream, reinterpret_cast<uint32_t*>(ts->grad_x),
-                           kXcds * 2 * entries);
+    const uint32_t big_mask = ((1u << L) - 1u) & ~lds_mask;
     // levels whose cells span at least 1 / kRunMaxStepCells marching steps
     uint32_t run_mask = 0;
     for (int l = 0; l < L; ++l)
         if (ctx->cfg.dt * gp.scale[l] <= kRunMaxStepCells) run_mask |= 1u << l;
-    if (tc.grid_grad_fp16)
-        hipLaunchKernelGGL((train_backward_kernel<L, true, X>), sgrid, dim3(kMlpThreads), 0, stream, ctx->d_params, gp,
-                           n_dev, ts->c_idx, ts->s_cpos, ts->act, ts->c_dout, ts->dact, cap, ts->grad_x, ts->grad_xh,
-                           entries, run_mask, ts->denc, lds_mask);
-    else
-        hipLaunchKernelGGL((train_backward_kernel<L, false, X>), sgrid, dim3(kMlpThreads), 0, stream, ctx->d_params, gp,
-                           n_dev, ts->c_idx, ts->s_cpos, ts->act, ts->c_dout, ts->dact, cap, ts->grad_x, ts->grad_xh,
-                           entries, run_mask, ts->denc, lds_mask);
+    hipLaunchKernelGGL((train_backward_kernel<L, X>), sgrid, dim3(kMlpThreads), 0, stream, ctx->d_params, n_dev, ts->act,
+                       ts->c_dout, ts->dact, cap, ts->denc);
     INSTA_HIP(hipGetLastError());
     const uint32_t chunks =
         std::min<uint32_t>(std::max<uint32_t>((cap + kScatterChunk - 1) / kScatterChunk, 1u), kScatterMaxChunks);
@@ -1346,11 +1342,32 @@ insta_status launch_train_backward(insta_ctx* ctx, TrainState* ts, const insta_t
         else
             hipLaunchKernelGGL(scatter_lds_kernel<false>, grid, dim3(kScatterThreads), 0, stream, gp, n_dev, ts->c_idx,
                                ts->s_cpos, ts->denc, cap, run_mask, ts->grad_p, lds_end);
+        hipLaunchKernelGGL(grad_partials_reduce_kernel, dim3((lds_end + 255) / 256), dim3(256), 0, stream, ts->grad_p,
+                           lds_end, chunks, grad_tab);
         INSTA_HIP(hipGetLastError());
     }
-    hipLaunchKernelGGL(grad_copies_reduce_kernel, dim3(2048), dim3(256), 0, stream, ts->grad_x, ts->grad_xh, entries,
-                       use_x ? 1u : 0u, use_xh ? 1u : 0u, ts->grad_p, lds_end, chunks, grad_tab, 0u);
-    INSTA_HIP(hipGetLastError());
+    if (big_mask) {
+        const uint64_t entries = ctx->layout.n_grid_params / 2;
+        const uint32_t blocks =
+            ((cap + kLevelThreads - 1) / kLevelThreads + kHalfCopies - 1) / kHalfCopies * kHalfCopies;
+        const uint32_t slots = (__builtin_popcount(big_mask) + kXcds - 1) / kXcds;
+        const dim3 grid(kXcds * slots * blocks);
+        if (tc.grid_grad_fp16) {
+            // clear this backward's copies (a fill kernel: capturable)
+            hipLaunchKernelGGL(fill_zero_kernel, dim3(2048), dim3(256), 0, stream,
+                               reinterpret_cast<uint32_t*>(ts->grad_h), kHalfCopies * entries);
+            hipLaunchKernelGGL(scatter_levels_kernel<true>, grid, dim3(kLevelThreads), 0, stream, gp, big_mask,
+                               run_mask, blocks, n_dev, ts->c_idx, ts->s_cpos, ts->denc, cap, grad_tab, ts->grad_h,
+                               entries);
+            hipLaunchKernelGGL(grad_copies_reduce_kernel, dim3(2048), dim3(256), 0, stream, ts->grad_h,
+                               (uint64_t)lds_end, entries, grad_tab);
+        } else {
+            hipLaunchKernelGGL(scatter_levels_kernel<false>, grid, dim3(kLevelThreads), 0, stream, gp, big_mask,
+                               run_mask, blocks, n_dev, ts->c_idx, ts->s_cpos, ts->denc, cap, grad_tab, ts->grad_h,
+                               entries);
+        }
+        INSTA_HIP(hipGetLastError());
+    }
     WArgs wa;
     wa.p[0] = WProduct{Dact::DH1, A::ENC, kW, DIN, O::W0};
     wa.p[1] = WProduct{Dact::DDENS, A::H1, kDOut, kW, O::W1};
@@ -1529,7 +1546,7 @@ void free_train(insta_ctx* ctx) {
     if (!ts) return;
     free_workspace_train(ts);
     dev_free(ts->images); dev_free(ts->meta); dev_free(ts->seg); dev_free(ts->depth);
-    dev_free(ts->grad); dev_free(ts->grad_x); dev_free(ts->grad_xh); dev_free(ts->grad_p);
+    dev_free(ts->grad); dev_free(ts->grad_h); dev_free(ts->grad_p);
     dev_free(ts->adam_m); dev_free(ts->adam_v); dev_free(ts->counters); dev_free(ts->net_extra);
     if (ctx->net_src == ts->ema_infer) ctx->net_src = nullptr;
     dev_free(ts->ema); dev_free(ts->ema_infer);
@@ -1552,8 +1569,7 @@ static insta_status ensure_train_state(insta_ctx* ctx, hipStream_t stream) {
         bool ok = train_alloc(ts->grad, np * sizeof(float)) && train_alloc(ts->adam_m, np * sizeof(float)) &&
                   train_alloc(ts->adam_v, np * sizeof(float)) && train_alloc(ts->ema, np * sizeof(float)) &&
                   train_alloc(ts->ema_infer, np * sizeof(float)) &&
-                  train_alloc(ts->grad_x, kXcds * ctx->layout.n_grid_params * sizeof(float)) &&
-                  train_alloc(ts->grad_xh, kXcds * (ctx->layout.n_grid_params / 2) * sizeof(__half2)) &&
+                  train_alloc(ts->grad_h, kHalfCopies * (ctx->layout.n_grid_params / 2) * sizeof(__half2)) &&
                   (ts->lds_end == 0 ||
                    train_alloc(ts->grad_p, (size_t)kScatterMaxChunks * 2 * ts->lds_end * sizeof(float))) &&
                   train_alloc(ts->counters, kTCounters * sizeof(uint32_t)) &&
