@@ -140,6 +140,11 @@ struct TrainState {
     // hash-table gradients under FP16 accumulation: kHalfCopies partial tables
     // of the levels beyond the LDS-scattered ones, summed into grad afterwards
     __half2* grad_h = nullptr;
+    // partitioned scatter: its levels (0: the batch is not partitioned), the
+    // records of one pass and their directory
+    uint32_t part_levels = 0;
+    void* recs = nullptr;
+    uint32_t* rec_dir = nullptr;
     float* denc = nullptr;         // dL/dencoding of the batch [32][batch cap], for the scatters
     // LDS-scattered levels (a prefix of the levels, entries [0, lds_end)):
     // one partial table per chunk of the batch, [kScatterMaxChunks][2 lds_end]
@@ -663,19 +668,17 @@ __global__ __launch_bounds__(256) void train_loss_kernel(LossArgs a, Pcg32 rng0,
 }
 
 // Gradients of the LDS-scattered entries into grad_tab: the sum of the
-// scatter's chunk partials in chunk order.
+// scatter's chunk partials ([chunk][feature][lds_end]) in chunk order.
 __global__ void grad_partials_reduce_kernel(const float* __restrict__ grad_p, uint32_t lds_end, uint32_t chunks,
                                             float* __restrict__ grad_tab) {
     const uint32_t e = blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= lds_end) return;
     float a = 0.0f, b = 0.0f;
     for (uint32_t c = 0; c < chunks; ++c) {
-        const float2 v = *reinterpret_cast<const float2*>(grad_p + 2 * ((uint64_t)c * lds_end + e));
-        a = a + v.x;
-        b = b + v.y;
+        a = a + grad_p[(size_t)(2u * c) * lds_end + e];
+        b = b + grad_p[(size_t)(2u * c + 1u) * lds_end + e];
     }
-    grad_tab[2 * e] = a;
-    grad_tab[2 * e + 1] = b;
+    *reinterpret_cast<float2*>(grad_tab + 2 * (size_t)e) = make_float2(a, b);
 }
 
 // Sum of v over the run of equal keys that starts at this lane, in the run's
@@ -701,14 +704,20 @@ INSTA_DEV float2 run_sum(uint32_t key, float2 v, bool& head) {
 }
 
 // Hash-grid scatter of the leading levels whose tables fit in LDS (at most
-// kLdsEntries entries each): one workgroup per (level, chunk of the batch)
-// adds its samples' corner gradients into an LDS copy of the level's table
-// (LDS float atomics, or packed FP16 atomics under H16, one per corner
-// instead of two; on levels in run_mask a wave first sums runs of
-// consecutive samples with one corner, as the per-sample scatter does), then
-// stores the whole table as its chunk's partial (plain coalesced stores, no
-// global atomics); grad_partials_reduce_kernel sums the partials in chunk
-// order.  Same corner and weight arithmetic as the per-sample scatter.
+// kLdsEntries entries each): a workgroup adds its chunk's corner gradients
+// into an LDS copy of the level's table, then stores the whole table as its
+// chunk's partial (plain coalesced stores, no global atomics);
+// grad_partials_reduce_kernel sums the partials in chunk order.
+// FP32 gradients (scatter_lds64_kernel): one workgroup per (chunk, level,
+// feature) with FP64 LDS atomics.  An FP32 LDS atomic retires 200 G lanes/s
+// over the chip, an FP64 one 1,760 G (random entries or 64 hot ones alike), so
+// the table holds doubles, one feature of them; recomputing the corners for
+// the other feature costs less than the adds did, and neither conflicts nor
+// runs of equal entries need care.  The sums are exact but for one rounding.
+// LDS64_FIGURES
+// H16 (scatter_lds_kernel): one workgroup per (chunk, level), packed FP16
+// atomics, one per corner; on levels in run_mask a wave first sums runs of
+// consecutive samples with one corner.
 constexpr uint32_t kLdsEntries = 16384;
 constexpr uint32_t kScatterThreads = 1024;
 constexpr uint32_t kScatterChunk = 8192;    // samples per workgroup
@@ -726,16 +735,75 @@ uint32_t lds_scatter_levels(const GridParams& gp, int n_levels, uint32_t* end) {
     return mask;
 }
 
-template <bool H16>
+// partial tables: [chunk][feature][lds_end]
+__global__ __launch_bounds__(kScatterThreads) void scatter_lds64_kernel(GridParams gp,
+                                                                        const uint32_t* __restrict__ n_dev,
+                                                                        const uint32_t* __restrict__ c_idx,
+                                                                        const float4* __restrict__ cpos,
+                                                                        const float* __restrict__ denc_g, uint32_t ld,
+                                                                        float* __restrict__ grad_p, uint32_t lds_end) {
+    __shared__ double tab[kLdsEntries];  // 128 KB: one workgroup per CU
+    const uint32_t l = blockIdx.y, f = blockIdx.z;
+    const uint32_t n = *n_dev;
+    const uint32_t chunk = (n + gridDim.x - 1) / gridDim.x;
+    // an empty chunk still stores its (zero) partial
+    const uint32_t s0 = min(n, blockIdx.x * chunk), s1 = min(n, s0 + chunk);
+    const uint32_t size = gp.size[l], res = gp.res[l];
+    const bool dense_l = (gp.dense_mask >> l) & 1u;
+    const float sc = gp.scale[l];
+    for (uint32_t j = threadIdx.x; j < size; j += kScatterThreads) tab[j] = 0.0;
+    __syncthreads();
+    const float* __restrict__ de = denc_g + (size_t)(2u * l + f) * ld;
+    // the next sample is loaded before this one's corners are added
+    uint32_t i = s0 + threadIdx.x;
+    float4 pn = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    float en = 0.0f;
+    if (i < s1) {
+        pn = cpos[c_idx[i]];
+        en = de[i];
+    }
+    while (i < s1) {
+        const float xs[3] = {pn.x, pn.y, pn.z};
+        const float e = en;
+        i += kScatterThreads;
+        if (i < s1) {
+            pn = cpos[c_idx[i]];
+            en = de[i];
+        }
+        float frac[3];
+        uint32_t g[3];
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            const float pp = xs[d] * sc + 0.5f;
+            const float fl = floorf(pp);
+            frac[d] = pp - fl;
+            g[d] = (uint32_t)(int32_t)fl;
+        }
+#pragma unroll
+        for (uint32_t c = 0; c < 8; ++c) {
+            float w = 1.0f;
+            uint32_t cg[3];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                const bool up = (c >> k) & 1u;
+                w = w * (up ? frac[k] : 1.0f - frac[k]);
+                cg[k] = g[k] + (up ? 1u : 0u);
+            }
+            unsafeAtomicAdd(&tab[grid_index(cg, dense_l, res, size)], (double)(w * e));
+        }
+    }
+    __syncthreads();
+    float* __restrict__ dst = grad_p + ((size_t)blockIdx.x * 2u + f) * lds_end + gp.offset[l];
+    for (uint32_t j = threadIdx.x; j < size; j += kScatterThreads) dst[j] = (float)tab[j];
+}
+
 __global__ __launch_bounds__(kScatterThreads) void scatter_lds_kernel(GridParams gp, const uint32_t* __restrict__ n_dev,
                                                                       const uint32_t* __restrict__ c_idx,
                                                                       const float4* __restrict__ cpos,
                                                                       const float* __restrict__ denc_g, uint32_t ld,
                                                                       uint32_t run_mask, float* __restrict__ grad_p,
                                                                       uint32_t lds_end) {
-    // FP32 pairs (128 KB, one workgroup per CU) or packed FP16 (64 KB, two)
-    using Entry = std::conditional_t<H16, __half2, float2>;
-    __shared__ Entry tab[kLdsEntries];
+    __shared__ __half2 tab[kLdsEntries];  // 64 KB: two workgroups per CU
     const uint32_t l = blockIdx.y;  // grid.y: the LDS-scattered levels
     const uint32_t n = *n_dev;
     const uint32_t chunk = (n + gridDim.x - 1) / gridDim.x;
@@ -744,12 +812,7 @@ __global__ __launch_bounds__(kScatterThreads) void scatter_lds_kernel(GridParams
     const uint32_t size = gp.size[l], off = gp.offset[l], res = gp.res[l];
     const bool dense_l = (gp.dense_mask >> l) & 1u;
     const float sc = gp.scale[l];
-    for (uint32_t j = threadIdx.x; j < size; j += kScatterThreads) {
-        if constexpr (H16)
-            tab[j] = __floats2half2_rn(0.0f, 0.0f);
-        else
-            tab[j] = make_float2(0.0f, 0.0f);
-    }
+    for (uint32_t j = threadIdx.x; j < size; j += kScatterThreads) tab[j] = __floats2half2_rn(0.0f, 0.0f);
     __syncthreads();
     const bool runs = (run_mask >> l) & 1u;
     // every thread runs every round (run_sum needs whole waves); the next
@@ -801,24 +864,15 @@ __global__ __launch_bounds__(kScatterThreads) void scatter_lds_kernel(GridParams
                 v = run_sum(valid ? idx : ~0u, v, head);
                 lead = valid && head;
             }
-            if (lead) {
-                if constexpr (H16) {
-                    unsafeAtomicAdd(&tab[idx], __floats2half2_rn(v.x, v.y));
-                } else {
-                    atomicAdd(&tab[idx].x, v.x);
-                    atomicAdd(&tab[idx].y, v.y);
-                }
-            }
+            if (lead) unsafeAtomicAdd(&tab[idx], __floats2half2_rn(v.x, v.y));
         }
     }
     __syncthreads();
-    float* __restrict__ dst = grad_p + 2u * ((size_t)blockIdx.x * lds_end + off);
-    float2* __restrict__ dst2 = reinterpret_cast<float2*>(dst);
+    float* __restrict__ dst = grad_p + (size_t)blockIdx.x * 2u * lds_end + off;
     for (uint32_t j = threadIdx.x; j < size; j += kScatterThreads) {
-        if constexpr (H16)
-            dst2[j] = __half22float2(tab[j]);
-        else
-            dst2[j] = tab[j];
+        const float2 v = __half22float2(tab[j]);
+        dst[j] = v.x;
+        dst[lds_end + j] = v.y;
     }
 }
 
@@ -840,6 +894,13 @@ __global__ __launch_bounds__(kScatterThreads) void scatter_lds_kernel(GridParams
 // Bound by the L2's atomics.  LEVELS_FIGURES
 constexpr uint32_t kLevelThreads = 256;
 constexpr uint32_t kHalfCopies = 8;
+// Batches above kPartMinBatch, with no table above kPartMaxEntries (the
+// partition's directory), are partitioned, kPartPass samples at a time (352 MB
+// of records at full size); below, the fixed work of walking every slice costs
+// more than the atomics.  PARTITION_LINE
+constexpr uint32_t kPartMinBatch = 8192;
+constexpr uint32_t kPartMaxEntries = 1u << 19;
+constexpr uint32_t kPartPass = 1u << 18;
 template <bool H16>
 __global__ __launch_bounds__(kLevelThreads) void scatter_levels_kernel(GridParams gp, uint32_t level_mask,
                                                                        uint32_t run_mask, uint32_t blocks,
@@ -912,6 +973,199 @@ __global__ __launch_bounds__(kLevelThreads) void scatter_levels_kernel(GridParam
             if (ie != ~0u) atomicAdd(grad_tab + 2u * (size_t)ie + (odd ? 1u : 0u), ve);
             if (io != ~0u) atomicAdd(grad_tab + 2u * (size_t)io + (odd ? 1u : 0u), vo);
         }
+    }
+}
+
+// The same levels for large batches, in two kernels without global atomics
+// (an XCD's L2 retires about one request of them per clock, 5.6 ms per 10^6
+// samples at full size).  partition_kernel writes each chunk's corner
+// gradients as records (entry, value), sorted by slice of the level's table;
+// accumulate_kernel, one workgroup per (slice, level), adds its slice's records
+// of every chunk into an LDS copy of the slice and stores it: every entry of
+// the level is written once, so the gradients need no clearing either.
+// FP32: 12-byte records, slices of 8,192 entries, FP64 LDS atomics (as
+// scatter_lds64_kernel).  H16: 8-byte records of FP16 pairs (runs summed first,
+// as in scatter_levels_kernel), the same slices; chunk c is of copy
+// c % kHalfCopies, and the slice's copies are accumulated one after the other
+// and summed in order.  Bound by the records' trip through memory (8 corners
+// x 12 bytes, written and read).  PARTITION_FIGURES
+template <bool H16>
+struct Part {
+    static constexpr uint32_t kChunkSamples = H16 ? kLevelThreads : 1024u;
+    static constexpr uint32_t kSliceShift = 13u;
+    static constexpr uint32_t kMaxSlices = kPartMaxEntries >> kSliceShift;
+    static_assert(kMaxSlices <= 64u, "one wave scans a chunk's slices");
+    static constexpr uint32_t kLanes = H16 ? 32u : 64u;  // lanes reading one chunk's records
+    struct Rec32 {
+        uint32_t idx;
+        float x, y;
+    };
+    struct Rec16 {
+        uint32_t idx;
+        __half2 v;
+    };
+    using Rec = std::conditional_t<H16, Rec16, Rec32>;
+    // per chunk: record slots, directory words (first record of each slice, end)
+    static constexpr uint32_t kRecs = 8u * kChunkSamples;
+    static constexpr uint32_t kDir = kMaxSlices + 1u;
+};
+
+template <bool H16>
+__global__ __launch_bounds__(Part<H16>::kChunkSamples) void partition_kernel(
+    GridParams gp, uint32_t first_level, uint32_t run_mask, uint32_t pass0, const uint32_t* __restrict__ n_dev,
+    const uint32_t* __restrict__ c_idx, const float4* __restrict__ cpos, const float* __restrict__ denc_g, uint32_t ld,
+    typename Part<H16>::Rec* __restrict__ recs, uint32_t* __restrict__ dir) {
+    using P = Part<H16>;
+    __shared__ uint32_t s_cnt[P::kMaxSlices], s_base[P::kMaxSlices];
+    const uint32_t n = *n_dev, s0 = pass0 + blockIdx.x * P::kChunkSamples;
+    if (s0 >= n) return;
+    const uint32_t l = first_level + blockIdx.y, t = threadIdx.x;
+    const uint32_t size = gp.size[l], res = gp.res[l];
+    const bool dense_l = (gp.dense_mask >> l) & 1u;
+    const float sc = gp.scale[l];
+    for (uint32_t j = t; j < P::kMaxSlices; j += P::kChunkSamples) s_cnt[j] = 0u;
+    __syncthreads();
+    const bool valid = s0 + t < n;
+    const uint32_t i = valid ? s0 + t : n - 1u;  // tail lanes repeat the last sample and emit nothing
+    const float4 p4 = cpos[c_idx[i]];
+    const float e0 = denc_g[(size_t)(2u * l) * ld + i], e1 = denc_g[(size_t)(2u * l + 1u) * ld + i];
+    const float xs[3] = {p4.x, p4.y, p4.z};
+    float frac[3];
+    uint32_t g[3];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        const float pp = xs[d] * sc + 0.5f;
+        const float fl = floorf(pp);
+        frac[d] = pp - fl;
+        g[d] = (uint32_t)(int32_t)fl;
+    }
+    uint32_t idx[8], rank[8];
+    float2 v[8];
+#pragma unroll
+    for (uint32_t c = 0; c < 8; ++c) {
+        float w = 1.0f;
+        uint32_t cg[3];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            const bool up = (c >> q) & 1u;
+            w = w * (up ? frac[q] : 1.0f - frac[q]);
+            cg[q] = g[q] + (up ? 1u : 0u);
+        }
+        idx[c] = grid_index(cg, dense_l, res, size);
+        v[c] = make_float2(w * e0, w * e1);
+        bool lead = valid;
+        if constexpr (H16) {
+            if ((run_mask >> l) & 1u) {
+                bool head;
+                v[c] = run_sum(valid ? idx[c] : ~0u, v[c], head);
+                lead = valid && head;
+            }
+        }
+        if (lead)
+            rank[c] = atomicAdd(&s_cnt[idx[c] >> P::kSliceShift], 1u);
+        else
+            idx[c] = ~0u;
+    }
+    __syncthreads();
+    // first record of each slice (one wave; at most 64 slices)
+    const size_t chunk = (size_t)blockIdx.y * gridDim.x + blockIdx.x;
+    if (t < 64u) {
+        const uint32_t cnt = t < P::kMaxSlices ? s_cnt[t] : 0u;
+        uint32_t incl = cnt;
+#pragma unroll
+        for (uint32_t o = 1; o < 64u; o <<= 1) {
+            const uint32_t up = __shfl_up(incl, o);
+            if (t >= o) incl += up;
+        }
+        if (t < P::kMaxSlices) {
+            s_base[t] = incl - cnt;
+            dir[chunk * P::kDir + t] = incl - cnt;
+            if (t == P::kMaxSlices - 1u) dir[chunk * P::kDir + t + 1u] = incl;
+        }
+    }
+    __syncthreads();
+    typename P::Rec* __restrict__ out = recs + chunk * P::kRecs;
+#pragma unroll
+    for (uint32_t c = 0; c < 8; ++c) {
+        if (idx[c] == ~0u) continue;
+        const uint32_t slot = s_base[idx[c] >> P::kSliceShift] + rank[c];
+        const uint32_t e = idx[c] & ((1u << P::kSliceShift) - 1u);
+        if constexpr (H16)
+            out[slot] = {e, __floats2half2_rn(v[c].x, v[c].y)};
+        else
+            out[slot] = {e, v[c].x, v[c].y};
+    }
+}
+
+constexpr uint32_t kAccThreads = 1024;
+template <bool H16>
+__global__ __launch_bounds__(kAccThreads) void accumulate_kernel(GridParams gp, uint32_t first_level, uint32_t pass0,
+                                                                 uint32_t chunks, const uint32_t* __restrict__ n_dev,
+                                                                 const typename Part<H16>::Rec* __restrict__ recs,
+                                                                 const uint32_t* __restrict__ dir,
+                                                                 float* __restrict__ grad_tab) {
+    using P = Part<H16>;
+    constexpr uint32_t kSlice = 1u << P::kSliceShift;
+    constexpr uint32_t kCopies = H16 ? kHalfCopies : 1u;
+    constexpr uint32_t kPer = kSlice / kAccThreads;  // entries per thread
+    struct D2 {
+        double x, y;
+    };
+    using Entry = std::conditional_t<H16, __half2, D2>;
+    __shared__ Entry tab[kSlice];  // 32 KB of FP16 pairs, 128 KB of FP64 pairs
+    const uint32_t l = first_level + blockIdx.y, t = threadIdx.x;
+    const uint32_t lane = t % P::kLanes, reader = t / P::kLanes;
+    const uint32_t e0 = blockIdx.x * kSlice, size = gp.size[l];
+    if (e0 >= size) return;
+    const uint32_t n = *n_dev;
+    if (pass0 && n <= pass0) return;  // nothing to add to the first pass's sums
+    const uint32_t used = n > pass0 ? min((n - pass0 + P::kChunkSamples - 1u) / P::kChunkSamples, chunks) : 0u;
+    float2* __restrict__ out = reinterpret_cast<float2*>(grad_tab) + gp.offset[l] + e0;
+    float2 acc[kPer];
+#pragma unroll
+    for (uint32_t q = 0; q < kPer; ++q) {
+        const uint32_t e = t + kAccThreads * q;
+        acc[q] = pass0 && e0 + e < size ? out[e] : make_float2(0.0f, 0.0f);
+    }
+    for (uint32_t copy = 0; copy < kCopies; ++copy) {
+        for (uint32_t q = 0; q < kPer; ++q) {
+            if constexpr (H16)
+                tab[t + kAccThreads * q] = __floats2half2_rn(0.0f, 0.0f);
+            else
+                tab[t + kAccThreads * q] = {0.0, 0.0};
+        }
+        __syncthreads();
+        for (uint32_t ch = copy + reader * kCopies; ch < used; ch += kCopies * (kAccThreads / P::kLanes)) {
+            const size_t c = (size_t)blockIdx.y * chunks + ch;
+            const uint32_t r0 = dir[c * P::kDir + blockIdx.x], r1 = dir[c * P::kDir + blockIdx.x + 1u];
+            const typename P::Rec* __restrict__ rec = recs + c * P::kRecs;
+            for (uint32_t r = r0 + lane; r < r1; r += P::kLanes) {
+                const typename P::Rec x = rec[r];
+                if constexpr (H16) {
+                    unsafeAtomicAdd(&tab[x.idx], x.v);
+                } else {
+                    unsafeAtomicAdd(&tab[x.idx].x, (double)x.x);
+                    unsafeAtomicAdd(&tab[x.idx].y, (double)x.y);
+                }
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (uint32_t q = 0; q < kPer; ++q) {
+            const Entry e = tab[t + kAccThreads * q];
+            if constexpr (H16) {
+                acc[q].x = acc[q].x + __low2float(e);
+                acc[q].y = acc[q].y + __high2float(e);
+            } else {
+                acc[q].x = (float)((double)acc[q].x + e.x);
+                acc[q].y = (float)((double)acc[q].y + e.y);
+            }
+        }
+    }
+#pragma unroll
+    for (uint32_t q = 0; q < kPer; ++q) {
+        const uint32_t e = t + kAccThreads * q;
+        if (e0 + e < size) out[e] = acc[q];
     }
 }
 
@@ -1238,7 +1492,8 @@ void free_workspace_train(TrainState* ts) {
     dev_free(ts->s_cpos); dev_free(ts->s_cdir); dev_free(ts->s_out); dev_free(ts->s_hit);
     dev_free(ts->c_idx); dev_free(ts->c_dout); dev_free(ts->act); dev_free(ts->dact); dev_free(ts->part);
     dev_free(ts->t_buf);
-    dev_free(ts->denc);
+    dev_free(ts->denc); dev_free(ts->recs); dev_free(ts->rec_dir);
+    ts->part_levels = 0;
     dev_free(ts->ray_T); dev_free(ts->ray_alive); dev_free(ts->ray_gbase);
     dev_free(ts->r_pos); dev_free(ts->r_cpos); dev_free(ts->r_cdir); dev_free(ts->r_out);
     ts->ray_cap = ts->sample_cap = ts->compact_cap = 0;
@@ -1274,6 +1529,20 @@ insta_status grow_train_workspace(insta_ctx* ctx, TrainState* ts, uint32_t n_ray
     ok = ok && train_alloc(ts->part, ((cc + kChunk - 1) / kChunk) * n_mlp * sizeof(float));
     ok = ok && train_alloc(ts->t_buf, (size_t)rc * ctx->cfg.max_steps * sizeof(float));
     ok = ok && train_alloc(ts->denc, (size_t)2 * INSTA_MAX_LEVELS * cc * sizeof(float));
+    const GridParams gp = grid_params(ctx);
+    uint32_t largest = 0;
+    for (uint32_t l = 0; l < ctx->cfg.n_levels; ++l) largest = std::max(largest, gp.size[l]);
+    const uint32_t big = ctx->cfg.n_levels - (uint32_t)__builtin_popcount(ts->lds_levels);
+    if (big && cc > kPartMinBatch && largest <= kPartMaxEntries) {
+        const size_t pass = std::min(cc, kPartPass);
+        const size_t c32 = (pass + Part<false>::kChunkSamples - 1) / Part<false>::kChunkSamples;
+        const size_t c16 = (pass + Part<true>::kChunkSamples - 1) / Part<true>::kChunkSamples;
+        const size_t rec_bytes = std::max(c32 * Part<false>::kRecs * sizeof(Part<false>::Rec),
+                                          c16 * Part<true>::kRecs * sizeof(Part<true>::Rec));
+        const size_t dirs = std::max(c32 * Part<false>::kDir, c16 * Part<true>::kDir);
+        ok = ok && train_alloc(ts->recs, big * rec_bytes) && train_alloc(ts->rec_dir, big * dirs * sizeof(uint32_t));
+        if (ok) ts->part_levels = big;
+    }
     if (!ok) {
         free_workspace_train(ts);
         set_error("training workspace allocation failed");
@@ -1310,6 +1579,20 @@ insta_status launch_train_forward(insta_ctx* ctx, TrainState* ts, hipStream_t st
     return INSTA_OK;
 }
 
+template <bool H16>
+void launch_partition(TrainState* ts, const GridParams& gp, uint32_t run_mask, uint32_t pass0, float* grad_tab,
+                      hipStream_t stream) {
+    using P = Part<H16>;
+    const uint32_t cap = ts->compact_cap, first = (uint32_t)__builtin_popcount(ts->lds_levels);
+    const uint32_t chunks = (std::min(cap - pass0, kPartPass) + P::kChunkSamples - 1) / P::kChunkSamples;
+    typename P::Rec* recs = reinterpret_cast<typename P::Rec*>(ts->recs);
+    const uint32_t* n_dev = ts->counters + kTCompactN;
+    hipLaunchKernelGGL(partition_kernel<H16>, dim3(chunks, ts->part_levels), dim3(P::kChunkSamples), 0, stream, gp,
+                       first, run_mask, pass0, n_dev, ts->c_idx, ts->s_cpos, ts->denc, cap, recs, ts->rec_dir);
+    hipLaunchKernelGGL(accumulate_kernel<H16>, dim3(P::kMaxSlices, ts->part_levels), dim3(kAccThreads), 0, stream, gp,
+                       first, pass0, chunks, n_dev, recs, ts->rec_dir, grad_tab);
+}
+
 template <int L, int X>
 insta_status launch_train_backward(insta_ctx* ctx, TrainState* ts, const insta_train_config& tc, hipStream_t stream) {
     constexpr int DIN = 2 * L + X;
@@ -1337,16 +1620,24 @@ insta_status launch_train_backward(insta_ctx* ctx, TrainState* ts, const insta_t
     if (lds_mask) {
         const dim3 grid(chunks, __builtin_popcount(lds_mask));
         if (tc.grid_grad_fp16)
-            hipLaunchKernelGGL(scatter_lds_kernel<true>, grid, dim3(kScatterThreads), 0, stream, gp, n_dev, ts->c_idx,
+            hipLaunchKernelGGL(scatter_lds_kernel, grid, dim3(kScatterThreads), 0, stream, gp, n_dev, ts->c_idx,
                                ts->s_cpos, ts->denc, cap, run_mask, ts->grad_p, lds_end);
         else
-            hipLaunchKernelGGL(scatter_lds_kernel<false>, grid, dim3(kScatterThreads), 0, stream, gp, n_dev, ts->c_idx,
-                               ts->s_cpos, ts->denc, cap, run_mask, ts->grad_p, lds_end);
+            hipLaunchKernelGGL(scatter_lds64_kernel, dim3(grid.x, grid.y, 2), dim3(kScatterThreads), 0, stream, gp,
+                               n_dev, ts->c_idx, ts->s_cpos, ts->denc, cap, ts->grad_p, lds_end);
         hipLaunchKernelGGL(grad_partials_reduce_kernel, dim3((lds_end + 255) / 256), dim3(256), 0, stream, ts->grad_p,
                            lds_end, chunks, grad_tab);
         INSTA_HIP(hipGetLastError());
     }
-    if (big_mask) {
+    if (big_mask && ts->part_levels) {
+        for (uint32_t pass0 = 0; pass0 < cap; pass0 += kPartPass) {
+            if (tc.grid_grad_fp16)
+                launch_partition<true>(ts, gp, run_mask, pass0, grad_tab, stream);
+            else
+                launch_partition<false>(ts, gp, run_mask, pass0, grad_tab, stream);
+        }
+        INSTA_HIP(hipGetLastError());
+    } else if (big_mask) {
         const uint64_t entries = ctx->layout.n_grid_params / 2;
         const uint32_t blocks =
             ((cap + kLevelThreads - 1) / kLevelThreads + kHalfCopies - 1) / kHalfCopies * kHalfCopies;
@@ -1362,6 +1653,10 @@ insta_status launch_train_backward(insta_ctx* ctx, TrainState* ts, const insta_t
             hipLaunchKernelGGL(grad_copies_reduce_kernel, dim3(2048), dim3(256), 0, stream, ts->grad_h,
                                (uint64_t)lds_end, entries, grad_tab);
         } else {
+            // the added-to gradients start at zero (a fill kernel: capturable);
+            // every other path writes all of its gradients
+            hipLaunchKernelGGL(fill_zero_kernel, dim3(1024), dim3(256), 0, stream,
+                               reinterpret_cast<uint32_t*>(grad_tab + 2 * (size_t)lds_end), 2 * (entries - lds_end));
             hipLaunchKernelGGL(scatter_levels_kernel<false>, grid, dim3(kLevelThreads), 0, stream, gp, big_mask,
                                run_mask, blocks, n_dev, ts->c_idx, ts->s_cpos, ts->denc, cap, grad_tab, ts->grad_h,
                                entries);
@@ -1655,8 +1950,6 @@ insta_status train_step(insta_ctx* ctx, const insta_train_config& tc, insta_trai
     const uint64_t np = ctx->layout.n_params, n_mlp = ctx->layout.n_mlp_params;
     // the marched-sample cap is the step's (a larger reservation changes nothing)
     const uint32_t cap = tc.max_samples;
-    // zero gradients with a fill kernel (capturable, unlike memset nodes)
-    hipLaunchKernelGGL(fill_zero_kernel, dim3(1024), dim3(256), 0, stream, reinterpret_cast<uint32_t*>(ts->grad), np);
     hipLaunchKernelGGL(train_clear_kernel, dim3(1), dim3(64), 0, stream, ts->counters, cap);
     INSTA_HIP(hipGetLastError());
 
@@ -1952,8 +2245,6 @@ insta_status network_backward(insta_ctx* ctx, uint32_t n, uint32_t stride, const
     TrainState* ts = ctx->train;
     const uint64_t np = ctx->layout.n_params;
     INSTA_HIP(hipMemcpyAsync(ts->c_dout, dL_dout, (size_t)n * sizeof(float4), hipMemcpyDeviceToDevice, stream));
-    hipLaunchKernelGGL(fill_zero_kernel, dim3(1024), dim3(256), 0, stream, reinterpret_cast<uint32_t*>(ts->grad), np);
-    INSTA_HIP(hipGetLastError());
     insta_train_config tc{};
     tc.grid_grad_fp16 = 0;
     const bool x16 = ctx->cfg.n_extra_dims != 0;
