@@ -714,7 +714,8 @@ INSTA_DEV float2 run_sum(uint32_t key, float2 v, bool& head) {
 // the table holds doubles, one feature of them; recomputing the corners for
 // the other feature costs less than the adds did, and neither conflicts nor
 // runs of equal entries need care.  The sums are exact but for one rounding.
-// LDS64_FIGURES
+// 237,000 samples on the eight levels of the small shapes: 77 us, with FP32 atomics and run sums 167; 100,003
+// random samples, two levels: 30 us against 194.
 // H16 (scatter_lds_kernel): one workgroup per (chunk, level), packed FP16
 // atomics, one per corner; on levels in run_mask a wave first sums runs of
 // consecutive samples with one corner.
@@ -891,16 +892,20 @@ __global__ __launch_bounds__(kScatterThreads) void scatter_lds_kernel(GridParams
 // tables (by block of kLevelThreads samples; a level's first copy before its
 // second), which keep the rounding of many small adds in check and are summed
 // in a fixed order afterwards.
-// Bound by the L2's atomics.  LEVELS_FIGURES
+// Bound by the L2's atomics, about one request per clock and XCD: 100,003
+// random samples at full size (14 levels of up to 2^19 entries) take 698 us,
+// added per sample into one copy of the tables per XCD they took 1,300.
 constexpr uint32_t kLevelThreads = 256;
 constexpr uint32_t kHalfCopies = 8;
 // Batches above kPartMinBatch, with no table above kPartMaxEntries (the
 // partition's directory), are partitioned, kPartPass samples at a time (352 MB
-// of records at full size); below, the fixed work of walking every slice costs
-// more than the atomics.  PARTITION_LINE
+// of records at full size).  Below, the atomics are cheaper than the fixed
+// work of walking every slice and storing every entry: about 7 us per 1,000
+// samples against 60 us.
 constexpr uint32_t kPartMinBatch = 8192;
 constexpr uint32_t kPartMaxEntries = 1u << 19;
 constexpr uint32_t kPartPass = 1u << 18;
+constexpr uint32_t kPartSlices = 64;  // one wave scans a chunk's slice counts
 template <bool H16>
 __global__ __launch_bounds__(kLevelThreads) void scatter_levels_kernel(GridParams gp, uint32_t level_mask,
                                                                        uint32_t run_mask, uint32_t blocks,
@@ -983,18 +988,19 @@ __global__ __launch_bounds__(kLevelThreads) void scatter_levels_kernel(GridParam
 // accumulate_kernel, one workgroup per (slice, level), adds its slice's records
 // of every chunk into an LDS copy of the slice and stores it: every entry of
 // the level is written once, so the gradients need no clearing either.
-// FP32: 12-byte records, slices of 8,192 entries, FP64 LDS atomics (as
+// FP32: 12-byte records, slices of up to 8,192 entries, FP64 LDS atomics (as
 // scatter_lds64_kernel).  H16: 8-byte records of FP16 pairs (runs summed first,
 // as in scatter_levels_kernel), the same slices; chunk c is of copy
 // c % kHalfCopies, and the slice's copies are accumulated one after the other
 // and summed in order.  Bound by the records' trip through memory (8 corners
-// x 12 bytes, written and read).  PARTITION_FIGURES
+// x 12 bytes, written and read) and, FP16, its LDS atomics: 100,003 random
+// samples at full size take 50 + 82 us (scatter_levels_kernel: 698), the
+// 225,000 samples of a training step under FP16 83 + 140 us (718).  With
+// slices of 8,192 entries on every level the small dense ones, a few crowded
+// slices, set the second kernel's time (310 and 250 us).
 template <bool H16>
 struct Part {
     static constexpr uint32_t kChunkSamples = H16 ? kLevelThreads : 1024u;
-    static constexpr uint32_t kSliceShift = 13u;
-    static constexpr uint32_t kMaxSlices = kPartMaxEntries >> kSliceShift;
-    static_assert(kMaxSlices <= 64u, "one wave scans a chunk's slices");
     static constexpr uint32_t kLanes = H16 ? 32u : 64u;  // lanes reading one chunk's records
     struct Rec32 {
         uint32_t idx;
@@ -1005,10 +1011,18 @@ struct Part {
         __half2 v;
     };
     using Rec = std::conditional_t<H16, Rec16, Rec32>;
+    static constexpr uint32_t kMaxChunks = kPartPass / kChunkSamples;
     // per chunk: record slots, directory words (first record of each slice, end)
     static constexpr uint32_t kRecs = 8u * kChunkSamples;
-    static constexpr uint32_t kDir = kMaxSlices + 1u;
+    static constexpr uint32_t kDir = kPartSlices + 1u;
 };
+// A level has at most kPartSlices slices of 2^shift entries, and above 32 of
+// them: a small dense level's records, which all fall near the skin, still
+// spread over many workgroups.
+INSTA_DEV uint32_t slice_shift(uint32_t size) {
+    const uint32_t m = (size - 1u) / kPartSlices;
+    return m ? 32u - (uint32_t)__builtin_clz(m) : 0u;
+}
 
 template <bool H16>
 __global__ __launch_bounds__(Part<H16>::kChunkSamples) void partition_kernel(
@@ -1016,14 +1030,14 @@ __global__ __launch_bounds__(Part<H16>::kChunkSamples) void partition_kernel(
     const uint32_t* __restrict__ c_idx, const float4* __restrict__ cpos, const float* __restrict__ denc_g, uint32_t ld,
     typename Part<H16>::Rec* __restrict__ recs, uint32_t* __restrict__ dir) {
     using P = Part<H16>;
-    __shared__ uint32_t s_cnt[P::kMaxSlices], s_base[P::kMaxSlices];
+    __shared__ uint32_t s_cnt[kPartSlices], s_base[kPartSlices];
     const uint32_t n = *n_dev, s0 = pass0 + blockIdx.x * P::kChunkSamples;
     if (s0 >= n) return;
     const uint32_t l = first_level + blockIdx.y, t = threadIdx.x;
-    const uint32_t size = gp.size[l], res = gp.res[l];
+    const uint32_t size = gp.size[l], res = gp.res[l], shift = slice_shift(size);
     const bool dense_l = (gp.dense_mask >> l) & 1u;
     const float sc = gp.scale[l];
-    for (uint32_t j = t; j < P::kMaxSlices; j += P::kChunkSamples) s_cnt[j] = 0u;
+    for (uint32_t j = t; j < kPartSlices; j += P::kChunkSamples) s_cnt[j] = 0u;
     __syncthreads();
     const bool valid = s0 + t < n;
     const uint32_t i = valid ? s0 + t : n - 1u;  // tail lanes repeat the last sample and emit nothing
@@ -1062,7 +1076,7 @@ __global__ __launch_bounds__(Part<H16>::kChunkSamples) void partition_kernel(
             }
         }
         if (lead)
-            rank[c] = atomicAdd(&s_cnt[idx[c] >> P::kSliceShift], 1u);
+            rank[c] = atomicAdd(&s_cnt[idx[c] >> shift], 1u);
         else
             idx[c] = ~0u;
     }
@@ -1070,17 +1084,17 @@ __global__ __launch_bounds__(Part<H16>::kChunkSamples) void partition_kernel(
     // first record of each slice (one wave; at most 64 slices)
     const size_t chunk = (size_t)blockIdx.y * gridDim.x + blockIdx.x;
     if (t < 64u) {
-        const uint32_t cnt = t < P::kMaxSlices ? s_cnt[t] : 0u;
+        const uint32_t cnt = t < kPartSlices ? s_cnt[t] : 0u;
         uint32_t incl = cnt;
 #pragma unroll
         for (uint32_t o = 1; o < 64u; o <<= 1) {
             const uint32_t up = __shfl_up(incl, o);
             if (t >= o) incl += up;
         }
-        if (t < P::kMaxSlices) {
+        if (t < kPartSlices) {
             s_base[t] = incl - cnt;
             dir[chunk * P::kDir + t] = incl - cnt;
-            if (t == P::kMaxSlices - 1u) dir[chunk * P::kDir + t + 1u] = incl;
+            if (t == kPartSlices - 1u) dir[chunk * P::kDir + t + 1u] = incl;
         }
     }
     __syncthreads();
@@ -1088,8 +1102,8 @@ __global__ __launch_bounds__(Part<H16>::kChunkSamples) void partition_kernel(
 #pragma unroll
     for (uint32_t c = 0; c < 8; ++c) {
         if (idx[c] == ~0u) continue;
-        const uint32_t slot = s_base[idx[c] >> P::kSliceShift] + rank[c];
-        const uint32_t e = idx[c] & ((1u << P::kSliceShift) - 1u);
+        const uint32_t slot = s_base[idx[c] >> shift] + rank[c];
+        const uint32_t e = idx[c] & ((1u << shift) - 1u);
         if constexpr (H16)
             out[slot] = {e, __floats2half2_rn(v[c].x, v[c].y)};
         else
@@ -1105,7 +1119,7 @@ __global__ __launch_bounds__(kAccThreads) void accumulate_kernel(GridParams gp, 
                                                                  const uint32_t* __restrict__ dir,
                                                                  float* __restrict__ grad_tab) {
     using P = Part<H16>;
-    constexpr uint32_t kSlice = 1u << P::kSliceShift;
+    constexpr uint32_t kSlice = kPartMaxEntries / kPartSlices;
     constexpr uint32_t kCopies = H16 ? kHalfCopies : 1u;
     constexpr uint32_t kPer = kSlice / kAccThreads;  // entries per thread
     struct D2 {
@@ -1113,59 +1127,75 @@ __global__ __launch_bounds__(kAccThreads) void accumulate_kernel(GridParams gp, 
     };
     using Entry = std::conditional_t<H16, __half2, D2>;
     __shared__ Entry tab[kSlice];  // 32 KB of FP16 pairs, 128 KB of FP64 pairs
+    __shared__ uint2 s_dir[P::kMaxChunks];  // this slice's records of each chunk
     const uint32_t l = first_level + blockIdx.y, t = threadIdx.x;
     const uint32_t lane = t % P::kLanes, reader = t / P::kLanes;
-    const uint32_t e0 = blockIdx.x * kSlice, size = gp.size[l];
+    const uint32_t size = gp.size[l], shift = slice_shift(size), e0 = blockIdx.x << shift;
     if (e0 >= size) return;
+    const uint32_t here = min(1u << shift, size - e0);
     const uint32_t n = *n_dev;
     if (pass0 && n <= pass0) return;  // nothing to add to the first pass's sums
     const uint32_t used = n > pass0 ? min((n - pass0 + P::kChunkSamples - 1u) / P::kChunkSamples, chunks) : 0u;
+    for (uint32_t ch = t; ch < used; ch += kAccThreads) {
+        const uint32_t* d = dir + ((size_t)blockIdx.y * chunks + ch) * P::kDir + blockIdx.x;
+        s_dir[ch] = make_uint2(d[0], d[1]);
+    }
     float2* __restrict__ out = reinterpret_cast<float2*>(grad_tab) + gp.offset[l] + e0;
     float2 acc[kPer];
 #pragma unroll
     for (uint32_t q = 0; q < kPer; ++q) {
         const uint32_t e = t + kAccThreads * q;
-        acc[q] = pass0 && e0 + e < size ? out[e] : make_float2(0.0f, 0.0f);
+        acc[q] = pass0 && e < here ? out[e] : make_float2(0.0f, 0.0f);
     }
     for (uint32_t copy = 0; copy < kCopies; ++copy) {
-        for (uint32_t q = 0; q < kPer; ++q) {
+        for (uint32_t e = t; e < here; e += kAccThreads) {
             if constexpr (H16)
-                tab[t + kAccThreads * q] = __floats2half2_rn(0.0f, 0.0f);
+                tab[e] = __floats2half2_rn(0.0f, 0.0f);
             else
-                tab[t + kAccThreads * q] = {0.0, 0.0};
+                tab[e] = {0.0, 0.0};
         }
         __syncthreads();
         for (uint32_t ch = copy + reader * kCopies; ch < used; ch += kCopies * (kAccThreads / P::kLanes)) {
-            const size_t c = (size_t)blockIdx.y * chunks + ch;
-            const uint32_t r0 = dir[c * P::kDir + blockIdx.x], r1 = dir[c * P::kDir + blockIdx.x + 1u];
-            const typename P::Rec* __restrict__ rec = recs + c * P::kRecs;
-            for (uint32_t r = r0 + lane; r < r1; r += P::kLanes) {
-                const typename P::Rec x = rec[r];
+            const uint2 seg = s_dir[ch];
+            const typename P::Rec* __restrict__ rec = recs + ((size_t)blockIdx.y * chunks + ch) * P::kRecs;
+            auto add = [&](const typename P::Rec& x) {
                 if constexpr (H16) {
                     unsafeAtomicAdd(&tab[x.idx], x.v);
                 } else {
                     unsafeAtomicAdd(&tab[x.idx].x, (double)x.x);
                     unsafeAtomicAdd(&tab[x.idx].y, (double)x.y);
                 }
+            };
+            uint32_t r = seg.x + lane;
+            for (; r + 3u * P::kLanes < seg.y; r += 4u * P::kLanes) {  // four loads in flight
+                const typename P::Rec a = rec[r], b = rec[r + P::kLanes], c = rec[r + 2u * P::kLanes],
+                                      d = rec[r + 3u * P::kLanes];
+                add(a);
+                add(b);
+                add(c);
+                add(d);
             }
+            for (; r < seg.y; r += P::kLanes) add(rec[r]);
         }
         __syncthreads();
 #pragma unroll
         for (uint32_t q = 0; q < kPer; ++q) {
-            const Entry e = tab[t + kAccThreads * q];
+            const uint32_t e = t + kAccThreads * q;
+            if (e >= here) break;
+            const Entry v = tab[e];
             if constexpr (H16) {
-                acc[q].x = acc[q].x + __low2float(e);
-                acc[q].y = acc[q].y + __high2float(e);
+                acc[q].x = acc[q].x + __low2float(v);
+                acc[q].y = acc[q].y + __high2float(v);
             } else {
-                acc[q].x = (float)((double)acc[q].x + e.x);
-                acc[q].y = (float)((double)acc[q].y + e.y);
+                acc[q].x = (float)((double)acc[q].x + v.x);
+                acc[q].y = (float)((double)acc[q].y + v.y);
             }
         }
     }
 #pragma unroll
     for (uint32_t q = 0; q < kPer; ++q) {
         const uint32_t e = t + kAccThreads * q;
-        if (e0 + e < size) out[e] = acc[q];
+        if (e < here) out[e] = acc[q];
     }
 }
 
@@ -1589,7 +1619,7 @@ void launch_partition(TrainState* ts, const GridParams& gp, uint32_t run_mask, u
     const uint32_t* n_dev = ts->counters + kTCompactN;
     hipLaunchKernelGGL(partition_kernel<H16>, dim3(chunks, ts->part_levels), dim3(P::kChunkSamples), 0, stream, gp,
                        first, run_mask, pass0, n_dev, ts->c_idx, ts->s_cpos, ts->denc, cap, recs, ts->rec_dir);
-    hipLaunchKernelGGL(accumulate_kernel<H16>, dim3(P::kMaxSlices, ts->part_levels), dim3(kAccThreads), 0, stream, gp,
+    hipLaunchKernelGGL(accumulate_kernel<H16>, dim3(kPartSlices, ts->part_levels), dim3(kAccThreads), 0, stream, gp,
                        first, pass0, chunks, n_dev, recs, ts->rec_dir, grad_tab);
 }
 
