@@ -257,7 +257,7 @@ __global__ __launch_bounds__(kDeformThreads) void deform_aos_kernel(MeshSet ms, 
 //         the sample was deformed off the lips region (mask 7), else the
 //         frame's values (warp only overwrites them in the first case,
 //         src/core.cu:514-519).
-constexpr uint32_t kMaxBlocks = 65536;
+constexpr uint32_t kMaxBlocks = 16384;  // larger launches stride (an empty round's blocks cost little)
 
 // Frame of a sample: the per-ray table when given (training batches mix
 // frames), else the call's frame; -1 leaves the sample undeformed.

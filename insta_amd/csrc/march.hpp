@@ -73,15 +73,85 @@ INSTA_DEV float advance_to_next_voxel(float t, float dt, V3 pos, V3 dir, V3 idir
     return t;
 }
 
+// The walk along a ray (one step per sample, one jump per empty voxel) waits
+// for an occupancy bit before each step, and neither step needs it: the next
+// position if this one is occupied (t + dt) and if it is empty (the next
+// voxel) depend on t alone.  So kSpec positions ahead are formed as if the
+// ray stayed in occupied cells (or in empty ones, whichever it was in last),
+// their bits are loaded together, and the walk takes them in order up to the
+// first that is different: the t values visited are those of the walk one bit
+// at a time.  Bound by that chain of loads in small frames (64 x 64 of the
+// small sphere, 85 samples a ray: 124 -> 108 us with the rays' t values
+// reloaded four at a time too; eight ahead: 7 % slower) and by the vector ALUs
+// in large ones.
+constexpr int kSpec = 4;
+struct Ahead {
+    float t[kSpec + 1];
+    bool in[kSpec], occ[kSpec];
+    INSTA_DEV Ahead(const RenderArgs& a, V3 o, V3 d, V3 idir, float t0, bool through_occupied) {
+        t[0] = t0;
+#pragma unroll
+        for (int q = 0; q < kSpec; ++q) {
+            const V3 pos = o + d * t[q];
+            in[q] = box_contains(a, pos);
+            occ[q] = occupied(a.grid, a.G, pos);
+            // (a position outside the box ends the walk: nothing is formed past it)
+            t[q + 1] = through_occupied ? t[q] + a.dt
+                                        : (in[q] ? advance_to_next_voxel(t[q], a.dt, pos, d, idir, a.G) : t[q]);
+        }
+    }
+};
+
 // Walk from t to the next occupied position inside the box.  Returns false
 // if the ray leaves the box first.
-INSTA_DEV bool skip_empty(const RenderArgs& a, V3 o, V3 d, V3 idir, float& t, V3& pos) {
+INSTA_DEV bool skip_empty(const RenderArgs& a, V3 o, V3 d, V3 idir, float& t) {
     while (true) {
-        pos = o + d * t;
-        if (!box_contains(a, pos)) return false;
-        if (occupied(a.grid, a.G, pos)) return true;
-        t = advance_to_next_voxel(t, a.dt, pos, d, idir, a.G);
+        const Ahead w(a, o, d, idir, t, false);
+#pragma unroll
+        for (int q = 0; q < kSpec; ++q) {
+            t = w.t[q];
+            if (!w.in[q]) return false;
+            if (w.occ[q]) return true;
+        }
+        t = w.t[kSpec];
     }
+}
+
+// Up to `most` samples from t: sample(j, t) for each, in order; t ends at the
+// next unvisited position.  exited: the ray left the box.
+template <class Sample>
+INSTA_DEV uint32_t walk_samples(const RenderArgs& a, V3 o, V3 d, V3 idir, float& t, uint32_t most, bool& exited,
+                                Sample&& sample) {
+    uint32_t count = 0;
+    bool through = true;  // the last position seen was occupied
+    exited = false;
+    while (count < most && !exited) {
+        const Ahead w(a, o, d, idir, t, through);
+        bool go = true;
+        float at = t;
+        t = w.t[kSpec];
+#pragma unroll
+        for (int q = 0; q < kSpec; ++q) {
+            if (!go) continue;
+            if (count >= most || !w.in[q]) {
+                exited = count < most;
+                t = w.t[q];
+                go = false;
+            } else {
+                if (w.occ[q]) sample(count++, w.t[q]);
+                if (w.occ[q] != through) {  // the positions ahead were formed the other way
+                    at = w.t[q];
+                    go = false;
+                    t = -1.0f;
+                }
+            }
+        }
+        if (t == -1.0f) {
+            through = !through;
+            t = through ? at + a.dt : advance_to_next_voxel(at, a.dt, o + d * at, d, idir, a.G);
+        }
+    }
+    return count;
 }
 
 INSTA_DEV float box_ray_tmin(const RenderArgs& a, V3 o, V3 d) {
@@ -99,33 +169,42 @@ INSTA_DEV float box_ray_tmin(const RenderArgs& a, V3 o, V3 d) {
     return tmin;
 }
 
-// wave-aggregated append: returns this lane's slot (only meaningful if `want`)
-INSTA_DEV uint32_t wave_append(uint32_t* counter, bool want) {
-    const uint64_t mask = __ballot(want);
-    if (mask == 0) return 0;
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t leader = __ffsll((unsigned long long)mask) - 1;
-    uint32_t base = 0;
-    if (lane == leader) base = atomicAdd(counter, (uint32_t)__popcll(mask));
-    base = __shfl(base, leader);
-    const uint64_t below = mask & ((1ull << lane) - 1ull);
-    return base + (uint32_t)__popcll(below);
-}
+// Reservations: one atomic per workgroup of `kWaves` full waves, every thread
+// calling.  Atomics on one counter retire one at a time over the whole chip,
+// about 6.4 ns each (with one per wave, the 16,384 waves of a 1024 x 1024
+// frame spent 105 us of their ray set-up on it), so a workgroup sums its
+// waves' counts in LDS first.
 
-// wave-wide exclusive prefix sum of `v` plus one atomic reservation
-INSTA_DEV uint32_t wave_reserve(uint32_t* counter, uint32_t v) {
-    const uint32_t lane = threadIdx.x & 63u;
+// exclusive prefix of v over the workgroup, plus one atomic reservation
+template <uint32_t kWaves>
+INSTA_DEV uint32_t block_reserve(uint32_t* counter, uint32_t v) {
+    __shared__ uint32_t s_wave[kWaves], s_base;
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     uint32_t incl = v;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
         const uint32_t up = __shfl_up(incl, o);
         if (lane >= (uint32_t)o) incl += up;
     }
-    const uint32_t total = __shfl(incl, 63);
-    uint32_t base = 0;
-    if (lane == 63 && total > 0) base = atomicAdd(counter, total);
-    base = __shfl(base, 63);
-    return base + incl - v;
+    if (lane == 63u) s_wave[wave] = incl;
+    __syncthreads();
+    uint32_t before = 0, total = 0;
+#pragma unroll
+    for (uint32_t w = 0; w < kWaves; ++w) {
+        if (w < wave) before += s_wave[w];
+        total += s_wave[w];
+    }
+    if (threadIdx.x == 0) s_base = total ? atomicAdd(counter, total) : 0u;
+    __syncthreads();
+    const uint32_t slot = s_base + before + incl - v;
+    __syncthreads();  // a later reservation reuses the LDS words
+    return slot;
+}
+
+// this thread's slot in a list (only meaningful if `want`)
+template <uint32_t kWaves>
+INSTA_DEV uint32_t block_append(uint32_t* counter, bool want) {
+    return block_reserve<kWaves>(counter, want ? 1u : 0u);
 }
 
 INSTA_DEV uint32_t wave_max(uint32_t v) {

@@ -6,7 +6,8 @@
 //   init      one thread per pixel: pinhole ray, render-box entry, one-step
 //             ld jitter and empty-space skip; live rays appended to a list
 //   repeat    march: each live ray emits up to K samples (K = sample
-//                    capacity / live rays, computed on the device), one
+//                    capacity / live rays, at most the round's window, computed
+//                    on the device), one
 //                    walk with t to scratch; a wave's samples take one
 //                    contiguous range (one atomic), step-major inside it:
 //                    step j of the wave's 64 adjacent rays side by side, so
@@ -21,8 +22,9 @@
 //   finalize  one thread per pixel writes RGBA/depth/step counts.
 // Each ray's samples depend only on its own t sequence, so the result does
 // not depend on K or on the order rays are processed in.  Live counts stay on
-// the device: the first round is queued with init and finalize, and the host
+// the device: the first rounds are queued with init and finalize, and the host
 // reads the counters once, adding rounds only for rays still live.
+#include <algorithm>
 #include <cmath>
 #include <type_traits>
 
@@ -33,6 +35,26 @@ namespace insta {
 namespace {
 
 constexpr uint32_t kRayThreads = 256;
+constexpr uint32_t kRayWaves = kRayThreads / 64;
+constexpr uint32_t kInitThreads = 256;   // (1,024: fewer reservations, slower small frames)
+
+// Windows: a trained avatar's rays end within a few samples of the skin, so a
+// frame of at least kWindowPixels evaluates its rays' samples in rounds of
+// kWindow, kWindow, 2 kWindow, 4 kWindow, ... and only while the rays live; a
+// smaller frame, where a round's launches cost more than its samples, takes
+// them all in one.  A 1024 x 1024 FP16 frame of a head with an opaque skin
+// (50 samples marched per live ray, 25 composited) takes 3.41 ms, in one round
+// 4.35 ms (first windows of 8 and 16: 3.64 and 3.57 ms); a 512 x 512 frame of a
+// translucent volume, whose rays end nowhere, takes one more round, 50 us of
+// 2.4 ms.
+constexpr uint32_t kWindow = 12;
+constexpr uint32_t kWindowPixels = 1u << 15;
+constexpr uint32_t kAllSamples = 0xffffffffu;
+constexpr float kClearAlpha = 0.02f;
+uint32_t round_window(uint32_t n_pix, bool whole, uint32_t round) {
+    if (whole || n_pix < kWindowPixels) return kAllSamples;
+    return round < 2 ? kWindow : (round < 12 ? kWindow << (round - 1) : kAllSamples);
+}
 
 enum : uint32_t {
     kCntAliveA = 0,
@@ -44,6 +66,9 @@ enum : uint32_t {
     kCntRounds = 6,
     kCntMisses = 7,   // in-box samples whose nearest-triangle query found nothing
     kCntQueue = 8,    // queries left for the deformation's second pass
+    kCntLimit = 9,    // samples a ray may emit this round
+    kCntOpaque = 10,  // rays ended by opacity so far
+    kCntClear = 11,   // rays that go on from this round with next to no opacity
     kNumCounters = 16
 };
 
@@ -57,7 +82,7 @@ INSTA_HD uint32_t tiled_threads(uint32_t w, uint32_t h) {
     return ((w + kTile - 1) / kTile) * ((h + kTile - 1) / kTile) * kTile * kTile;
 }
 
-__global__ __launch_bounds__(kRayThreads) void init_rays_kernel(RenderArgs a, float4* __restrict__ r_o,
+__global__ __launch_bounds__(kInitThreads) void init_rays_kernel(RenderArgs a, float4* __restrict__ r_o,
                                                                 float4* __restrict__ r_d, float4* __restrict__ r_rgba,
                                                                 float* __restrict__ r_depth,
                                                                 uint32_t* __restrict__ r_steps,
@@ -84,8 +109,7 @@ __global__ __launch_bounds__(kRayThreads) void init_rays_kernel(RenderArgs a, fl
         if (box_contains(a, o + d * t)) {
             const V3 idir = v3(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
             t += ld_random_val0(a.spp, i * 786433u) * a.dt;  // advance_pos_nerf (testbed_nerf.cu:663-664)
-            V3 pos;
-            live = skip_empty(a, o, d, idir, t, pos);
+            live = skip_empty(a, o, d, idir, t);
         }
         r_o[i] = make_float4(o.x, o.y, o.z, t);
         r_d[i] = make_float4(d.x, d.y, d.z, 0.0f);
@@ -93,7 +117,7 @@ __global__ __launch_bounds__(kRayThreads) void init_rays_kernel(RenderArgs a, fl
         r_depth[i] = 0.0f;
         r_steps[i] = 0;
     }
-    const uint32_t slot = wave_append(&counters[kCntAliveA], live);
+    const uint32_t slot = block_append<kInitThreads / 64>(&counters[kCntAliveA], live);
     if (live) alive[slot] = i;
     // counters[kCntAlive0] is derived from the first live count on the host
 }
@@ -114,9 +138,10 @@ __global__ __launch_bounds__(kRayThreads) void march_kernel(RenderArgs a, const 
                                                             uint32_t* __restrict__ counters) {
     const uint32_t n_alive = *n_alive_dev;
     const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-    if ((k & ~63u) >= n_alive) return;  // whole wave past the live list
+    if (blockIdx.x * kRayThreads >= n_alive) return;  // whole workgroup past the live list
     // samples per live ray this round: all fit the sample buffer
     uint64_t K64 = sample_cap / n_alive;
+    if (K64 > counters[kCntLimit]) K64 = counters[kCntLimit];
     if (K64 > a.max_steps) K64 = a.max_steps;
     if (K64 < 1) K64 = 1;
     const uint32_t K = (uint32_t)K64;
@@ -135,34 +160,25 @@ __global__ __launch_bounds__(kRayThreads) void march_kernel(RenderArgs a, const 
         const uint32_t done = r_steps[r];
         const uint32_t budget = a.max_steps > done ? a.max_steps - done : 0u;
         const uint32_t kmax = K < budget ? K : budget;
-        // one loop iteration per sample or per empty-voxel skip (the t
-        // sequence of skip_empty + t += dt, without a nested loop whose trip
-        // count differs between lanes)
-        while (count < kmax) {
-            const V3 pos = o + d * t;
-            if (!box_contains(a, pos)) {
-                exited = true;
-                break;
-            }
-            if (occupied(a.grid, a.G, pos)) {
-                t_buf[(size_t)count * n_alive + k] = t;
-                ++count;
-                t += a.dt;
-            } else {
-                t = advance_to_next_voxel(t, a.dt, pos, d, idir, a.G);
-            }
-        }
+        count = walk_samples(a, o, d, idir, t, kmax, exited,
+                             [&](uint32_t j, float tj) { t_buf[(size_t)j * n_alive + k] = tj; });
     }
     // the wave's samples are one contiguous range, written step-major
-    const uint32_t wave_base = __shfl(wave_reserve(&counters[kCntSamples], count), 0);
+    const uint32_t wave_base = __shfl(block_reserve<kRayWaves>(&counters[kCntSamples], count), 0);
     const uint32_t maxc = wave_max(count);
     StepMajor sm;
-    for (uint32_t j = 0; j < maxc; ++j) {
-        bool mine;
-        const uint32_t slot = sm.next(j, count, mine);
-        if (mine) {
-            const V3 pos = o + d * t_buf[(size_t)j * n_alive + k];
-            s_pos[wave_base + slot] = make_float4(pos.x, pos.y, pos.z, __uint_as_float(r));
+    for (uint32_t j0 = 0; j0 < maxc; j0 += kSpec) {
+        float tj[kSpec];  // loaded together
+#pragma unroll
+        for (uint32_t q = 0; q < kSpec; ++q) tj[q] = j0 + q < count ? t_buf[(size_t)(j0 + q) * n_alive + k] : 0.0f;
+#pragma unroll
+        for (uint32_t q = 0; q < kSpec; ++q) {
+            bool mine;
+            const uint32_t slot = sm.next(j0 + q, count, mine);
+            if (mine) {
+                const V3 pos = o + d * tj[q];
+                s_pos[wave_base + slot] = make_float4(pos.x, pos.y, pos.z, __uint_as_float(r));
+            }
         }
     }
     if (!valid) return;
@@ -190,13 +206,13 @@ __global__ __launch_bounds__(kRayThreads) void composite_kernel(RenderArgs a, co
         counters[kCntEmitted] += counters[kCntSamples];
         counters[kCntRounds] += 1;
     }
-    if ((k & ~63u) >= n_alive) return;
+    if (blockIdx.x * kRayThreads >= n_alive) return;
     const bool valid = k < n_alive;
-    bool keep = false;
+    bool keep = false, opaque = false, clear = false;
     uint32_t r = 0, used = 0;
     // the march's step-major layout of this wave's samples
     const uint32_t cnt = valid ? r_cnt[k] : 0u;
-    const uint32_t off = r_off[k & ~63u];  // the wave's base (lane 0 is live)
+    const uint32_t off = (k & ~63u) < n_alive ? r_off[k & ~63u] : 0u;  // the wave's base
     const uint32_t maxc = wave_max(cnt);
     if (valid) {
         r = alive[k];
@@ -208,46 +224,80 @@ __global__ __launch_bounds__(kRayThreads) void composite_kernel(RenderArgs a, co
         const V3 cam_fwd = v3(a.M[2], a.M[6], a.M[10]);
         bool terminated = false;
         StepMajor sm;
-        for (uint32_t j = 0; j < maxc; ++j) {
+        // each step's network output is loaded two steps ahead of its use; the
+        // position behind the depth is the heaviest sample's, read once
+        constexpr uint32_t kLead = 2;
+        float4 ahead[kLead];
+        uint32_t slots[kLead], heaviest = kAllSamples;
+#pragma unroll
+        for (uint32_t q = 0; q < kLead; ++q) {
             bool mine;
-            const uint32_t slot = sm.next(j, cnt, mine);
-            if (!mine || terminated) continue;
-            const float4 out = s_out[off + slot];
-            const float4 sp = s_pos[off + slot];
-            // composite_kernel_nerf (testbed_nerf.cu:853-999), render mode Shade
-            const float T = 1.0f - acc.w;
-            const float sigma = expf(out.w + a.density_bias);
-            const float alpha = 1.0f - expf(-sigma * a.dt);
-            const float weight = alpha * T;
-            acc.x = acc.x + (1.0f / (1.0f + expf(-out.x))) * weight;
-            acc.y = acc.y + (1.0f / (1.0f + expf(-out.y))) * weight;
-            acc.z = acc.z + (1.0f / (1.0f + expf(-out.z))) * weight;
-            acc.w = acc.w + weight;
-            if (weight > rd.w) {
-                rd.w = weight;
-                depth = dot(cam_fwd, v3(sp.x, sp.y, sp.z) - cam_pos);
+            slots[q] = sm.next(q, cnt, mine);
+            if (mine) ahead[q] = s_out[off + slots[q]];
+        }
+        for (uint32_t j0 = 0; j0 < maxc; j0 += kLead) {
+            if (__ballot(j0 < cnt && !terminated) == 0ull) break;
+#pragma unroll
+            for (uint32_t q = 0; q < kLead; ++q) {
+                const float4 out = ahead[q];
+                const uint32_t slot = slots[q];
+                bool mine;
+                slots[q] = sm.next(j0 + q + kLead, cnt, mine);
+                if (mine && !terminated) ahead[q] = s_out[off + slots[q]];
+                if (j0 + q >= cnt || terminated) continue;
+                // composite_kernel_nerf (testbed_nerf.cu:853-999), render mode Shade
+                const float T = 1.0f - acc.w;
+                const float sigma = expf(out.w + a.density_bias);
+                const float alpha = 1.0f - expf(-sigma * a.dt);
+                const float weight = alpha * T;
+                acc.x = acc.x + (1.0f / (1.0f + expf(-out.x))) * weight;
+                acc.y = acc.y + (1.0f / (1.0f + expf(-out.y))) * weight;
+                acc.z = acc.z + (1.0f / (1.0f + expf(-out.z))) * weight;
+                acc.w = acc.w + weight;
+                if (weight > rd.w) {
+                    rd.w = weight;
+                    heaviest = slot;
+                }
+                ++n;
+                ++used;
+                if (acc.w > 1.0f - a.min_transmittance) {
+                    const float s = acc.w;
+                    acc.x /= s; acc.y /= s; acc.z /= s; acc.w /= s;
+                    terminated = true;
+                }
             }
-            ++n;
-            ++used;
-            if (acc.w > 1.0f - a.min_transmittance) {
-                const float s = acc.w;
-                acc.x /= s; acc.y /= s; acc.z /= s; acc.w /= s;
-                terminated = true;
-            }
+        }
+        if (heaviest != kAllSamples) {
+            const float4 sp = s_pos[off + heaviest];
+            depth = dot(cam_fwd, v3(sp.x, sp.y, sp.z) - cam_pos);
         }
         r_rgba[r] = acc;
         r_d[r] = rd;
         r_depth[r] = depth;
         r_steps[r] = n;
         keep = !terminated && !(r_flags[r] & 2u) && n < a.max_steps;
+        opaque = terminated;
+        clear = keep && acc.w < kClearAlpha;
     }
-    const uint32_t slot = wave_append(&counters[next_slot], keep);
+    const uint32_t slot = block_append<kRayWaves>(&counters[next_slot], keep);
     if (keep) next_alive[slot] = r;
-    // statistics: composited samples this round
+    // statistics: samples composited this round, rays by how it left them
+    __shared__ uint32_t s_stat[3];
+    if (threadIdx.x < 3u) s_stat[threadIdx.x] = 0u;
+    __syncthreads();
     uint32_t total = used;
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) total += __shfl_xor(total, o);
-    if ((threadIdx.x & 63u) == 0 && total) atomicAdd(&counters[kCntComposited], total);
+    const uint32_t n_opaque = (uint32_t)__popcll(__ballot(opaque)), n_clear = (uint32_t)__popcll(__ballot(clear));
+    if ((threadIdx.x & 63u) == 0) {
+        atomicAdd(&s_stat[0], total);
+        atomicAdd(&s_stat[1], n_opaque);
+        atomicAdd(&s_stat[2], n_clear);
+    }
+    __syncthreads();
+    if (threadIdx.x < 3u && s_stat[threadIdx.x])
+        atomicAdd(&counters[threadIdx.x == 0 ? kCntComposited : (threadIdx.x == 1 ? kCntOpaque : kCntClear)],
+                  s_stat[threadIdx.x]);
 }
 
 __global__ void finalize_kernel(uint32_t n, const float4* __restrict__ r_rgba, const float* __restrict__ r_depth,
@@ -329,10 +379,17 @@ __global__ void clear_counters_kernel(uint32_t* counters, uint32_t first, uint32
 }
 
 // Before a round: clear the next live list's count and the round's sample and
-// queue counts; the first round also keeps the initial live count.
-__global__ void round_begin_kernel(uint32_t* counters, uint32_t next_slot, uint32_t first) {
+// queue counts, and set how many samples a ray may emit in it; the first round
+// also keeps the initial live count.  Rounds after the first stay at their
+// window only while at least a quarter of the rays either ended by opacity or
+// have met next to none yet (the surface is still ahead); in a translucent
+// volume, where rays will not end early, one round takes all that is left.
+__global__ void round_begin_kernel(uint32_t* counters, uint32_t next_slot, uint32_t first, uint32_t window) {
     if (threadIdx.x != 0) return;
     if (first) counters[kCntAlive0] = counters[kCntAliveA];
+    const uint32_t seen = counters[kCntOpaque] + counters[kCntClear];
+    counters[kCntLimit] = first || 4u * seen >= counters[kCntAlive0] ? window : 0xffffffffu;
+    counters[kCntClear] = 0;
     counters[next_slot] = 0;
     counters[kCntSamples] = 0;
     counters[kCntQueue] = 0;
@@ -570,12 +627,13 @@ RenderArgs render_args(const insta_ctx* ctx, const insta_camera* cam, uint32_t w
 // live count read on the device.  `max_alive` bounds the live count (it
 // sizes the ray grids).
 insta_status enqueue_round(insta_ctx* ctx, RenderWS& ws, const RenderArgs& a, int32_t frame, uint32_t cur,
-                           bool first, uint32_t max_alive, bool prof, hipStream_t stream) {
+                           bool first, uint32_t window, uint32_t max_alive, bool prof, hipStream_t stream) {
     uint32_t* cnt = ws.d_counters;
     const uint32_t next = 1u - cur;
     const uint32_t cur_slot = cur == 0 ? kCntAliveA : kCntAliveB;
     const uint32_t next_slot = next == 0 ? kCntAliveA : kCntAliveB;
-    hipLaunchKernelGGL(round_begin_kernel, dim3(1), dim3(64), 0, stream, cnt, next_slot, first ? 1u : 0u);
+    hipLaunchKernelGGL(round_begin_kernel, dim3(1), dim3(64), 0, stream, cnt, next_slot, first ? 1u : 0u,
+                       window);
     const dim3 rgrid((max_alive + kRayThreads - 1) / kRayThreads);
     prof_begin(ctx, prof, INSTA_KERNEL_MARCH, stream);
     hipLaunchKernelGGL(march_kernel, rgrid, dim3(kRayThreads), 0, stream, a, ws.alive[cur], cnt + cur_slot,
@@ -583,8 +641,10 @@ insta_status enqueue_round(insta_ctx* ctx, RenderWS& ws, const RenderArgs& a, in
                        reinterpret_cast<float*>(ws.s_hit), ws.s_pos, cnt);
     INSTA_HIP(hipGetLastError());
     prof_end(ctx, prof, INSTA_KERNEL_MARCH, 0, stream);
-    // at most max_alive * K <= sample capacity samples this round
-    const uint32_t n_max = (uint32_t)ws.samples;
+    // at most max_alive * K <= sample capacity samples this round (a later
+    // round's window may have been opened on the device)
+    const uint32_t n_max =
+        (uint32_t)(first ? std::min<uint64_t>(ws.samples, (uint64_t)max_alive * window) : ws.samples);
     prof_begin(ctx, prof, INSTA_KERNEL_DEFORM, stream);
     insta_status st = launch_deform_soa(ctx, ws, frame, cnt + kCntSamples, n_max, cnt + kCntMisses, cnt + kCntQueue, stream);
     if (st != INSTA_OK) return st;
@@ -634,13 +694,13 @@ insta_status enqueue_render(insta_ctx* ctx, RenderWS& ws, const insta_camera* ca
     uint32_t* cnt = ws.d_counters;
     hipLaunchKernelGGL(clear_counters_kernel, dim3(1), dim3(64), 0, stream, cnt, 0u, (uint32_t)kNumCounters);
     prof_begin(ctx, prof, INSTA_KERNEL_INIT, stream);
-    hipLaunchKernelGGL(init_rays_kernel, dim3((tiled_threads(width, height) + kRayThreads - 1) / kRayThreads),
-                       dim3(kRayThreads), 0, stream, a,
+    hipLaunchKernelGGL(init_rays_kernel, dim3((tiled_threads(width, height) + kInitThreads - 1) / kInitThreads),
+                       dim3(kInitThreads), 0, stream, a,
                        ws.r_o, ws.r_d, ws.r_rgba, ws.r_depth, ws.r_steps, ws.alive[0], cnt);
     INSTA_HIP(hipGetLastError());
     prof_end(ctx, prof, INSTA_KERNEL_INIT, n_pix, stream);
     for (uint32_t r = 0; r < rounds; ++r) {
-        st = enqueue_round(ctx, ws, a, frame, r & 1u, r == 0, n_pix, prof, stream);
+        st = enqueue_round(ctx, ws, a, frame, r & 1u, r == 0, round_window(n_pix, prof, r), n_pix, prof, stream);
         if (st != INSTA_OK) return st;
     }
     return enqueue_finalize(ctx, ws, n_pix, rgba, depth, steps, prof, stream);
@@ -661,8 +721,9 @@ insta_status finish_render(insta_ctx* ctx, RenderWS& ws, const insta_camera* cam
     if (n_alive) {
         // rays left after the enqueued rounds: one round per host check
         const RenderArgs a = render_args(ctx, cam, width, height, occupancy, spp);
-        while (n_alive) {
-            insta_status st = enqueue_round(ctx, ws, a, frame, cur, false, n_alive, prof, stream);
+        for (uint32_t r = rounds; n_alive; ++r) {
+            insta_status st =
+                enqueue_round(ctx, ws, a, frame, cur, false, round_window(n_pix, prof, r), n_alive, prof, stream);
             if (st != INSTA_OK) return st;
             INSTA_HIP(hipMemcpyAsync(ws.h_counters, cnt, kNumCounters * sizeof(uint32_t), hipMemcpyDeviceToHost,
                                      stream));
@@ -689,9 +750,12 @@ insta_status finish_render(insta_ctx* ctx, RenderWS& ws, const insta_camera* cam
 insta_status render(insta_ctx* ctx, RenderWS& ws, const insta_camera* cam, uint32_t width, uint32_t height,
                     int32_t frame, int32_t occupancy, uint32_t spp, float* rgba, float* depth, uint32_t* steps,
                     hipStream_t stream) {
-    insta_status st = enqueue_render(ctx, ws, cam, width, height, frame, occupancy, spp, 1, rgba, depth, steps, stream);
+    // profiled renders time one round over all samples per kernel class
+    const uint32_t rounds = width * height < kWindowPixels || (ctx->profiling && &ws == &ctx->ws) ? 1u : 2u;
+    insta_status st =
+        enqueue_render(ctx, ws, cam, width, height, frame, occupancy, spp, rounds, rgba, depth, steps, stream);
     if (st != INSTA_OK) return st;
-    return finish_render(ctx, ws, cam, width, height, frame, occupancy, spp, 1, rgba, depth, steps, stream);
+    return finish_render(ctx, ws, cam, width, height, frame, occupancy, spp, rounds, rgba, depth, steps, stream);
 }
 
 insta_status set_profiling(insta_ctx* ctx, int level) {

@@ -85,6 +85,7 @@ constexpr int kCin = 32;             // density outputs + 16 SH
 constexpr uint32_t kMlpThreads = 256;  // backward: one weight copy in LDS per block
 constexpr uint32_t kChunk = 1024;    // samples per weight-gradient partial
 constexpr uint32_t kRaySeedStride = 8;
+constexpr uint32_t kRayWaves = 4;    // waves per workgroup of the per-ray kernels
 // backward: wave-level run sums on levels where one marching step covers at
 // most this fraction of a cell (runs of about two or more samples per entry)
 constexpr float kRunMaxStepCells = 0.5f;
@@ -246,26 +247,16 @@ __global__ __launch_bounds__(256) void train_rays_kernel(RayArgs a, uint32_t n_r
     RenderArgs ra = a.box;
     if (i < n_rays && train_ray(a, i, n_rays, rays_total, rng, img, pix, o, d, dn, t0, ra)) {
         idir = v3(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
-        // one iteration per sample or empty-voxel skip; sample t values to
-        // step-major scratch (t_buf[j * n_rays + i])
-        float t = t0;
-        while (count < a.box.max_steps) {
-            const V3 pos = o + d * t;
-            if (!box_contains(ra, pos)) break;
-            if (occupied(ra.grid, ra.G, pos)) {
-                t_buf[(size_t)count * n_rays + i] = t;
-                ++count;
-                t += a.box.dt;
-            } else {
-                t = advance_to_next_voxel(t, a.box.dt, pos, d, idir, ra.G);
-            }
-        }
+        // sample t values to step-major scratch (t_buf[j * n_rays + i])
+        bool exited;
+        count = walk_samples(ra, o, d, idir, t0, a.box.max_steps, exited,
+                             [&](uint32_t j, float tj) { t_buf[(size_t)j * n_rays + i] = tj; });
     }
-    const uint32_t base = wave_reserve(&counters[kTSamples], count);
+    const uint32_t base = block_reserve<kRayWaves>(&counters[kTSamples], count);
     const bool fits = base + count <= a.max_samples;
     if (count > 0 && !fits && base < a.max_samples) atomicMin(&counters[kTLimit], base);
     const bool keep = count > 0 && fits;
-    const uint32_t r = wave_append(&counters[kTRays], keep);
+    const uint32_t r = block_append<kRayWaves>(&counters[kTRays], keep);
     if (!keep) return;
     ray_d[r] = make_float4(d.x, d.y, d.z, 0.0f);
     ray_o[r] = make_float4(o.x, o.y, o.z, dn);
@@ -481,7 +472,7 @@ __global__ __launch_bounds__(256) void train_gather_kernel(uint32_t lo, uint32_t
         const uint32_t cnt = ray_cnt[r];
         n = cnt > lo ? min(cnt, hi) - lo : 0u;
     }
-    const uint32_t g = wave_reserve(&counters[round_slot], n);
+    const uint32_t g = block_reserve<kRayWaves>(&counters[round_slot], n);
     if (n == 0) return;
     ray_gbase[r] = g;
     // posed positions from the march's t values (the march's own arithmetic)
@@ -622,7 +613,7 @@ __global__ __launch_bounds__(256) void train_loss_kernel(LossArgs a, Pcg32 rng0,
         ray_loss = ray_loss / 3.0f * a.inv_rays;
     }
     // compaction of the composited samples into the training batch
-    const uint32_t cb = wave_reserve(&counters[kTCompactRes], used);
+    const uint32_t cb = block_reserve<kRayWaves>(&counters[kTCompactRes], used);
     const uint32_t n_c = cb < compact_cap ? min(used, compact_cap - cb) : 0u;
     if (valid) {
         const float ls = a.loss_scale_per_ray;
@@ -653,7 +644,14 @@ __global__ __launch_bounds__(256) void train_loss_kernel(LossArgs a, Pcg32 rng0,
             c_dout[cb + j] = make_float4(drgb[0], drgb[1], drgb[2], ls * (sigma * (a.dt * dsig)));
         }
     }
-    // statistics
+    // statistics, one atomic each per workgroup
+    __shared__ uint32_t s_used;
+    __shared__ float s_loss;
+    if (threadIdx.x == 0) {
+        s_used = 0u;
+        s_loss = 0.0f;
+    }
+    __syncthreads();
     uint32_t u = used;
     float lsum = ray_loss;
 #pragma unroll
@@ -662,8 +660,13 @@ __global__ __launch_bounds__(256) void train_loss_kernel(LossArgs a, Pcg32 rng0,
         lsum += __shfl_xor(lsum, off);
     }
     if ((threadIdx.x & 63u) == 0) {
-        if (u) atomicAdd(&counters[kTUsed], u);
-        if (lsum != 0.0f) atomicAdd(reinterpret_cast<float*>(&counters[kTLoss]), lsum);
+        atomicAdd(&s_used, u);
+        atomicAdd(&s_loss, lsum);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        if (s_used) atomicAdd(&counters[kTUsed], s_used);
+        if (s_loss != 0.0f) atomicAdd(reinterpret_cast<float*>(&counters[kTLoss]), s_loss);
     }
 }
 
