@@ -317,7 +317,8 @@ INSTA_DEV Hit bvh_closest(const MeshView& m, V3 p, uint32_t* stack, uint32_t str
 //          triangle (BVH order); the seed (nearest at the centre) first, the
 //          rest ascending
 //   state  [kClState] occupied cells, entries used, valid (1: lists answer
-//          queries), occupied cells beyond the cap, sub-cells without a list
+//          queries), occupied cells beyond the cap, sub-cells without a list,
+//          (build) cells left by the first and the second pass over the cells
 // ---------------------------------------------------------------------------
 constexpr uint32_t kNoList = 0xffffffffu;
 constexpr uint32_t kClState = 8;
