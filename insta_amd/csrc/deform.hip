@@ -269,6 +269,7 @@ INSTA_DEV int32_t sample_frame(int32_t frame, const int32_t* __restrict__ ray_fr
 // (sample, best triangle so far); its samples' s_hit is kLongHit.
 constexpr int32_t kLongHit = -2;
 constexpr uint32_t kLongBlocks = 256;  // second pass: four waves per CU beside the first pass's samples
+constexpr uint32_t kRecordLongBlocks = 2048;  // the records' second pass runs alone: 408 us with 256 blocks, 170 us with these (2^20 samples)
 
 // kCount: also sum the traversal work into counts[4] (queries, inner nodes,
 // leaves, triangles) -- a separate build for measurement runs
@@ -527,7 +528,7 @@ insta_status launch_deform_records(insta_ctx* ctx, float4* rec, uint32_t n, uint
     const MeshSet ms = mesh_set(ctx, ctx->d_built);
     hipLaunchKernelGGL(deform_records_kernel, dim3((n + kDeformThreads - 1) / kDeformThreads), dim3(kDeformThreads),
                        shmem, stream, ms, rec, n, ctx->d_misses, queue, queue_n);
-    hipLaunchKernelGGL(deform_records_long_kernel, dim3(kLongBlocks), dim3(kDeformThreads), 0, stream, ms, rec,
+    hipLaunchKernelGGL(deform_records_long_kernel, dim3(kRecordLongBlocks), dim3(kDeformThreads), 0, stream, ms, rec,
                        ctx->d_misses, queue, queue_n);
     INSTA_HIP(hipGetLastError());
     return INSTA_OK;

@@ -26,6 +26,7 @@
 // loaded as the first layer's starting accumulator; the per-sample selector
 // (0: ones, 1 + f: frame f) rides in the canonical direction's w.
 #include "context.hpp"
+#include "encoding.hpp"
 
 namespace insta {
 
@@ -211,48 +212,31 @@ INSTA_DEV void sh16_dev(float x, float y, float z, float* o) {
 // same operation order as the scalar encode)
 template <typename TT>
 INSTA_DEV float2 encode_level2(const TT* __restrict__ table, const GridParams& gp, uint32_t l, V3 x) {
-    const float sc = gp.scale[l];
-    const float px = x.x * sc + 0.5f, py = x.y * sc + 0.5f, pz = x.z * sc + 0.5f;
-    const float fx = floorf(px), fy = floorf(py), fz = floorf(pz);
-    const float frac[3] = {px - fx, py - fy, pz - fz};
-    const uint32_t g[3] = {(uint32_t)(int32_t)fx, (uint32_t)(int32_t)fy, (uint32_t)(int32_t)fz};
-    const bool dense = (gp.dense_mask >> l) & 1u;
-    const uint32_t res = gp.res[l], size = gp.size[l];
-    const TT* base = table + (size_t)gp.offset[l] * 2;
-    float a0 = 0.0f, a1 = 0.0f;
+    if constexpr (sizeof(TT) == 4) {
+        float acc[2];
+        encode_level<2>(table, gp, l, x, acc);
+        return make_float2(acc[0], acc[1]);
+    } else {
+        typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+        uint32_t idx[8];
+        float w[8];
+        const Pairs pairs = cell_corners(gp, l, x, idx, w);
+        const char* base = reinterpret_cast<const char*>(table + (size_t)gp.offset[l] * 2);
+        h2 v[8];
+        gather_corners(base, idx, pairs, v);
+        float a0 = 0.0f, a1 = 0.0f;
 #pragma unroll
-    for (uint32_t c = 0; c < 8; ++c) {
-        float w = 1.0f;
-        uint32_t cg[3];
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            const bool up = (c >> d) & 1u;
-            w = w * (up ? frac[d] : 1.0f - frac[d]);
-            cg[d] = g[d] + (up ? 1u : 0u);
+        for (uint32_t c = 0; c < 8; ++c) {
+            a0 = a0 + w[c] * (float)v[c].x;
+            a1 = a1 + w[c] * (float)v[c].y;
         }
-        uint32_t idx;
-        if (dense) {
-            idx = cg[0] + cg[1] * res + cg[2] * (res * res);
-            if (idx >= size) idx %= size;
-        } else {
-            idx = (cg[0] ^ (cg[1] * 2654435761u) ^ (cg[2] * 805459861u)) & (size - 1u);
-        }
-        float v0, v1;
-        if constexpr (sizeof(TT) == 4) {
-            const float2 v = *reinterpret_cast<const float2*>(base + (size_t)idx * 2);
-            v0 = v.x;
-            v1 = v.y;
-        } else {
-            typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-            const h2 v = *reinterpret_cast<const h2*>(base + (size_t)idx * 2);
-            v0 = (float)v.x;
-            v1 = (float)v.y;
-        }
-        a0 = a0 + w * v0;
-        a1 = a1 + w * v1;
+        return make_float2(a0, a1);
     }
-    return make_float2(a0, a1);
 }
+
+// max(x, 0) in one instruction (fmaxf first canonicalises its operands in
+// another; NaN gives 0 either way)
+INSTA_DEV float relu(float x) { return __builtin_amdgcn_fmed3f(x, 0.0f, __builtin_huge_valf()); }
 
 // ---------------------------------------------------------------------------
 // FP32 MFMA kernel
@@ -350,7 +334,7 @@ __global__ __launch_bounds__(256) void network_f32_kernel(const float* __restric
             for (int t = 0; t < 4; ++t)
 #pragma unroll
                 for (int b = 0; b < 4; ++b)
-                    dn = __builtin_amdgcn_mfma_f32_16x16x4f32(W[(t * 4 + b) * 64], fmaxf(h[t][b], 0.0f), dn, 0, 0, 0);
+                    dn = __builtin_amdgcn_mfma_f32_16x16x4f32(W[(t * 4 + b) * 64], relu(h[t][b]), dn, 0, 0, 0);
             W += 16 * 64;
             f4 r[4];
 #pragma unroll
@@ -373,7 +357,7 @@ __global__ __launch_bounds__(256) void network_f32_kernel(const float* __restric
                 for (int s2 = 0; s2 < 4; ++s2)
 #pragma unroll
                     for (int b = 0; b < 4; ++b)
-                        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(W[(t * 16 + s2 * 4 + b) * 64], fmaxf(r[s2][b], 0.0f),
+                        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(W[(t * 16 + s2 * 4 + b) * 64], relu(r[s2][b]),
                                                                    acc, 0, 0, 0);
                 q[t] = acc;
             }
@@ -383,7 +367,7 @@ __global__ __launch_bounds__(256) void network_f32_kernel(const float* __restric
             for (int s2 = 0; s2 < 4; ++s2)
 #pragma unroll
                 for (int b = 0; b < 4; ++b)
-                    o = __builtin_amdgcn_mfma_f32_16x16x4f32(W[(s2 * 4 + b) * 64], fmaxf(q[s2][b], 0.0f), o, 0, 0, 0);
+                    o = __builtin_amdgcn_mfma_f32_16x16x4f32(W[(s2 * 4 + b) * 64], relu(q[s2][b]), o, 0, 0, 0);
             if (g == 0 && i < n) src.out[i] = make_float4(o[0], o[1], o[2], dn[0]);
         }
     }
@@ -412,8 +396,8 @@ INSTA_DEV typename Vec8<T>::type pack_relu(f4 a, f4 b) {
     typename Vec8<T>::type v;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        v[i] = (T)fmaxf(a[i], 0.0f);
-        v[4 + i] = (T)fmaxf(b[i], 0.0f);
+        v[i] = (T)relu(a[i]);
+        v[4 + i] = (T)relu(b[i]);
     }
     return v;
 }

@@ -318,20 +318,30 @@ __global__ __launch_bounds__(256) void train_forward_kernel(const float* __restr
             const uint32_t smp = c_idx[i];
             const float4 p4 = cpos[smp], d4 = cdir[smp];
             const V3 x = v3(p4.x, p4.y, p4.z);
-            float enc[DIN];
+            // two levels' gathers in flight; rolled, so that a level's
+            // corners do not all live at once (one wave per SIMD)
+#pragma unroll 2
+            for (int l = 0; l < L; ++l) {
+                float f[2];
+                encode_level<2>(table, gp, (uint32_t)l, x, f);
 #pragma unroll
-            for (int l = 0; l < L; ++l) encode_level<2>(table, gp, (uint32_t)l, x, enc + 2 * l);
+                for (int k = 0; k < 2; ++k) {
+                    row[2 * l + k] = f[k];
+                    act[(size_t)(A::ENC + 2 * l + k) * ld + i] = f[k];
+                }
+            }
             if constexpr (X > 0) {
                 const uint32_t sel = __float_as_uint(d4.w);
                 const float* fx = x_extra ? x_extra + (size_t)smp * X
                                           : (sel != kExtraOnes && sel <= n_frames ? frame_extra + (size_t)(sel - 1u) * X
                                                                                   : nullptr);
 #pragma unroll
-                for (int e = 0; e < X; ++e) enc[E + e] = fx ? fx[e] : 1.0f;
+                for (int e = 0; e < X; ++e) {
+                    const float v = fx ? fx[e] : 1.0f;
+                    row[E + e] = v;
+                    act[(size_t)(A::ENC + E + e) * ld + i] = v;
+                }
             }
-#pragma unroll
-            for (int k = 0; k < DIN; ++k) row[k] = enc[k];
-            store_rows<DIN, DIN>(act, ld, A::ENC, i, enc);
             float sh[16];
             sh16(d4.x * 2.0f - 1.0f, d4.y * 2.0f - 1.0f, d4.z * 2.0f - 1.0f, sh);
             store_rows<16, 16>(act, ld, A::SH, i, sh);
@@ -752,9 +762,7 @@ __global__ __launch_bounds__(kScatterThreads) void scatter_lds64_kernel(GridPara
     const uint32_t chunk = (n + gridDim.x - 1) / gridDim.x;
     // an empty chunk still stores its (zero) partial
     const uint32_t s0 = min(n, blockIdx.x * chunk), s1 = min(n, s0 + chunk);
-    const uint32_t size = gp.size[l], res = gp.res[l];
-    const bool dense_l = (gp.dense_mask >> l) & 1u;
-    const float sc = gp.scale[l];
+    const uint32_t size = gp.size[l];
     for (uint32_t j = threadIdx.x; j < size; j += kScatterThreads) tab[j] = 0.0;
     __syncthreads();
     const float* __restrict__ de = denc_g + (size_t)(2u * l + f) * ld;
@@ -767,33 +775,20 @@ __global__ __launch_bounds__(kScatterThreads) void scatter_lds64_kernel(GridPara
         en = de[i];
     }
     while (i < s1) {
-        const float xs[3] = {pn.x, pn.y, pn.z};
+        const V3 x = xyz(pn);
         const float e = en;
         i += kScatterThreads;
         if (i < s1) {
             pn = cpos[c_idx[i]];
             en = de[i];
         }
-        float frac[3];
-        uint32_t g[3];
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            const float pp = xs[d] * sc + 0.5f;
-            const float fl = floorf(pp);
-            frac[d] = pp - fl;
-            g[d] = (uint32_t)(int32_t)fl;
-        }
+        uint32_t corner[8];
+        float weight[8];
+        cell_corners(gp, l, x, corner, weight);
 #pragma unroll
         for (uint32_t c = 0; c < 8; ++c) {
-            float w = 1.0f;
-            uint32_t cg[3];
-#pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                const bool up = (c >> k) & 1u;
-                w = w * (up ? frac[k] : 1.0f - frac[k]);
-                cg[k] = g[k] + (up ? 1u : 0u);
-            }
-            unsafeAtomicAdd(&tab[grid_index(cg, dense_l, res, size)], (double)(w * e));
+            const float w = weight[c];
+            unsafeAtomicAdd(&tab[corner[c]], (double)(w * e));
         }
     }
     __syncthreads();
@@ -813,9 +808,7 @@ __global__ __launch_bounds__(kScatterThreads) void scatter_lds_kernel(GridParams
     const uint32_t chunk = (n + gridDim.x - 1) / gridDim.x;
     // an empty chunk still stores its (zero) partial
     const uint32_t s0 = min(n, blockIdx.x * chunk), s1 = min(n, s0 + chunk);
-    const uint32_t size = gp.size[l], off = gp.offset[l], res = gp.res[l];
-    const bool dense_l = (gp.dense_mask >> l) & 1u;
-    const float sc = gp.scale[l];
+    const uint32_t size = gp.size[l], off = gp.offset[l];
     for (uint32_t j = threadIdx.x; j < size; j += kScatterThreads) tab[j] = __floats2half2_rn(0.0f, 0.0f);
     __syncthreads();
     const bool runs = (run_mask >> l) & 1u;
@@ -838,29 +831,16 @@ __global__ __launch_bounds__(kScatterThreads) void scatter_lds_kernel(GridParams
     if (rounds) load(0, pn, en0, en1);
     for (uint32_t q = 0; q < rounds; ++q) {
         const bool valid = s0 + q * kScatterThreads + threadIdx.x < s1;
-        const float xs[3] = {pn.x, pn.y, pn.z};
+        const V3 x = xyz(pn);
         const float e0 = en0, e1 = en1;
         if (q + 1 < rounds) load(q + 1, pn, en0, en1);
-        float frac[3];
-        uint32_t g[3];
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            const float pp = xs[d] * sc + 0.5f;
-            const float fl = floorf(pp);
-            frac[d] = pp - fl;
-            g[d] = (uint32_t)(int32_t)fl;
-        }
+        uint32_t corner[8];
+        float weight[8];
+        cell_corners(gp, l, x, corner, weight);
 #pragma unroll
         for (uint32_t c = 0; c < 8; ++c) {
-            float w = 1.0f;
-            uint32_t cg[3];
-#pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                const bool up = (c >> k) & 1u;
-                w = w * (up ? frac[k] : 1.0f - frac[k]);
-                cg[k] = g[k] + (up ? 1u : 0u);
-            }
-            const uint32_t idx = grid_index(cg, dense_l, res, size);
+            const float w = weight[c];
+            const uint32_t idx = corner[c];
             float2 v = make_float2(w * e0, w * e1);
             bool lead = valid;
             if (runs) {
@@ -932,35 +912,21 @@ __global__ __launch_bounds__(kLevelThreads) void scatter_levels_kernel(GridParam
     uint32_t rest = level_mask;
     for (uint32_t j = 0; j < li; ++j) rest &= rest - 1u;  // drop the li lowest levels of the list
     const uint32_t l = (uint32_t)__builtin_ctz(rest);
-    const uint32_t size = gp.size[l], res = gp.res[l], off = gp.offset[l];
-    const bool dense_l = (gp.dense_mask >> l) & 1u, runs = (run_mask >> l) & 1u;
-    const float sc = gp.scale[l];
+    const uint32_t off = gp.offset[l];
+    const bool runs = (run_mask >> l) & 1u;
     const bool valid = s0 + threadIdx.x < n, odd = threadIdx.x & 1u;
     const uint32_t i = valid ? s0 + threadIdx.x : n - 1u;  // tail lanes repeat the last sample and add nothing
     const float4 p4 = cpos[c_idx[i]];
     const float e0 = valid ? denc_g[(size_t)(2u * l) * ld + i] : 0.0f;
     const float e1 = valid ? denc_g[(size_t)(2u * l + 1u) * ld + i] : 0.0f;
-    const float xs[3] = {p4.x, p4.y, p4.z};
-    float frac[3];
-    uint32_t g[3];
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        const float pp = xs[d] * sc + 0.5f;
-        const float fl = floorf(pp);
-        frac[d] = pp - fl;
-        g[d] = (uint32_t)(int32_t)fl;
-    }
+    const V3 x = xyz(p4);
+    uint32_t corner[8];
+    float weight[8];
+    cell_corners(gp, l, x, corner, weight);
 #pragma unroll
     for (uint32_t c = 0; c < 8; ++c) {
-        float w = 1.0f;
-        uint32_t cg[3];
-#pragma unroll
-        for (int q = 0; q < 3; ++q) {
-            const bool up = (c >> q) & 1u;
-            w = w * (up ? frac[q] : 1.0f - frac[q]);
-            cg[q] = g[q] + (up ? 1u : 0u);
-        }
-        uint32_t idx = off + grid_index(cg, dense_l, res, size);
+        const float w = weight[c];
+        uint32_t idx = off + corner[c];
         float2 v = make_float2(w * e0, w * e1);
         bool lead = valid;
         if (runs) {
@@ -1037,38 +1003,23 @@ __global__ __launch_bounds__(Part<H16>::kChunkSamples) void partition_kernel(
     const uint32_t n = *n_dev, s0 = pass0 + blockIdx.x * P::kChunkSamples;
     if (s0 >= n) return;
     const uint32_t l = first_level + blockIdx.y, t = threadIdx.x;
-    const uint32_t size = gp.size[l], res = gp.res[l], shift = slice_shift(size);
-    const bool dense_l = (gp.dense_mask >> l) & 1u;
-    const float sc = gp.scale[l];
+    const uint32_t shift = slice_shift(gp.size[l]);
     for (uint32_t j = t; j < kPartSlices; j += P::kChunkSamples) s_cnt[j] = 0u;
     __syncthreads();
     const bool valid = s0 + t < n;
     const uint32_t i = valid ? s0 + t : n - 1u;  // tail lanes repeat the last sample and emit nothing
     const float4 p4 = cpos[c_idx[i]];
     const float e0 = denc_g[(size_t)(2u * l) * ld + i], e1 = denc_g[(size_t)(2u * l + 1u) * ld + i];
-    const float xs[3] = {p4.x, p4.y, p4.z};
-    float frac[3];
-    uint32_t g[3];
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        const float pp = xs[d] * sc + 0.5f;
-        const float fl = floorf(pp);
-        frac[d] = pp - fl;
-        g[d] = (uint32_t)(int32_t)fl;
-    }
+    const V3 x = xyz(p4);
+    uint32_t corner[8];
+    float weight[8];
+    cell_corners(gp, l, x, corner, weight);
     uint32_t idx[8], rank[8];
     float2 v[8];
 #pragma unroll
     for (uint32_t c = 0; c < 8; ++c) {
-        float w = 1.0f;
-        uint32_t cg[3];
-#pragma unroll
-        for (int q = 0; q < 3; ++q) {
-            const bool up = (c >> q) & 1u;
-            w = w * (up ? frac[q] : 1.0f - frac[q]);
-            cg[q] = g[q] + (up ? 1u : 0u);
-        }
-        idx[c] = grid_index(cg, dense_l, res, size);
+        const float w = weight[c];
+        idx[c] = corner[c];
         v[c] = make_float2(w * e0, w * e1);
         bool lead = valid;
         if constexpr (H16) {
@@ -1800,27 +1751,22 @@ __global__ __launch_bounds__(128) void net_input_grad_kernel(const float* __rest
     for (int l = 0; l < L; ++l) {
         const float sc = gp.scale[l];
         float frac[3];
-        uint32_t g0[3];
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
             const float pp = xs[d] * sc + 0.5f;
-            const float fl = floorf(pp);
-            frac[d] = pp - fl;
-            g0[d] = (uint32_t)(int32_t)fl;
+            frac[d] = pp - floorf(pp);
         }
-        const bool dense_l = (gp.dense_mask >> l) & 1u;
+        uint32_t corner[8];
+        float weight[8];
+        const Pairs pairs = cell_corners(gp, (uint32_t)l, xyz(p4), corner, weight);
+        float2 v[8];
+        gather_corners(reinterpret_cast<const char*>(table + 2 * (size_t)gp.offset[l]), corner, pairs, v);
 #pragma unroll
         for (uint32_t c = 0; c < 8; ++c) {
-            uint32_t cg[3];
             float wk[3];
 #pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                const bool up = (c >> k) & 1u;
-                wk[k] = up ? frac[k] : 1.0f - frac[k];
-                cg[k] = g0[k] + (up ? 1u : 0u);
-            }
-            const uint32_t idx = gp.offset[l] + grid_index(cg, dense_l, gp.res[l], gp.size[l]);
-            const float s = denc[2 * l] * table[2 * (size_t)idx] + denc[2 * l + 1] * table[2 * (size_t)idx + 1];
+            for (int k = 0; k < 3; ++k) wk[k] = ((c >> k) & 1u) ? frac[k] : 1.0f - frac[k];
+            const float s = denc[2 * l] * v[c].x + denc[2 * l + 1] * v[c].y;
             gx[0] += s * (((c & 1u) ? sc : -sc) * wk[1] * wk[2]);
             gx[1] += s * (((c & 2u) ? sc : -sc) * wk[0] * wk[2]);
             gx[2] += s * (((c & 4u) ? sc : -sc) * wk[0] * wk[1]);
