@@ -25,23 +25,13 @@ INSTA_DEV uint32_t grid_index(const uint32_t cg[3], bool dense, uint32_t res, ui
     return (cg[0] ^ (cg[1] * 2654435761u) ^ (cg[2] * 805459861u)) & (size - 1u);
 }
 
-// The eight corners of position x's cell on level l: table entries (as
-// grid_index) and trilinear weights, corner c's bit d the upper one on axis d.
-// All indices come before any use, with one test of the whole cell for the
-// wrap of a dense level (which only positions outside [0, 1]^3 need): tested
-// corner by corner, every corner's load sat behind a branch of its own and
-// the eight loads went out one after another (FP32 render of the 16-level head
-// at 512 x 512: 1,355 us, with this 1,294 us; training forward 284 / 233 us).
-// Returns how the corners of an
-// x pair (2j, 2j + 1) lie: neighbours (dense), in one aligned pair of entries
-// (hashed, even x: the two hashes differ in bit 0 only) or apart.
-enum Pairs { kNeighbours, kAlignedPair, kApart };
-INSTA_DEV Pairs cell_corners(const GridParams& gp, uint32_t l, V3 x, uint32_t idx[8], float w[8]) {
-    const float sc = gp.scale[l];
+// Position x's cell on level l: its lower corner g, the offset in it and the
+// trilinear weights, corner c's bit d the upper one on axis d.
+INSTA_DEV void cell_weights(float sc, V3 x, uint32_t g[3], float frac[3], float w[8]) {
     const float px = x.x * sc + 0.5f, py = x.y * sc + 0.5f, pz = x.z * sc + 0.5f;
     const float fx = floorf(px), fy = floorf(py), fz = floorf(pz);
-    const float frac[3] = {px - fx, py - fy, pz - fz};
-    const uint32_t g[3] = {(uint32_t)(int32_t)fx, (uint32_t)(int32_t)fy, (uint32_t)(int32_t)fz};
+    frac[0] = px - fx, frac[1] = py - fy, frac[2] = pz - fz;
+    g[0] = (uint32_t)(int32_t)fx, g[1] = (uint32_t)(int32_t)fy, g[2] = (uint32_t)(int32_t)fz;
     const float u0 = 1.0f - frac[0], u1 = 1.0f - frac[1], u2 = 1.0f - frac[2];
     const float xy[4] = {u0 * u1, frac[0] * u1, u0 * frac[1], frac[0] * frac[1]};
 #pragma unroll
@@ -49,6 +39,29 @@ INSTA_DEV Pairs cell_corners(const GridParams& gp, uint32_t l, V3 x, uint32_t id
         w[c] = xy[c] * u2;
         w[c + 4] = xy[c] * frac[2];
     }
+}
+
+// Entries of a cell's corners on a dense level, wrapped as grid_index: only
+// positions outside [0, 1]^3 need it, so the callers test the whole cell once
+// (tested corner by corner, every corner's load sat behind a branch of its own
+// and the eight loads went out one after another).
+INSTA_DEV void dense_corners(const uint32_t g[3], uint32_t res, uint32_t size, uint32_t idx[8]) {
+    const uint32_t res2 = res * res, first = g[0] + g[1] * res + g[2] * res2;
+#pragma unroll
+    for (uint32_t c = 0; c < 8; ++c) {
+        idx[c] = first + (c & 1u) + ((c & 2u) ? res : 0u) + ((c & 4u) ? res2 : 0u);
+        if (idx[c] >= size) idx[c] %= size;
+    }
+}
+
+constexpr uint32_t kPrimeY = 2654435761u, kPrimeZ = 805459861u;
+
+// The eight corners of position x's cell on level l: table entries (as
+// grid_index) and weights, for the gradient scatters.
+INSTA_DEV void cell_corners(const GridParams& gp, uint32_t l, V3 x, uint32_t idx[8], float w[8]) {
+    uint32_t g[3];
+    float frac[3];
+    cell_weights(gp.scale[l], x, g, frac, w);
     const uint32_t res = gp.res[l], size = gp.size[l];
     if ((gp.dense_mask >> l) & 1u) {
         const uint32_t res2 = res * res;
@@ -57,85 +70,105 @@ INSTA_DEV Pairs cell_corners(const GridParams& gp, uint32_t l, V3 x, uint32_t id
         for (uint32_t c = 0; c < 8; ++c)
             idx[c] = first + (c & 1u) + ((c & 2u) ? res : 0u) + ((c & 4u) ? res2 : 0u);
         // inside the grid the last corner's entry is the largest
-        if (!(g[0] < res && g[1] < res && g[2] < res && idx[7] < size)) {
-#pragma unroll
-            for (uint32_t c = 0; c < 8; ++c)
-                if (idx[c] >= size) idx[c] %= size;
-            return kApart;
-        }
-        return kNeighbours;
+        if (!(g[0] < res && g[1] < res && g[2] < res && idx[7] < size)) dense_corners(g, res, size, idx);
     } else {
-        const uint32_t hy = g[1] * 2654435761u, hz = g[2] * 805459861u;
-        const uint32_t yz[4] = {hy ^ hz, (hy + 2654435761u) ^ hz, hy ^ (hz + 805459861u),
-                                (hy + 2654435761u) ^ (hz + 805459861u)};
+        const uint32_t hy = g[1] * kPrimeY, hz = g[2] * kPrimeZ;
+        const uint32_t yz[4] = {hy ^ hz, (hy + kPrimeY) ^ hz, hy ^ (hz + kPrimeZ), (hy + kPrimeY) ^ (hz + kPrimeZ)};
 #pragma unroll
         for (uint32_t c = 0; c < 8; ++c) idx[c] = ((g[0] + (c & 1u)) ^ yz[c >> 1]) & (size - 1u);
-        return (g[0] & 1u) == 0u ? kAlignedPair : kApart;
     }
 }
 
-// Entries of the eight corners (E: an entry of two features).  A gather costs
-// a cache lookup per lane and instruction, not bytes: neighbours and aligned
-// pairs come with one load of two entries, half the lookups on dense levels,
-// a quarter fewer on hashed ones (half of the cells have an even x).  On the
-// 16-level head, 8 loads / pairs on dense levels only / pairs on all:
-// 1,048,576 BF16 positions 412 / 383 / 359 us, FP32 render at 512 x 512
-// (two rounds) 1,294 / 1,610 / 1,262 us, training forward of 100,000
-// positions 156 / 166 / 145 us (a branch between the two kinds of level
-// costs more than the hashed pairs' unused halves).
+// Values of the corners' entries (E: an entry of two features, base: the
+// level's table), the offsets in the cell and the weights.  Coherent positions
+// (renders) are bound by the instructions of this function, scattered ones by
+// cache lookups, one per lane and load.  So the corners of an x pair come with
+// one load: neighbours on dense levels; on hashed ones the two hashes of an
+// even x differ in bit 0 only, and lanes with an odd x load the upper corner
+// by itself.  Offsets are computed in bytes (the hash's factors times the
+// entry's size), dense rows lie at four scalar bases, and which half of its
+// aligned pair a corner is follows from the cell's parity, the factors being
+// odd.
+// On the 16-level head, 8 loads one after another / 8 together / pairs: FP32
+// render at 512 x 512 (two rounds) 1,355 / 1,294 / 1,255 us; 1,048,576 BF16
+// positions 433 / 412 / 362 us; training forward of 100,000 positions 284 (of
+// the render's samples) / 156 / 144 us.
 template <class E>
-INSTA_DEV void gather_corners(const char* __restrict__ base, const uint32_t idx[8], Pairs pairs, E v[8]) {
+INSTA_DEV void cell_fetch(const GridParams& gp, uint32_t l, V3 x, const char* __restrict__ base, E v[8], float frac[3],
+                          float w[8]) {
     struct Two {  // aligned as one entry: half of the pairs start at an odd one
         E a, b;
     };
-    if (pairs == kNeighbours) {
+    constexpr uint32_t S = sizeof(E);
+    uint32_t g[3];
+    cell_weights(gp.scale[l], x, g, frac, w);
+    const uint32_t size = gp.size[l];
+    if ((gp.dense_mask >> l) & 1u) {
+        // a dense level has at most 2^26 entries, so a slab of it less than
+        // 2^18: the byte strides fit the 24-bit multiplier
+        const uint32_t res = gp.res[l], row = res * S, slab = res * res * S;
+        const uint32_t at = g[0] * S + __umul24(g[1], row) + __umul24(g[2], slab);
+        // inside the grid the last corner's entry is the largest
+        if (__builtin_expect(g[0] < res && g[1] < res && g[2] < res && at + row + slab + S < size * S, 1)) {
+            const char* rows[4] = {base, base + row, base + slab, base + slab + row};
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const Two t = *reinterpret_cast<const Two*>(rows[j] + at);
+                v[2 * j] = t.a;
+                v[2 * j + 1] = t.b;
+            }
+        } else {
+            uint32_t idx[8];
+            dense_corners(g, res, size, idx);
+#pragma unroll
+            for (int c = 0; c < 8; ++c) v[c] = *reinterpret_cast<const E*>(base + idx[c] * S);
+        }
+    } else {
+        const uint32_t mask = (size - 1u) * S;
+        const uint32_t hy = g[1] * (kPrimeY * S), hz = g[2] * (kPrimeZ * S);
+        const uint32_t hy1 = hy + kPrimeY * S, hz1 = hz + kPrimeZ * S;
+        const uint32_t yz[4] = {hy ^ hz, hy1 ^ hz, hy ^ hz1, hy1 ^ hz1};
+        const uint32_t x0 = g[0] * S, x1 = x0 + S;
+        Two t[4];  // level tables hold an even number of entries
+#pragma unroll
+        for (int j = 0; j < 4; ++j) t[j] = *reinterpret_cast<const Two*>(base + ((x0 ^ yz[j]) & (mask & ~S)));
+        const bool apart = g[0] & 1u;
+        E up[4];
+        if (apart) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) up[j] = *reinterpret_cast<const E*>(base + ((x1 ^ yz[j]) & mask));
+        }
+        const bool upper = (g[0] ^ g[1] ^ g[2]) & 1u;  // rows 0 and 3; rows 1 and 2 the other half
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            const Two t = *reinterpret_cast<const Two*>(base + idx[2 * j] * (uint32_t)sizeof(E));
-            v[2 * j] = t.a;
-            v[2 * j + 1] = t.b;
+            const bool odd = (j == 0 || j == 3) ? upper : !upper;
+            v[2 * j] = odd ? t[j].b : t[j].a;
+            const E other = odd ? t[j].a : t[j].b;
+            v[2 * j + 1] = apart ? up[j] : other;
         }
-        return;
-    }
-    // the aligned pair around the lower corner (level tables hold an even
-    // number of entries); the upper one's own entry where it lies apart
-    E lo[4], hi[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const Two t = *reinterpret_cast<const Two*>(base + (idx[2 * j] & ~1u) * (uint32_t)sizeof(E));
-        lo[j] = t.a;
-        hi[j] = t.b;
-    }
-    E up[4];
-    if (pairs == kApart) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) up[j] = *reinterpret_cast<const E*>(base + idx[2 * j + 1] * (uint32_t)sizeof(E));
-    }
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const bool odd = idx[2 * j] & 1u;
-        v[2 * j] = odd ? hi[j] : lo[j];
-        v[2 * j + 1] = pairs == kApart ? up[j] : (odd ? lo[j] : hi[j]);
     }
 }
 
 template <int F>
 INSTA_DEV void encode_level(const float* __restrict__ table, const GridParams& gp, uint32_t l, V3 x, float acc[F]) {
-    uint32_t idx[8];
     float w[8];
-    const Pairs pairs = cell_corners(gp, l, x, idx, w);
     const char* base = reinterpret_cast<const char*>(table + (size_t)gp.offset[l] * F);
 #pragma unroll
     for (int f = 0; f < F; ++f) acc[f] = 0.0f;
     if constexpr (F == 2) {
         float2 v[8];
-        gather_corners(base, idx, pairs, v);
+        float frac[3];
+        cell_fetch(gp, l, x, base, v, frac, w);
 #pragma unroll
         for (uint32_t c = 0; c < 8; ++c) {
             acc[0] = acc[0] + w[c] * v[c].x;
             acc[1] = acc[1] + w[c] * v[c].y;
         }
-    } else if constexpr (F == 4) {
+        return;
+    }
+    uint32_t idx[8];
+    cell_corners(gp, l, x, idx, w);
+    if constexpr (F == 4) {
 #pragma unroll
         for (uint32_t c = 0; c < 8; ++c) {
             const float4 v = *reinterpret_cast<const float4*>(base + (size_t)idx[c] * 16u);
@@ -144,7 +177,7 @@ INSTA_DEV void encode_level(const float* __restrict__ table, const GridParams& g
             acc[2] = acc[2] + w[c] * v.z;
             acc[3] = acc[3] + w[c] * v.w;
         }
-    } else {
+    } else if constexpr (F != 2) {
 #pragma unroll
         for (uint32_t c = 0; c < 8; ++c) {
             const float* e = reinterpret_cast<const float*>(base + (size_t)idx[c] * (4u * F));

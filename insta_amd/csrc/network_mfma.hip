@@ -218,17 +218,17 @@ INSTA_DEV float2 encode_level2(const TT* __restrict__ table, const GridParams& g
         return make_float2(acc[0], acc[1]);
     } else {
         typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-        uint32_t idx[8];
-        float w[8];
-        const Pairs pairs = cell_corners(gp, l, x, idx, w);
-        const char* base = reinterpret_cast<const char*>(table + (size_t)gp.offset[l] * 2);
+        float w[8], frac[3];
         h2 v[8];
-        gather_corners(base, idx, pairs, v);
-        float a0 = 0.0f, a1 = 0.0f;
+        cell_fetch(gp, l, x, reinterpret_cast<const char*>(table + (size_t)gp.offset[l] * 2), v, frac, w);
+        // fma(w, v, 0) rounds as w * v and takes the FP16 value as it is (one
+        // v_fma_mix_f32 for a conversion and a product)
+        float a0 = __builtin_fmaf(w[0], (float)v[0].x, 0.0f);
+        float a1 = __builtin_fmaf(w[0], (float)v[0].y, 0.0f);
 #pragma unroll
-        for (uint32_t c = 0; c < 8; ++c) {
-            a0 = a0 + w[c] * (float)v[c].x;
-            a1 = a1 + w[c] * (float)v[c].y;
+        for (uint32_t c = 1; c < 8; ++c) {
+            a0 = a0 + __builtin_fmaf(w[c], (float)v[c].x, 0.0f);
+            a1 = a1 + __builtin_fmaf(w[c], (float)v[c].y, 0.0f);
         }
         return make_float2(a0, a1);
     }
@@ -250,8 +250,8 @@ constexpr int kF32Stride = 33;  // floats per sample in LDS: 32 features + 1 pad
 // of all of it.  Grids that are not a multiple of 8 blocks stride plainly.
 struct XcdTiles {
     uint32_t tile, end, step;
-    INSTA_DEV explicit XcdTiles(uint32_t n) {
-        const uint32_t tiles = (n + kTile - 1) / kTile;
+    INSTA_DEV XcdTiles(uint32_t n, uint32_t tile_samples) {
+        const uint32_t tiles = (n + tile_samples - 1) / tile_samples;
         if (gridDim.x % 8u == 0) {
             const uint32_t xcd = blockIdx.x % 8u, chunk = (tiles + 7u) / 8u;
             tile = xcd * chunk + blockIdx.x / 8u;
@@ -265,35 +265,46 @@ struct XcdTiles {
     }
 };
 
-template <int L, int X, class Src>
-__global__ __launch_bounds__(256) void network_f32_kernel(const float* __restrict__ table, GridParams gp,
-                                                          const float* __restrict__ frag,
-                                                          const float* __restrict__ xbias, uint32_t xrows,
-                                                          Src src) {
+// Samples a workgroup takes at once: kTile, a sample a lane in the encode and
+// four column blocks of 16 a wave; or a quarter, a quarter of the levels and
+// one column block a wave, which brings a quarter of the latency where the
+// samples fill few CUs.
+// The line is 131,072 samples: network rounds of a training step of 8,192 rays
+// 204 us with whole tiles, 175 us; above it the whole tiles win (BF16
+// inference of 1,048,576 positions 362 us, with quarter tiles 435 us; FP32
+// render at 512 x 512 1,262 / 1,316 us).
+constexpr uint32_t kSmallTileMax = 256u * 512u;
+
+template <int L, int X, int NB, class Src>
+INSTA_DEV void f32_tiles(float* s_x, const float* __restrict__ table, const GridParams& gp,
+                         const float* __restrict__ frag, const float* __restrict__ xbias, uint32_t xrows, uint32_t n,
+                         const Src& src) {
     constexpr int DIN = L * 2;
     static_assert(DIN < kF32Stride, "LDS row holds the features and the extra-dims selector");
     constexpr int KB0 = DIN / 4;
-    __shared__ float s_x[kTile * kF32Stride];
+    constexpr uint32_t kSamples = 64 * NB;
+    constexpr int kSplit = 4 / NB;  // waves that share a sample's levels
+    static_assert(L % kSplit == 0, "whole levels a wave");
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-    const uint32_t n = src.count();
     const uint32_t g = lane >> 4, col = lane & 15u;
-    for (XcdTiles it(n); it.tile < it.end; it.tile += it.step) {
-        const uint32_t base = it.tile * kTile;
+    for (XcdTiles it(n, kSamples); it.tile < it.end; it.tile += it.step) {
+        const uint32_t base = it.tile * kSamples;
         __syncthreads();
         {
-            const uint32_t i = base + tid;
-            float* row = s_x + tid * kF32Stride;
+            const uint32_t i = base + tid % kSamples;
+            const int l0 = __builtin_amdgcn_readfirstlane((int)(tid / kSamples)) * (L / kSplit);
+            float* row = s_x + tid % kSamples * kF32Stride;
             if (i < n) {
                 V3 p, d;
                 src.load(i, p, d);
 #pragma unroll 2
-                for (int l = 0; l < L; ++l) {
+                for (int l = l0; l < l0 + L / kSplit; ++l) {
                     const float2 e = encode_level2<float>(table, gp, (uint32_t)l, p);
                     row[2 * l] = e.x;
                     row[2 * l + 1] = e.y;
                 }
             } else {
-                for (int k = 0; k < DIN; ++k) row[k] = 0.0f;
+                for (int k = 2 * l0; k < 2 * (l0 + L / kSplit); ++k) row[k] = 0.0f;
             }
             if constexpr (X > 0) {
                 const uint32_t sel = i < n ? src.sel(i) : 0u;
@@ -301,8 +312,8 @@ __global__ __launch_bounds__(256) void network_f32_kernel(const float* __restric
             }
         }
         __syncthreads();
-        for (uint32_t nb = 0; nb < 4; ++nb) {
-            const uint32_t s = wave * 64 + nb * 16 + col;  // sample (column) of this lane
+        for (uint32_t nb = 0; nb < NB; ++nb) {
+            const uint32_t s = (wave * NB + nb) * 16 + col;  // sample (column) of this lane
             const uint32_t i = base + s;
             const float* xr = s_x + s * kF32Stride;
             // SH of this column's direction; lane group g feeds rows 4g..4g+3
@@ -373,6 +384,17 @@ __global__ __launch_bounds__(256) void network_f32_kernel(const float* __restric
     }
 }
 
+template <int L, int X, class Src>
+__global__ __launch_bounds__(256) void network_f32_kernel(const float* __restrict__ table, GridParams gp,
+                                                          const float* __restrict__ frag,
+                                                          const float* __restrict__ xbias, uint32_t xrows,
+                                                          Src src) {
+    __shared__ float s_x[kTile * kF32Stride];
+    const uint32_t n = src.count();
+    if (n <= kSmallTileMax) f32_tiles<L, X, 1>(s_x, table, gp, frag, xbias, xrows, n, src);
+    else f32_tiles<L, X, 4>(s_x, table, gp, frag, xbias, xrows, n, src);
+}
+
 // ---------------------------------------------------------------------------
 // FP16 / BF16 MFMA kernel (16x16x32), FP16 hash tables
 // ---------------------------------------------------------------------------
@@ -402,43 +424,52 @@ INSTA_DEV typename Vec8<T>::type pack_relu(f4 a, f4 b) {
     return v;
 }
 
-template <int L, int X, typename T, class Src>
-__global__ __launch_bounds__(256, 4) void network_x32_kernel(const _Float16* __restrict__ table, GridParams gp,
-                                                          const T* __restrict__ frag, const float* __restrict__ xbias,
-                                                          uint32_t xrows, Src src) {
+template <int L, int X, int NB, typename T, class Src>
+INSTA_DEV void x32_tiles(T* s_x, const typename Vec8<T>::type* A, const _Float16* __restrict__ table,
+                         const GridParams& gp, const float* __restrict__ xbias, uint32_t xrows, uint32_t n,
+                         const Src& src) {
     typedef typename Vec8<T>::type V8;
     constexpr int DIN = L * 2;
     static_assert(DIN <= 32, "one K block for the first layer");
-    __shared__ __attribute__((aligned(16))) T s_x[kTile * kX32Stride];
+    constexpr uint32_t kSamples = 64 * NB;
+    constexpr int kSplit = 4 / NB;  // waves that share a sample's levels
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
     const uint32_t g = lane >> 4, col = lane & 15u;
-    // weight fragments into registers (kFragX32 x 8 values per lane)
-    V8 A[kFragX32];
-#pragma unroll
-    for (uint32_t f = 0; f < kFragX32; ++f) A[f] = *reinterpret_cast<const V8*>(frag + ((size_t)f * 64 + lane) * 8);
-    const uint32_t n = src.count();
-    for (XcdTiles it(n); it.tile < it.end; it.tile += it.step) {
-        const uint32_t base = it.tile * kTile;
+    for (XcdTiles it(n, kSamples); it.tile < it.end; it.tile += it.step) {
+        const uint32_t base = it.tile * kSamples;
         __syncthreads();
         {
-            const uint32_t i = base + tid;
-            T* row = s_x + tid * kX32Stride;
+            const uint32_t i = base + tid % kSamples;
+            const int part = __builtin_amdgcn_readfirstlane((int)(tid / kSamples)), l0 = part * (L / kSplit);
+            T* row = s_x + tid % kSamples * kX32Stride;
             if (i < n) {
                 V3 p, d;
                 src.load(i, p, d);
-#pragma unroll 2
-                for (int l = 0; l < L; ++l) {
+// one level at a time: two spill, and four waves a SIMD cover the latency
+#pragma unroll 1
+                for (int l = l0; l < l0 + L / kSplit; ++l) {
                     const float2 e = encode_level2<_Float16>(table, gp, (uint32_t)l, p);
                     row[2 * l] = (T)e.x;
                     row[2 * l + 1] = (T)e.y;
                 }
+                if (part == 0) {
 #pragma unroll
-                for (int k = DIN; k < 32; ++k) row[k] = (T)0.0f;
-                float sh[16];
-                sh16_dev(d.x * 2.0f - 1.0f, d.y * 2.0f - 1.0f, d.z * 2.0f - 1.0f, sh);
+                    for (int k = DIN; k < 32; ++k) row[k] = (T)0.0f;
+                    float sh[16];
+                    sh16_dev(d.x * 2.0f - 1.0f, d.y * 2.0f - 1.0f, d.z * 2.0f - 1.0f, sh);
+                    // values round to FP32, then to T: left to itself the
+                    // compiler fuses some of the last products with the
+                    // conversion, which ones depending on the code around
+                    V8 v[2];
 #pragma unroll
-                for (int k = 0; k < 16; ++k) row[32 + k] = (T)sh[k];
-            } else {
+                    for (int k = 0; k < 16; ++k) {
+                        if (k > 1) asm("" : "+v"(sh[k]));
+                        v[k / 8][k % 8] = (T)sh[k];
+                    }
+                    *reinterpret_cast<V8*>(row + 32) = v[0];
+                    *reinterpret_cast<V8*>(row + 40) = v[1];
+                }
+            } else if (part == 0) {
                 for (int k = 0; k < 48; ++k) row[k] = (T)0.0f;
             }
             // extra-dims selector in the row's padding (halfs 48-49, 4-byte aligned)
@@ -448,8 +479,8 @@ __global__ __launch_bounds__(256, 4) void network_x32_kernel(const _Float16* __r
             }
         }
         __syncthreads();
-        for (uint32_t nb = 0; nb < 4; ++nb) {
-            const uint32_t s = wave * 64 + nb * 16 + col;
+        for (uint32_t nb = 0; nb < NB; ++nb) {
+            const uint32_t s = (wave * NB + nb) * 16 + col;
             const T* xr = s_x + s * kX32Stride;
             V8 bx;
 #pragma unroll
@@ -489,8 +520,24 @@ __global__ __launch_bounds__(256, 4) void network_x32_kernel(const _Float16* __r
     }
 }
 
+template <int L, int X, typename T, class Src>
+__global__ __launch_bounds__(256, 4) void network_x32_kernel(const _Float16* __restrict__ table, GridParams gp,
+                                                          const T* __restrict__ frag, const float* __restrict__ xbias,
+                                                          uint32_t xrows, Src src) {
+    typedef typename Vec8<T>::type V8;
+    __shared__ __attribute__((aligned(16))) T s_x[kTile * kX32Stride];
+    const uint32_t lane = threadIdx.x & 63u;
+    // weight fragments into registers (kFragX32 x 8 values per lane)
+    V8 A[kFragX32];
+#pragma unroll
+    for (uint32_t f = 0; f < kFragX32; ++f) A[f] = *reinterpret_cast<const V8*>(frag + ((size_t)f * 64 + lane) * 8);
+    const uint32_t n = src.count();
+    if (n <= kSmallTileMax) x32_tiles<L, X, 1>(s_x, A, table, gp, xbias, xrows, n, src);
+    else x32_tiles<L, X, 4>(s_x, A, table, gp, xbias, xrows, n, src);
+}
+
 uint32_t grid_for(uint32_t n_max) {
-    const uint32_t tiles = (n_max + kTile - 1) / kTile;
+    const uint32_t tiles = (n_max + kTile / 4 - 1) / (kTile / 4);
     const uint32_t cap = 256 * 8;
     if (tiles >= cap) return cap;
     return tiles >= 8 ? (tiles + 7u) / 8u * 8u : (tiles ? tiles : 1);  // whole XCD rounds when possible

@@ -1746,21 +1746,13 @@ __global__ __launch_bounds__(128) void net_input_grad_kernel(const float* __rest
         for (int j = 0; j < 16; ++j) dsh[j] += params[O::W2 + k * kCin + 16 + j] * d2;
     }
     const float4 p4 = cpos[i];
-    const float xs[3] = {p4.x, p4.y, p4.z};
     float gx[3] = {0.0f, 0.0f, 0.0f};
     for (int l = 0; l < L; ++l) {
         const float sc = gp.scale[l];
-        float frac[3];
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            const float pp = xs[d] * sc + 0.5f;
-            frac[d] = pp - floorf(pp);
-        }
-        uint32_t corner[8];
-        float weight[8];
-        const Pairs pairs = cell_corners(gp, (uint32_t)l, xyz(p4), corner, weight);
+        float frac[3], weight[8];
         float2 v[8];
-        gather_corners(reinterpret_cast<const char*>(table + 2 * (size_t)gp.offset[l]), corner, pairs, v);
+        cell_fetch(gp, (uint32_t)l, xyz(p4), reinterpret_cast<const char*>(table + 2 * (size_t)gp.offset[l]), v, frac,
+                   weight);
 #pragma unroll
         for (uint32_t c = 0; c < 8; ++c) {
             float wk[3];

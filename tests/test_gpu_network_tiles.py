@@ -1,0 +1,35 @@
+"""The matrix-core network takes up to 2^17 samples in tiles of 64 and more in
+tiles of 256: an output depends on its own sample alone, so a call of any size
+returns, bit for bit, what the same samples return within a larger call.  Sizes
+at the edges of both tiles and on both sides of the line, with positions inside
+and outside the unit cube (where dense levels wrap)."""
+import numpy as np
+import pytest
+
+from insta_amd import synth
+from insta_amd.capi import PRECISION_BF16, PRECISION_FP16, PRECISION_FP32, full_config, small_config
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("precision", [PRECISION_FP32, PRECISION_FP16, PRECISION_BF16])
+@pytest.mark.parametrize("config", [small_config, full_config])
+def test_outputs_do_not_depend_on_the_tile(config, precision):
+    torch = pytest.importorskip("torch")
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from insta_amd.capi import Context
+    cfg = config(max_frames=1, precision=precision, n_extra_dims=0)
+    ctx = Context(cfg)
+    p = synth.network_params(7, ctx.layout, cfg)
+    p[ctx.layout.n_mlp_params:] = np.random.default_rng(3).uniform(
+        -0.3, 0.3, ctx.layout.n_grid_params).astype(np.float32)
+    ctx.set_params(torch.from_numpy(p).cuda())
+    rng = np.random.default_rng(5)
+    c = rng.uniform(0.0, 1.0, ((1 << 17) + 257, 11)).astype(np.float32)
+    c[::7, :3] = rng.uniform(-0.5, 1.5, c[::7, :3].shape)
+    c = torch.from_numpy(c).cuda()
+    whole = ctx.network_inference(c)
+    assert torch.isfinite(whole).all()
+    for n in (1, 15, 17, 63, 64, 65, 255, 257, 4097, 1 << 17):
+        assert torch.equal(ctx.network_inference(c[:n].contiguous()), whole[:n]), n
