@@ -85,7 +85,13 @@ constexpr int kCin = 32;             // density outputs + 16 SH
 constexpr uint32_t kMlpThreads = 256;  // backward: one weight copy in LDS per block
 constexpr uint32_t kChunk = 1024;    // samples per weight-gradient partial
 constexpr uint32_t kRaySeedStride = 8;
-constexpr uint32_t kRayWaves = 4;    // waves per workgroup of the per-ray kernels
+// One wave per workgroup of the per-ray kernels: a step has thousands of rays
+// where the chip has 1,024 SIMDs, and each lane walks its ray's samples one
+// after another, so a wave wants a CU (its L1, its memory port) to itself.
+// 8,192 rays, waves of four a workgroup / one: loss 180 / 108 us, the four
+// rounds' kernels 135 / 48 us, rays 124 / 111 us.
+constexpr uint32_t kRayThreads = 64;
+constexpr uint32_t kRayWaves = kRayThreads / 64;
 // backward: wave-level run sums on levels where one marching step covers at
 // most this fraction of a cell (runs of about two or more samples per entry)
 constexpr float kRunMaxStepCells = 0.5f;
@@ -227,7 +233,7 @@ INSTA_DEV bool train_ray(const RayArgs& a, uint32_t i, uint32_t n_rays, uint64_t
     return true;
 }
 
-__global__ __launch_bounds__(256) void train_rays_kernel(RayArgs a, uint32_t n_rays, uint64_t rays_total,
+__global__ __launch_bounds__(kRayThreads) void train_rays_kernel(RayArgs a, uint32_t n_rays, uint64_t rays_total,
                                                          Pcg32 rng, float4* __restrict__ ray_d,
                                                          float4* __restrict__ ray_o,
                                                          int32_t* __restrict__ ray_frame,
@@ -462,9 +468,33 @@ INSTA_DEV float transmit(float T, float density_logit, float density_bias, float
     return T * (1.0f - alpha);
 }
 
+// f(j, load(j)) for j = 0..n-1 in order until it returns false.  A lane's walk
+// over its ray is a chain of memory latencies if each sample is loaded when it
+// is wanted: four are loaded while the four before them are worked on.
+// 8,192 rays: loss 193 us without, 180 us (108 us with one wave a workgroup);
+// gathers of the four rounds 64 -> 41 us (32 us).
+template <class V, class Load, class F>
+INSTA_DEV void walk_ray(uint32_t n, Load load, F f) {
+    if (n == 0) return;
+    V next[4];
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k) next[k] = load(min(k, n - 1u));
+    for (uint32_t j = 0; j < n; j += 4) {
+        V cur[4];
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k) {
+            cur[k] = next[k];
+            next[k] = load(min(j + 4u + k, n - 1u));
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k)
+            if (j + k < n && !f(j + k, cur[k])) return;
+    }
+}
+
 // Round `w` gather: the window's samples of every alive ray, packed into the
 // round buffers (each ray's samples contiguous from ray_gbase).
-__global__ __launch_bounds__(256) void train_gather_kernel(uint32_t lo, uint32_t hi,
+__global__ __launch_bounds__(kRayThreads) void train_gather_kernel(uint32_t lo, uint32_t hi,
                                                            const uint32_t* __restrict__ ray_base,
                                                            const uint32_t* __restrict__ ray_cnt,
                                                            const uint32_t* __restrict__ ray_alive,
@@ -489,16 +519,19 @@ __global__ __launch_bounds__(256) void train_gather_kernel(uint32_t lo, uint32_t
     const float4 o4 = ray_o[r], d4 = ray_d[r];
     const V3 o = v3(o4.x, o4.y, o4.z), d = v3(d4.x, d4.y, d4.z);
     const float* __restrict__ tr = t_buf + ray_src[r];
-    for (uint32_t k = 0; k < n; ++k) {
-        const V3 pos = o + d * tr[(size_t)(lo + k) * t_stride];
-        r_pos[g + k] = make_float4(pos.x, pos.y, pos.z, __uint_as_float(r));
-    }
+    walk_ray<float>(
+        n, [&](uint32_t k) { return tr[(size_t)(lo + k) * t_stride]; },
+        [&](uint32_t k, float t) {
+            const V3 pos = o + d * t;
+            r_pos[g + k] = make_float4(pos.x, pos.y, pos.z, __uint_as_float(r));
+            return true;
+        });
 }
 
 // Round `w` scatter and transmittance: each alive ray's evaluated samples go
 // back to their marched slots, and its transmittance advances over them; the
 // ray stays alive only while it is >= 1e-4 with samples left past the window.
-__global__ __launch_bounds__(256) void train_round_kernel(uint32_t lo, uint32_t hi, float density_bias, float dt,
+__global__ __launch_bounds__(kRayThreads) void train_round_kernel(uint32_t lo, uint32_t hi, float density_bias, float dt,
                                                           const uint32_t* __restrict__ ray_base,
                                                           const uint32_t* __restrict__ ray_cnt,
                                                           uint32_t* __restrict__ ray_alive,
@@ -517,16 +550,21 @@ __global__ __launch_bounds__(256) void train_round_kernel(uint32_t lo, uint32_t 
     const uint32_t base = ray_base[r] + lo, g = ray_gbase[r];
     float T = ray_T[r];
     bool alive = n > 0;
-    for (uint32_t k = 0; k < n; ++k) {
-        const float4 o = r_out[g + k];
-        s_cpos[base + k] = r_cpos[g + k];
-        s_cdir[base + k] = r_cdir[g + k];
-        s_out[base + k] = o;
-        if (alive) {
-            T = transmit(T, o.w, density_bias, dt);
-            if (T < 1e-4f) alive = false;
-        }
-    }
+    struct Sample {
+        float4 out, cpos, cdir;
+    };
+    walk_ray<Sample>(
+        n, [&](uint32_t k) { return Sample{r_out[g + k], r_cpos[g + k], r_cdir[g + k]}; },
+        [&](uint32_t k, const Sample& q) {
+            s_cpos[base + k] = q.cpos;
+            s_cdir[base + k] = q.cdir;
+            s_out[base + k] = q.out;
+            if (alive) {
+                T = transmit(T, q.out.w, density_bias, dt);
+                if (T < 1e-4f) alive = false;
+            }
+            return true;
+        });
     ray_T[r] = T;
     ray_alive[r] = alive && cnt > hi ? 1u : 0u;
 }
@@ -534,7 +572,8 @@ __global__ __launch_bounds__(256) void train_round_kernel(uint32_t lo, uint32_t 
 INSTA_DEV float srgb_to_linear(float c) { return c <= 0.04045f ? c / 12.92f : powf((c + 0.055f) / 1.055f, 2.4f); }
 INSTA_DEV float linear_to_srgb(float c) { return c < 0.0031308f ? 12.92f * c : 1.055f * powf(c, 0.41666f) - 0.055f; }
 
-__global__ __launch_bounds__(256) void train_loss_kernel(LossArgs a, Pcg32 rng0, const uint32_t* __restrict__ ray_src,
+__global__ __launch_bounds__(kRayThreads) void train_loss_kernel(LossArgs a, Pcg32 rng0,
+                                                         const uint32_t* __restrict__ ray_src,
                                                          const uint32_t* __restrict__ ray_img,
                                                          const uint32_t* __restrict__ ray_pix,
                                                          const uint32_t* __restrict__ ray_base,
@@ -554,6 +593,13 @@ __global__ __launch_bounds__(256) void train_loss_kernel(LossArgs a, Pcg32 rng0,
     float depth_ray = 0.0f, dgrad = 0.0f;
     V3 org = v3(0.0f, 0.0f, 0.0f), dir = v3(0.0f, 0.0f, 1.0f);
     const float* __restrict__ tr = t_buf;  // this ray's march t values, stride t_stride
+    struct RaySample {
+        float4 out;
+        float t;
+    };
+    const auto load_sample = [&](uint32_t j, bool with_t) {
+        return RaySample{s_out[base + j], with_t ? tr[(size_t)j * t_stride] : 0.0f};
+    };
     if (valid) {
         base = ray_base[r];
         tr = t_buf + ray_src[r];
@@ -592,21 +638,24 @@ __global__ __launch_bounds__(256) void train_loss_kernel(LossArgs a, Pcg32 rng0,
         const float target_depth = ro.w * ((lam > 0.0f && a.depth) ? a.depth[texel] : -1.0f);
         const bool supervise_depth = target_depth > 0.0f;
         float T = 1.0f;
-        for (; used < cnt; ++used) {
-            if (T < 1e-4f) break;
-            const float4 o = s_out[base + used];
-            const float sigma = expf(o.w + a.density_bias);
-            const float alpha = 1.0f - expf(-sigma * a.dt);
-            const float w = alpha * T;
-            acc[0] = acc[0] + w * sigmoid(o.x);
-            acc[1] = acc[1] + w * sigmoid(o.y);
-            acc[2] = acc[2] + w * sigmoid(o.z);
-            if (supervise_depth) {
-                const V3 p = org + dir * tr[(size_t)used * t_stride];
-                depth_ray = depth_ray + w * norm(p - org);
-            }
-            T = T * (1.0f - alpha);  // = transmit(T, o.w, ...), which the rounds use
-        }
+        walk_ray<RaySample>(
+            cnt, [&](uint32_t j) { return load_sample(j, supervise_depth); },
+            [&](uint32_t, const RaySample& q) {
+                if (T < 1e-4f) return false;
+                const float sigma = expf(q.out.w + a.density_bias);
+                const float alpha = 1.0f - expf(-sigma * a.dt);
+                const float w = alpha * T;
+                acc[0] = acc[0] + w * sigmoid(q.out.x);
+                acc[1] = acc[1] + w * sigmoid(q.out.y);
+                acc[2] = acc[2] + w * sigmoid(q.out.z);
+                if (supervise_depth) {
+                    const V3 p = org + dir * q.t;
+                    depth_ray = depth_ray + w * norm(p - org);
+                }
+                T = T * (1.0f - alpha);  // = transmit(T, o.w, ...), which the rounds use
+                ++used;
+                return true;
+            });
         // L1 depth loss (depth_loss_type's default, testbed_nerf.cu:133-139)
         if (supervise_depth) dgrad = copysignf(1.0f, depth_ray - target_depth) * lam;
         if (used == cnt) {
@@ -629,8 +678,8 @@ __global__ __launch_bounds__(256) void train_loss_kernel(LossArgs a, Pcg32 rng0,
         const float ls = a.loss_scale_per_ray;
         float T = 1.0f;
         float acc2[3] = {0.0f, 0.0f, 0.0f}, depth2 = 0.0f;
-        for (uint32_t j = 0; j < n_c; ++j) {
-            const float4 o = s_out[base + j];
+        const auto backprop = [&](uint32_t j, const RaySample& q) {
+            const float4 o = q.out;
             const float sg[3] = {sigmoid(o.x), sigmoid(o.y), sigmoid(o.z)};
             const float sigma = expf(o.w + a.density_bias);
             const float alpha = 1.0f - expf(-sigma * a.dt);
@@ -645,14 +694,16 @@ __global__ __launch_bounds__(256) void train_loss_kernel(LossArgs a, Pcg32 rng0,
             }
             if (dgrad != 0.0f) {
                 // dD/dsigma_j / dt = T_{j+1} depth_j - (depth suffix after j)
-                const V3 p = org + dir * tr[(size_t)j * t_stride];
+                const V3 p = org + dir * q.t;
                 const float dj = norm(p - org);
                 depth2 = depth2 + w * dj;
                 dsig = dsig + dgrad * (T * dj - (depth_ray - depth2));
             }
             c_idx[cb + j] = base + j;
             c_dout[cb + j] = make_float4(drgb[0], drgb[1], drgb[2], ls * (sigma * (a.dt * dsig)));
-        }
+            return true;
+        };
+        walk_ray<RaySample>(n_c, [&](uint32_t j) { return load_sample(j, dgrad != 0.0f); }, backprop);
     }
     // statistics, one atomic each per workgroup
     __shared__ uint32_t s_used;
@@ -1942,17 +1993,17 @@ insta_status train_step(insta_ctx* ctx, const insta_train_config& tc, insta_trai
     ra.height = ts->height;
     ra.max_samples = cap;
     ra.fixed_slot = tc.occupancy_slot;
-    hipLaunchKernelGGL(train_rays_kernel, dim3((n_rays + 255) / 256), dim3(256), 0, stream, ra, n_rays, ts->rays_total,
-                       rng, ts->ray_d, ts->ray_o, ts->ray_frame, ts->ray_img, ts->ray_pix, ts->ray_src, ts->ray_base,
+    hipLaunchKernelGGL(train_rays_kernel, dim3((n_rays + kRayThreads - 1) / kRayThreads), dim3(kRayThreads), 0, stream,
+                       ra, n_rays, ts->rays_total, rng, ts->ray_d, ts->ray_o, ts->ray_frame, ts->ray_img, ts->ray_pix, ts->ray_src, ts->ray_base,
                        ts->ray_cnt, ts->t_buf, ts->ray_T, ts->ray_alive, ts->counters);
     INSTA_HIP(hipGetLastError());
     hipLaunchKernelGGL(train_count_kernel, dim3(1), dim3(64), 0, stream, ts->counters);
     // deform and evaluate the marched samples window by window, only while
     // their rays are still alive
-    const dim3 rgrid((n_rays + 255) / 256);
+    const dim3 rgrid((n_rays + kRayThreads - 1) / kRayThreads);
     for (uint32_t w = 0; w < kRounds; ++w) {
         const uint32_t lo = kWin[w], hi = kWin[w + 1];
-        hipLaunchKernelGGL(train_gather_kernel, rgrid, dim3(256), 0, stream, lo, hi, ts->ray_base, ts->ray_cnt,
+        hipLaunchKernelGGL(train_gather_kernel, rgrid, dim3(kRayThreads), 0, stream, lo, hi, ts->ray_base, ts->ray_cnt,
                            ts->ray_alive, ts->ray_gbase, ts->ray_o, ts->ray_d, ts->ray_src, ts->t_buf, n_rays,
                            ts->r_pos, ts->counters, kTRound0 + w);
         INSTA_HIP(hipGetLastError());
@@ -1967,7 +2018,7 @@ insta_status train_step(insta_ctx* ctx, const insta_train_config& tc, insta_trai
         if (st != INSTA_OK) return st;
         st = launch_network_samples(ctx, n_round, cap, ts->r_cpos, ts->r_cdir, ts->r_out, stream);
         if (st != INSTA_OK) return st;
-        hipLaunchKernelGGL(train_round_kernel, rgrid, dim3(256), 0, stream, lo, hi, ctx->cfg.density_logit_bias,
+        hipLaunchKernelGGL(train_round_kernel, rgrid, dim3(kRayThreads), 0, stream, lo, hi, ctx->cfg.density_logit_bias,
                            ctx->cfg.dt, ts->ray_base, ts->ray_cnt, ts->ray_alive, ts->ray_gbase, ts->ray_T,
                            ts->r_cpos, ts->r_cdir, ts->r_out, ts->s_cpos, ts->s_cdir, ts->s_out, ts->counters);
         INSTA_HIP(hipGetLastError());
@@ -1984,7 +2035,7 @@ insta_status train_step(insta_ctx* ctx, const insta_train_config& tc, insta_trai
     la.density_bias = ctx->cfg.density_logit_bias;
     la.loss_scale_per_ray = tc.loss_scale / (float)n_rays;
     la.inv_rays = 1.0f / (float)n_rays;
-    hipLaunchKernelGGL(train_loss_kernel, dim3((n_rays + 255) / 256), dim3(256), 0, stream, la, rng, ts->ray_src,
+    hipLaunchKernelGGL(train_loss_kernel, rgrid, dim3(kRayThreads), 0, stream, la, rng, ts->ray_src,
                        ts->ray_img, ts->ray_pix, ts->ray_base, ts->ray_cnt, ts->ray_o, ts->ray_d, ts->t_buf,
                        n_rays, ts->s_out,
                        ts->c_idx, ts->c_dout,
