@@ -83,7 +83,19 @@ constexpr int kW = 64;
 constexpr int kDOut = 16;
 constexpr int kCin = 32;             // density outputs + 16 SH
 constexpr uint32_t kMlpThreads = 256;  // backward: one weight copy in LDS per block
-constexpr uint32_t kChunk = 1024;    // samples per weight-gradient partial
+// Samples per weight-gradient partial: a batch in 64 chunks of whole LDS
+// slices (32 samples), between 128 and 1,024 samples each.  A chunk's slices
+// follow one another, so a small batch in chunks of 1,024 sat on a few CUs
+// (1,000 samples: 48 us, in chunks of 128 9 us).
+constexpr uint32_t kChunk = 1024, kChunkMin = 128, kChunksFew = 64;
+__host__ __device__ inline uint32_t wgrad_chunk(uint32_t n) {
+    const uint32_t c = (n + 32u * kChunksFew - 1u) / (32u * kChunksFew) * 32u;
+    return c < kChunkMin ? kChunkMin : (c > kChunk ? kChunk : c);
+}
+// chunks of any batch of up to cap samples, at most
+inline uint32_t wgrad_chunks(uint32_t cap) {
+    return std::max((cap + kChunk - 1) / kChunk, std::min(kChunksFew, (cap + kChunkMin - 1) / kChunkMin));
+}
 constexpr uint32_t kRaySeedStride = 8;
 // One wave per workgroup of the per-ray kernels: a step has thousands of rays
 // where the chip has 1,024 SIMDs, and each lane walks its ray's samples one
@@ -296,6 +308,21 @@ INSTA_DEV void store_rows(float* __restrict__ act, uint32_t ld, int row0, uint32
 // per sample from x_extra [n][X] when given.
 typedef float tf_f4 __attribute__((ext_vector_type(4)));
 constexpr uint32_t kFwdTile = 256;
+
+// Column blocks of 16 samples a wave of the forward and backward kernels
+// takes: four, or one where the batch is small, so that a workgroup has 64
+// samples instead of 256, a quarter of the levels a wave to encode, and a
+// quarter of the latency.
+// 1,000 samples: backward 58 -> 16 us, forward 40 -> 13 us; at 100,000 (head)
+// four columns: forward 145 us, one column 148 us, backward 84 / 82 us; above
+// that one column costs the forward more (126 against 121 us at 8,192 rays).
+constexpr uint32_t kSmallBatch = 65536;
+INSTA_DEV uint32_t tile_columns(uint32_t n) { return n <= kSmallBatch ? 1u : 4u; }
+// workgroups that cover any batch of up to cap samples
+uint32_t mlp_blocks(uint32_t cap) {
+    return std::max((cap + kFwdTile - 1) / kFwdTile, (std::min(cap, kSmallBatch) + kFwdTile / 4 - 1) / (kFwdTile / 4));
+}
+
 template <int L, int X>
 __global__ __launch_bounds__(256) void train_forward_kernel(const float* __restrict__ params,
                                                           const float* __restrict__ table, GridParams gp,
@@ -313,13 +340,15 @@ __global__ __launch_bounds__(256) void train_forward_kernel(const float* __restr
     using O = Off<DIN>;
     __shared__ float s_x[kFwdTile * S];
     const uint32_t n = *n_dev;
-    const uint32_t base = blockIdx.x * kFwdTile;
+    const uint32_t cols = tile_columns(n), samples = 64u * cols;
+    const uint32_t base = blockIdx.x * samples;
     if (base >= n) return;  // whole block past the batch
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
     const uint32_t m = lane & 15u, g = lane >> 4;
     {
-        const uint32_t i = base + tid;
-        float* row = s_x + tid * S;
+        const uint32_t i = base + tid % samples;
+        const int part = __builtin_amdgcn_readfirstlane((int)(tid / samples)), per = (int)(L / 4u * cols);
+        float* row = s_x + tid % samples * S;
         if (i < n) {
             const uint32_t smp = c_idx[i];
             const float4 p4 = cpos[smp], d4 = cdir[smp];
@@ -327,7 +356,7 @@ __global__ __launch_bounds__(256) void train_forward_kernel(const float* __restr
             // two levels' gathers in flight; rolled, so that a level's
             // corners do not all live at once (one wave per SIMD)
 #pragma unroll 2
-            for (int l = 0; l < L; ++l) {
+            for (int l = part * per; l < (part + 1) * per; ++l) {
                 float f[2];
                 encode_level<2>(table, gp, (uint32_t)l, x, f);
 #pragma unroll
@@ -336,22 +365,24 @@ __global__ __launch_bounds__(256) void train_forward_kernel(const float* __restr
                     act[(size_t)(A::ENC + 2 * l + k) * ld + i] = f[k];
                 }
             }
-            if constexpr (X > 0) {
-                const uint32_t sel = __float_as_uint(d4.w);
-                const float* fx = x_extra ? x_extra + (size_t)smp * X
-                                          : (sel != kExtraOnes && sel <= n_frames ? frame_extra + (size_t)(sel - 1u) * X
-                                                                                  : nullptr);
+            if (part == 0) {
+                if constexpr (X > 0) {
+                    const uint32_t sel = __float_as_uint(d4.w);
+                    const float* fx = x_extra ? x_extra + (size_t)smp * X
+                                              : (sel != kExtraOnes && sel <= n_frames ? frame_extra + (size_t)(sel - 1u) * X
+                                                                                      : nullptr);
 #pragma unroll
-                for (int e = 0; e < X; ++e) {
-                    const float v = fx ? fx[e] : 1.0f;
-                    row[E + e] = v;
-                    act[(size_t)(A::ENC + E + e) * ld + i] = v;
+                    for (int e = 0; e < X; ++e) {
+                        const float v = fx ? fx[e] : 1.0f;
+                        row[E + e] = v;
+                        act[(size_t)(A::ENC + E + e) * ld + i] = v;
+                    }
                 }
+                float sh[16];
+                sh16(d4.x * 2.0f - 1.0f, d4.y * 2.0f - 1.0f, d4.z * 2.0f - 1.0f, sh);
+                store_rows<16, 16>(act, ld, A::SH, i, sh);
             }
-            float sh[16];
-            sh16(d4.x * 2.0f - 1.0f, d4.y * 2.0f - 1.0f, d4.z * 2.0f - 1.0f, sh);
-            store_rows<16, 16>(act, ld, A::SH, i, sh);
-        } else {
+        } else if (part == 0) {
 #pragma unroll
             for (int k = 0; k < DIN; ++k) row[k] = 0.0f;
         }
@@ -361,8 +392,8 @@ __global__ __launch_bounds__(256) void train_forward_kernel(const float* __restr
     const float* W1 = params + O::W1;
     const float* W2 = params + O::W2;
     const float* W3 = params + O::W3;
-    for (uint32_t nb = 0; nb < 4; ++nb) {
-        const uint32_t s = wave * 64 + nb * 16 + m;  // column (sample) of this lane
+    for (uint32_t nb = 0; nb < cols; ++nb) {
+        const uint32_t s = (wave * cols + nb) * 16 + m;  // column (sample) of this lane
         const uint32_t i = base + s;
         const bool live = i < n;
         const float* xr = s_x + s * S;
@@ -1238,16 +1269,20 @@ __global__ __launch_bounds__(kMlpThreads) void train_backward_kernel(const float
     using A = Act<DIN>;
     using O = Off<DIN>;
     typedef float bf4 __attribute__((ext_vector_type(4)));
-    __shared__ float w[O::N];                  // both MLPs' weights
+    __shared__ __attribute__((aligned(16))) float w[O::N];  // both MLPs' weights
     __shared__ float s_denc[E][kMlpThreads];   // dL/dencoding of the block's samples
     const uint32_t n = *n_dev;
-    const uint32_t base = blockIdx.x * kMlpThreads;
+    const uint32_t cols = tile_columns(n), samples = 64u * cols;
+    const uint32_t base = blockIdx.x * samples;
     if (base >= n) return;  // whole block past the batch
-    for (uint32_t e = threadIdx.x; e < O::N; e += kMlpThreads) w[e] = params[e];
+    static_assert(O::N % 4 == 0, "whole float4s of weights");
+#pragma unroll 8
+    for (uint32_t e = 4u * threadIdx.x; e < O::N; e += 4u * kMlpThreads)
+        *reinterpret_cast<float4*>(w + e) = *reinterpret_cast<const float4*>(params + e);
     __syncthreads();
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
     const uint32_t m = lane & 15u, g = lane >> 4;
-    for (uint32_t nb = 0; nb < 4; ++nb) {
+    for (uint32_t nb = 0; nb < cols; ++nb) {
         // Opaque copies of 0 and ld: the weight reads (LDS) and the row
         // addresses of act/dact are formed inside this loop.  Loop-invariant,
         // they were otherwise hoisted out of it into ~360 registers (1 wave
@@ -1259,9 +1294,19 @@ __global__ __launch_bounds__(kMlpThreads) void train_backward_kernel(const float
         const float* W2 = w + O::W2 + z;
         const float* W3 = w + O::W3 + z;
         const float* W4 = w + O::W4 + z;
-        const uint32_t s = wave * 64 + nb * 16 + m;  // column (sample) of this lane
+        const uint32_t s = (wave * cols + nb) * 16 + m;  // column (sample) of this lane
         const uint32_t i = base + s;
         const bool live = i < n;
+        // the masks of all layers at once: loaded layer by layer, each layer
+        // waited for its own
+        bool on1[16], on2[16], on3[16];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) {
+            const uint32_t row = 16 * (k / 4) + 4 * g + k % 4;
+            on3[k] = live && act[(size_t)(A::H3 + row) * ldz + i] > 0.0f;
+            on2[k] = live && act[(size_t)(A::H2 + row) * ldz + i] > 0.0f;
+            on1[k] = live && act[(size_t)(A::H1 + row) * ldz + i] > 0.0f;
+        }
         const float4 d4 = live ? dout[i] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         // colour output layer: dH3 = relu'(H3) (W4^T dRGB), K = 3 rgb rows (+ one zero)
         const float b_rgb = g == 0 ? d4.x : (g == 1 ? d4.y : (g == 2 ? d4.z : 0.0f));
@@ -1273,7 +1318,7 @@ __global__ __launch_bounds__(kMlpThreads) void train_backward_kernel(const float
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const uint32_t row = 16 * t + 4 * g + q;
-                dh3[t][q] = live && act[(size_t)(A::H3 + row) * ldz + i] > 0.0f ? acc[q] : 0.0f;
+                dh3[t][q] = on3[4 * t + q] ? acc[q] : 0.0f;
                 if (live) dact[(size_t)(Dact::DH3 + row) * ldz + i] = dh3[t][q];
             }
         }
@@ -1291,7 +1336,7 @@ __global__ __launch_bounds__(kMlpThreads) void train_backward_kernel(const float
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const uint32_t row = 16 * t + 4 * g + q;
-                dh2[t][q] = live && act[(size_t)(A::H2 + row) * ldz + i] > 0.0f ? acc[q] : 0.0f;
+                dh2[t][q] = on2[4 * t + q] ? acc[q] : 0.0f;
                 if (live) dact[(size_t)(Dact::DH2 + row) * ldz + i] = dh2[t][q];
             }
         }
@@ -1317,7 +1362,7 @@ __global__ __launch_bounds__(kMlpThreads) void train_backward_kernel(const float
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const uint32_t row = 16 * t + 4 * g + q;
-                dh1[t][q] = live && act[(size_t)(A::H1 + row) * ldz + i] > 0.0f ? acc[q] : 0.0f;
+                dh1[t][q] = on1[4 * t + q] ? acc[q] : 0.0f;
                 if (live) dact[(size_t)(Dact::DH1 + row) * ldz + i] = dh1[t][q];
             }
         }
@@ -1336,10 +1381,10 @@ __global__ __launch_bounds__(kMlpThreads) void train_backward_kernel(const float
         }
     }
     __syncthreads();
-    const uint32_t i = base + tid;
+    const uint32_t i = base + tid % samples, part = tid / samples;
     if ((i & ~63u) >= n) return;  // whole wave past the batch (no barrier follows)
     const bool valid = i < n;
-    if (valid) {
+    if (valid && part == 0) {
         const float4 d4 = dout[i];
         dact[(size_t)(Dact::DRGB + 0) * ld + i] = d4.x;
         dact[(size_t)(Dact::DRGB + 1) * ld + i] = d4.y;
@@ -1348,7 +1393,7 @@ __global__ __launch_bounds__(kMlpThreads) void train_backward_kernel(const float
     // dL/dencoding for the scatter kernels
     if (valid)
 #pragma unroll 4
-        for (int e = 0; e < E; ++e) denc_g[(size_t)e * ld + i] = s_denc[e][tid];
+        for (uint32_t e = part; e < E; e += 4u / cols) denc_g[(size_t)e * ld + i] = s_denc[e][tid % samples];
 }
 
 
@@ -1379,9 +1424,9 @@ __global__ __launch_bounds__(256) void wgrad_kernel(WArgs wa, const uint32_t* __
     __shared__ float Xs[64 * kP];
     const WProduct pr = wa.p[blockIdx.y];
     const uint32_t n = *n_dev;
-    const uint32_t s0 = blockIdx.x * kChunk;
+    const uint32_t chunk = wgrad_chunk(n), s0 = blockIdx.x * chunk;
     if (s0 >= n) return;
-    const uint32_t s1 = min(s0 + kChunk, n);
+    const uint32_t s1 = min(s0 + chunk, n);
     const uint32_t t = threadIdx.x, lane = t & 63u, wave = t >> 6;
     const uint32_t m = lane & 15u, g = lane >> 4;   // fragment row / k of this lane
     const uint32_t n_ot = (pr.O + 15u) / 16u;       // output tiles in use
@@ -1461,7 +1506,7 @@ __global__ void wgrad_reduce_kernel(const float* __restrict__ part, const uint32
                                     uint32_t n_mlp, float* __restrict__ grad) {
     const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= n_mlp) return;
-    const uint32_t nc = (*n_dev + kChunk - 1) / kChunk;
+    const uint32_t n = *n_dev, chunk = wgrad_chunk(n), nc = (n + chunk - 1) / chunk;
     // eight interleaved running sums (chunk c into sum c mod 8), added in a
     // fixed order: deterministic, with eight independent loads in flight
     float s[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
@@ -1561,7 +1606,7 @@ insta_status grow_train_workspace(insta_ctx* ctx, TrainState* ts, uint32_t n_ray
     ok = ok && train_alloc(ts->c_idx, cc * sizeof(uint32_t)) && train_alloc(ts->c_dout, cc * sizeof(float4));
     ok = ok && train_alloc(ts->act, act_rows * cc * sizeof(float));
     ok = ok && train_alloc(ts->dact, (size_t)Dact::N * cc * sizeof(float));
-    ok = ok && train_alloc(ts->part, ((cc + kChunk - 1) / kChunk) * n_mlp * sizeof(float));
+    ok = ok && train_alloc(ts->part, (size_t)wgrad_chunks(cc) * n_mlp * sizeof(float));
     ok = ok && train_alloc(ts->t_buf, (size_t)rc * ctx->cfg.max_steps * sizeof(float));
     ok = ok && train_alloc(ts->denc, (size_t)2 * INSTA_MAX_LEVELS * cc * sizeof(float));
     const GridParams gp = grid_params(ctx);
@@ -1606,7 +1651,7 @@ insta_status launch_train_forward(insta_ctx* ctx, TrainState* ts, hipStream_t st
     const uint32_t* n_dev = ts->counters + kTCompactN;
     const float* table = ctx->d_params + ctx->layout.n_mlp_params;
     const GridParams gp = grid_params(ctx);
-    const dim3 sgrid((cap + kFwdTile - 1) / kFwdTile);
+    const dim3 sgrid(mlp_blocks(cap));
     hipLaunchKernelGGL((train_forward_kernel<L, X>), sgrid, dim3(kFwdTile), 0, stream, ctx->d_params, table, gp,
                        ctx->d_frame_extra, ctx->cfg.max_frames, n_dev, ts->c_idx, ts->s_cpos, ts->s_cdir,
                        static_cast<const float*>(nullptr), ts->act, cap, static_cast<float4*>(nullptr));
@@ -1637,7 +1682,7 @@ insta_status launch_train_backward(insta_ctx* ctx, TrainState* ts, const insta_t
     const uint32_t* n_dev = ts->counters + kTCompactN;
     const GridParams gp = grid_params(ctx);
     const uint32_t n_mlp = (uint32_t)ctx->layout.n_mlp_params;
-    const dim3 sgrid((cap + kMlpThreads - 1) / kMlpThreads);
+    const dim3 sgrid(mlp_blocks(cap));
     float* grad_tab = ts->grad + n_mlp;
     // levels whose tables fit in LDS are scattered by scatter_lds_kernel (FP32
     // or packed FP16), the others by scatter_levels_kernel (FP32)
@@ -1704,7 +1749,7 @@ insta_status launch_train_backward(insta_ctx* ctx, TrainState* ts, const insta_t
     wa.p[2] = WProduct{Dact::DH2, A::DENS, kW, kCin, O::W2};
     wa.p[3] = WProduct{Dact::DH3, A::H2, kW, kW, O::W3};
     wa.p[4] = WProduct{Dact::DRGB, A::H3, 3, kW, O::W4};
-    const uint32_t n_chunks = (cap + kChunk - 1) / kChunk;
+    const uint32_t n_chunks = wgrad_chunks(cap);
     hipLaunchKernelGGL(wgrad_kernel, dim3(n_chunks, 5), dim3(256), 0, stream, wa, n_dev, ts->act, ts->dact, cap,
                        ts->part, n_mlp);
     INSTA_HIP(hipGetLastError());
@@ -1741,8 +1786,8 @@ __global__ void net_grad_out_kernel(const float* __restrict__ g, float* __restri
 
 // Input gradients of the backward (dL_dinput rows 0..2 and the direction rows
 // 8..10; the reference backpropagates through the position and direction
-// encodings only, nerf_network.h:318-380): dL/dencoding = W0^T dH1 and
-// dL/dSH = W2[:, 16:32]^T dH2 from the stored deltas; the position through
+// encodings only, nerf_network.h:318-380): dL/dencoding as the backward stored
+// it and dL/dSH = W2[:, 16:32]^T dH2 from the stored deltas; the position through
 // the derivative of each level's trilinear weights (scale_l per axis) times
 // the corner features, the direction (input in [0,1], d = 2 x - 1) through
 // the derivatives of the 16 SH polynomials.
@@ -1776,30 +1821,28 @@ __global__ __launch_bounds__(128) void net_input_grad_kernel(const float* __rest
                                                              const float* __restrict__ table, GridParams gp,
                                                              uint32_t n, const float4* __restrict__ cpos,
                                                              const float4* __restrict__ cdir,
-                                                             const float* __restrict__ dact, uint32_t ld,
+                                                             const float* __restrict__ dact,
+                                                             const float* __restrict__ denc_g, uint32_t ld,
                                                              float* __restrict__ dL_dinput, uint32_t stride) {
     constexpr int E = 2 * L, DIN = E + X;
     using O = Off<DIN>;
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    float denc[E];
-#pragma unroll
-    for (int e = 0; e < E; ++e) denc[e] = 0.0f;
     float dsh[16];
 #pragma unroll
     for (int j = 0; j < 16; ++j) dsh[j] = 0.0f;
+#pragma unroll 16
     for (int k = 0; k < kW; ++k) {
-        const float d1 = dact[(size_t)(Dact::DH1 + k) * ld + i];
         const float d2 = dact[(size_t)(Dact::DH2 + k) * ld + i];
-#pragma unroll
-        for (int e = 0; e < E; ++e) denc[e] += params[O::W0 + k * DIN + e] * d1;
 #pragma unroll
         for (int j = 0; j < 16; ++j) dsh[j] += params[O::W2 + k * kCin + 16 + j] * d2;
     }
     const float4 p4 = cpos[i];
     float gx[3] = {0.0f, 0.0f, 0.0f};
+#pragma unroll 2
     for (int l = 0; l < L; ++l) {
         const float sc = gp.scale[l];
+        const float de0 = denc_g[(size_t)(2 * l) * ld + i], de1 = denc_g[(size_t)(2 * l + 1) * ld + i];
         float frac[3], weight[8];
         float2 v[8];
         cell_fetch(gp, (uint32_t)l, xyz(p4), reinterpret_cast<const char*>(table + 2 * (size_t)gp.offset[l]), v, frac,
@@ -1809,7 +1852,7 @@ __global__ __launch_bounds__(128) void net_input_grad_kernel(const float* __rest
             float wk[3];
 #pragma unroll
             for (int k = 0; k < 3; ++k) wk[k] = ((c >> k) & 1u) ? frac[k] : 1.0f - frac[k];
-            const float s = denc[2 * l] * v[c].x + denc[2 * l + 1] * v[c].y;
+            const float s = de0 * v[c].x + de1 * v[c].y;
             gx[0] += s * (((c & 1u) ? sc : -sc) * wk[1] * wk[2]);
             gx[1] += s * (((c & 2u) ? sc : -sc) * wk[0] * wk[2]);
             gx[2] += s * (((c & 4u) ? sc : -sc) * wk[0] * wk[1]);
@@ -1831,7 +1874,7 @@ template <int L, int X>
 insta_status launch_net_forward(insta_ctx* ctx, TrainState* ts, float4* out, hipStream_t stream) {
     const uint32_t cap = ts->compact_cap;
     const float* table = ctx->d_params + ctx->layout.n_mlp_params;
-    hipLaunchKernelGGL((train_forward_kernel<L, X>), dim3((cap + kFwdTile - 1) / kFwdTile), dim3(kFwdTile), 0, stream,
+    hipLaunchKernelGGL((train_forward_kernel<L, X>), dim3(mlp_blocks(cap)), dim3(kFwdTile), 0, stream,
                        ctx->d_params, table, grid_params(ctx), ctx->d_frame_extra, ctx->cfg.max_frames,
                        ts->counters + kTCompactN, ts->c_idx, ts->s_cpos, ts->s_cdir,
                        X ? static_cast<const float*>(ts->net_extra) : nullptr, ts->act, cap, out);
@@ -1844,7 +1887,7 @@ insta_status launch_net_input_grad(insta_ctx* ctx, TrainState* ts, uint32_t n, f
                                    hipStream_t stream) {
     const float* table = ctx->d_params + ctx->layout.n_mlp_params;
     hipLaunchKernelGGL((net_input_grad_kernel<L, X>), dim3((n + 127) / 128), dim3(128), 0, stream, ctx->d_params,
-                       table, grid_params(ctx), n, ts->s_cpos, ts->s_cdir, ts->dact, ts->compact_cap, dL_dinput,
+                       table, grid_params(ctx), n, ts->s_cpos, ts->s_cdir, ts->dact, ts->denc, ts->compact_cap, dL_dinput,
                        stride);
     INSTA_HIP(hipGetLastError());
     return INSTA_OK;
