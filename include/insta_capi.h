@@ -476,8 +476,9 @@ typedef struct insta_train_config {
     float    loss_scale;      /* gradients are computed scaled by this, then unscaled */
     uint32_t grid_grad_fp16;  /* 1: hash-grid gradients accumulated in FP16 (packed atomics): per
                                  chunk of 8192 batch entries in LDS for levels of at most 16384
-                                 entries (the chunks then summed in FP32), per XCD copy for larger
-                                 levels; 0: FP32 throughout */
+                                 entries (the chunks then summed in FP32), in eight copies by batch
+                                 block (then summed in FP32) for larger levels; 0: FP32
+                                 throughout */
     uint32_t apply_update;    /* 0: gradients only, parameters unchanged */
     uint32_t seed;            /* PCG32 seed of the ray/background stream */
     int32_t  occupancy_slot;  /* grid the rays march: INSTA_OCCUPANCY_PER_FRAME (each image's

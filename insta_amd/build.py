@@ -7,8 +7,9 @@ with the source tree.  Flags that matter for correctness:
                            predicates round exactly as written (bit-exact
                            nearest-triangle ids, march steps, hash indices)
   -packed-fp32-ops off     no v_pk_* FP32 instructions
-  -munsafe-fp-atomics      hardware global_atomic_add_f32 for the hash-grid
-                           backward scatter (device memory is coarse-grained)
+  -munsafe-fp-atomics      hardware floating-point atomics for the hash-grid
+                           backward scatters: global_atomic_add_f32 and FP64
+                           adds in LDS (device memory is coarse-grained)
 """
 from __future__ import annotations
 

@@ -269,7 +269,9 @@ INSTA_DEV int32_t sample_frame(int32_t frame, const int32_t* __restrict__ ray_fr
 // (sample, best triangle so far); its samples' s_hit is kLongHit.
 constexpr int32_t kLongHit = -2;
 constexpr uint32_t kLongBlocks = 256;  // second pass: four waves per CU beside the first pass's samples
-constexpr uint32_t kRecordLongBlocks = 2048;  // the records' second pass runs alone: 408 us with 256 blocks, 170 us with these (2^20 samples)
+// the records' second pass runs alone: 408 us with 256 blocks, 170 us with
+// these (a full density-grid update's samples)
+constexpr uint32_t kRecordLongBlocks = 2048;
 
 // kCount: also sum the traversal work into counts[4] (queries, inner nodes,
 // leaves, triangles) -- a separate build for measurement runs
