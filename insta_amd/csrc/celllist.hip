@@ -119,8 +119,9 @@ __global__ void cl_cells_kernel(const uint64_t* __restrict__ bits, const uint32_
 struct ClArgs {
     MeshView m;
     const uint32_t* cells;
-    uint32_t* left;       // ranks of the cells cl_cell_kernel left over: after its first launch from
-                          // the front (state[5]), after its second from the back (state[6])
+    uint32_t* left;       // [2][cap] ranks of the cells cl_cell_kernel left over: by its first launch
+                          // (state[5] of them), and in words of their own, since the second launch
+                          // reads those while it writes these, by its second (state[6])
     uint32_t all;         // the per-lane kernels take every cell
     uint2* head;
     uint32_t* ent;
@@ -369,7 +370,7 @@ __global__ __launch_bounds__(kSecond ? kCellThreads2 : kCellThreads) void cl_cel
         if (overflow) {  // left to the second launch, then to the per-lane kernels
             if (tid == 0) {
                 if (kSecond)
-                    a.left[a.cap - 1u - atomicAdd(&a.state[6], 1u)] = rank;
+                    a.left[(size_t)a.cap + atomicAdd(&a.state[6], 1u)] = rank;
                 else
                     a.left[atomicAdd(&a.state[5], 1u)] = rank;
             }
@@ -470,7 +471,7 @@ __global__ __launch_bounds__(kSecond ? kCellThreads2 : kCellThreads) void cl_cel
 
 // cells the per-lane kernels walk, and the i-th one's rank
 INSTA_DEV uint32_t walk_cells(const ClArgs& a) { return a.all ? min(a.state[0], a.cap) : a.state[6]; }
-INSTA_DEV uint32_t walk_rank(const ClArgs& a, uint32_t i) { return a.all ? i : a.left[a.cap - 1u - i]; }
+INSTA_DEV uint32_t walk_rank(const ClArgs& a, uint32_t i) { return a.all ? i : a.left[(size_t)a.cap + i]; }
 
 __global__ __launch_bounds__(kClThreads) void cl_count_kernel(ClArgs a) {
     extern __shared__ uint32_t stack[];  // [stack_depth(k)][kClThreads]
@@ -590,7 +591,7 @@ ClArgs cl_args(insta_ctx* ctx, uint32_t slot) {
     a.head = ctx->d_cl_head + slot * (size_t)ctx->cfg.cell_list_cells * S * S * S;
     a.ent = ctx->d_cl_ent + slot * (size_t)ctx->cfg.cell_list_entries;
     a.state = ctx->d_cl_state + kClState * (size_t)slot;
-    a.left = ctx->d_cl_left + slot * (size_t)ctx->cfg.cell_list_cells;
+    a.left = ctx->d_cl_left + 2 * slot * (size_t)ctx->cfg.cell_list_cells;
     // a workgroup per cell pays for 64 sub-cells, not for 8 or 1: the small
     // sphere at S = 2 takes 230 + 150 us one lane per sub-cell, 920 us so
     a.all = S == 4 ? 0u : 1u;
@@ -615,7 +616,7 @@ insta_status alloc_cell_lists(insta_ctx* ctx) {
     alloc((void**)&ctx->d_cl_bits, n * words * sizeof(uint64_t));
     alloc((void**)&ctx->d_cl_rank, n * words * sizeof(uint32_t));
     alloc((void**)&ctx->d_cl_cells, n * cells * sizeof(uint32_t));
-    alloc((void**)&ctx->d_cl_left, n * cells * sizeof(uint32_t));
+    alloc((void**)&ctx->d_cl_left, 2 * n * cells * sizeof(uint32_t));
     alloc((void**)&ctx->d_cl_head, n * cells * S * S * S * sizeof(uint2));
     alloc((void**)&ctx->d_cl_ent, n * ents * sizeof(uint32_t));
     alloc((void**)&ctx->d_cl_state, n * kClState * sizeof(uint32_t));

@@ -203,3 +203,59 @@ def test_small_capacities_fall_back_to_the_bvh(head_avatar, caps):
     rid, rd2 = orc.closest_brute(0, pts)
     assert np.array_equal(ids.cpu().numpy(), rid)
     assert np.array_equal(dist.cpu().numpy(), np.sqrt(rd2))
+
+
+def _least_candidates(orc, verts, faces, cells, G, S):
+    """Triangles the per-cell build gathers for each cell, at least: those whose box lies within the largest
+    distance from a corner of the cell to the mesh, plus half a sub-cell's diagonal."""
+    tri = verts.astype(np.float64)[faces]
+    tlo, thi = tri.min(1), tri.max(1)
+    corner = np.array([[k & 1, (k >> 1) & 1, k >> 2] for k in range(8)])
+    pts = ((cells[:, None, :] + corner[None]) / G).reshape(-1, 3).astype(np.float32)
+    d2 = orc.closest_brute(0, pts)[1].reshape(-1, 8).max(1).astype(np.float64)
+    reach = np.sqrt(d2) + 0.5 * np.sqrt(3.0) / (G * S)
+    out = []
+    for c, r in zip(cells, reach):
+        gap = np.maximum(np.maximum(tlo - (c + 1) / G, c / G - thi), 0.0)
+        out.append(int(((gap ** 2).sum(1) <= r * r).sum()))
+    return np.array(out)
+
+
+@pytest.mark.parametrize("room", ["all", "exact", "few_more", "too_few"])
+def test_cells_that_overflow_both_passes(head_avatar, room):
+    """A coarse grid, most of whose cells have more candidates than either per-cell pass holds: what the first
+    pass leaves over and what the second does together exceed the cells' capacity where that is the occupied
+    cells' number or little more.  Ids and distances against brute force, also after the slot got another
+    expression (the heads of a cell that is left out would be the first one's)."""
+    torch = _torch()
+    from insta_amd.capi import Context
+    ensure_oracle()
+    G, S, thr = 16, 4, 0.3
+    from oracle.oracle import Oracle
+    orc = Oracle(full_config(max_frames=1, grid_size=G, cell_split=0))
+    orc.set_canonical_mesh(head_avatar.canonical, head_avatar.faces, head_avatar.masks)
+    frames = []
+    for k in (0, 1):
+        orc.set_frame(0, head_avatar.frames[k])
+        frames.append(_occupied_cells(orc.build_occupancy(0, thr)))
+    occupied = max(len(c) for c in frames)
+    cap = {"all": G ** 3, "exact": occupied, "few_more": occupied + 50, "too_few": occupied // 2}[room]
+    cfg = full_config(max_frames=1, grid_size=G, cell_split=S, cell_list_cells=cap, cell_list_entries=1 << 27)
+    ctx = Context(cfg)
+    ctx.set_canonical_mesh(head_avatar.canonical, head_avatar.faces, head_avatar.masks)
+    rng = np.random.default_rng(11)
+    for k in (0, 1):
+        orc.set_frame(0, head_avatar.frames[k])
+        cells = frames[k]
+        least = _least_candidates(orc, head_avatar.frames[k], head_avatar.faces, cells, G, S)
+        assert (least > 1024).sum() + (least > 3072).sum() > occupied + 50
+        ctx.set_frames(0, torch.from_numpy(head_avatar.frames[k][None]).cuda())
+        ctx.build_occupancy(0, thr)
+        info = ctx.cell_list_info(0)
+        assert info["occupied_cells"] == len(cells) and info["valid"] == (1 if len(cells) <= cap else 0), info
+        pts = _probe_points(cells, G, S, rng, 20000)
+        pts = pts[rng.choice(len(pts), 24000, replace=False)]
+        ids, dist = ctx.closest(0, torch.from_numpy(pts).cuda())
+        rid, rd2 = orc.closest_brute(0, pts)
+        assert np.array_equal(ids.cpu().numpy(), rid), k
+        assert np.array_equal(dist.cpu().numpy(), np.sqrt(rd2)), k
