@@ -236,7 +236,8 @@ insta_status insta_closest_triangles(insta_ctx* ctx, int32_t frame, const float*
                                      uint32_t n, int32_t* ids_dev, float* dist_dev, void* stream);
 
 /* Candidate lists of a frame (see insta_config.cell_split), as left by its
- * last insta_build_occupancy: occupied cells, entries used, whether the lists
+ * last insta_build_occupancy: occupied cells, entries that all lists would
+ * take (2^32 - 1 if more), whether the lists
  * answer queries (0 when cell_split is 0, before the first build, after the
  * frame's mesh changed, or when the occupied cells exceeded cell_list_cells),
  * and sub-cells that fell back to the BVH because cell_list_entries ran out.

@@ -129,6 +129,14 @@ struct ClArgs {
     uint32_t G, S, cap, ent_cap;
 };
 
+// First of n list entries.  Lists too long to keep claim theirs too, so that
+// the total tells what capacity would hold all; over a large, densely occupied
+// grid it passes 2^32 (256^3 sub-cells around a 16,000-triangle mesh: above 6e9), and
+// a 32-bit count would hand out the first entries again.
+INSTA_DEV uint64_t claim_entries(uint32_t* state, uint32_t n) {
+    return atomicAdd(reinterpret_cast<unsigned long long*>(state + kClClaim), (unsigned long long)n);
+}
+
 // sub-cell `sub` of occupied cell `cell`, grown by kCellEps
 INSTA_DEV void sub_box(const ClArgs& a, uint32_t cell, uint32_t sub, float4& lo, float4& hi) {
     const uint32_t cx = cell % a.G, cy = (cell / a.G) % a.G, cz = cell / (a.G * a.G);
@@ -251,7 +259,8 @@ __global__ __launch_bounds__(kSecond ? kCellThreads2 : kCellThreads) void cl_cel
     constexpr uint32_t kCand = kSecond ? kCellCand2 : kCellCand;  // candidates, and tree nodes of a level
     __shared__ uint16_t s_node[2][kCand], s_tri[kCand];
     __shared__ float s_lo[kCand][3], s_hi[kCand][3];
-    __shared__ uint32_t s_n[2], s_cand, s_base;
+    __shared__ uint32_t s_n[2], s_cand;
+    __shared__ uint64_t s_base;
     __shared__ uint32_t s_u[kThreads], s_v[kThreads], s_w[kThreads];
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
     const uint32_t S3 = a.S * a.S * a.S, shares = kThreads / S3;
@@ -441,14 +450,14 @@ __global__ __launch_bounds__(kSecond ? kCellThreads2 : kCellThreads) void cl_cel
                 const uint32_t up = __shfl_up(incl, o);
                 if (lane >= o) incl += up;
             }
-            if (lane == 63u) s_base = atomicAdd(&a.state[1], incl);
+            if (lane == 63u) s_base = claim_entries(a.state, incl);
             if (lane < S3) s_w[lane] = incl - c;
         }
         __syncthreads();
-        const uint32_t off = s_base + s_w[sub];
+        const uint64_t off = s_base + s_w[sub];
         uint2 hd = make_uint2(0u, kNoList);
-        if (found && count <= kMaxList && (uint64_t)off + count <= a.ent_cap)
-            hd = make_uint2(off, count | (seed << 16));
+        if (found && count <= kMaxList && off + count <= a.ent_cap)
+            hd = make_uint2((uint32_t)off, count | (seed << 16));
         if (share == 0) {
             a.head[(size_t)rank * S3 + sub] = hd;
             if (hd.y == kNoList) atomicAdd(&a.state[4], 1u);
@@ -490,9 +499,9 @@ __global__ __launch_bounds__(kClThreads) void cl_count_kernel(ClArgs a) {
             uint32_t count = 1;  // the seed, then every other triangle of the walk
             bvh_range(a.m, lo, hi, U2, stack + threadIdx.x, kClThreads,
                       [&](uint32_t t, float) { count += t != seed ? 1u : 0u; });
-            const uint32_t off = atomicAdd(&a.state[1], count);
-            if (count <= kMaxList && (uint64_t)off + count <= a.ent_cap)
-                hd = make_uint2(off, count | ((uint32_t)h.idx << 16));
+            const uint64_t off = claim_entries(a.state, count);
+            if (count <= kMaxList && off + count <= a.ent_cap)
+                hd = make_uint2((uint32_t)off, count | ((uint32_t)h.idx << 16));
         }
         if (hd.y == kNoList) atomicAdd(&a.state[4], 1u);
         a.head[(size_t)rank * S3 + i % S3] = hd;
@@ -580,7 +589,9 @@ __global__ __launch_bounds__(kClThreads) void cl_sort_kernel(ClArgs a) {
 }
 
 __global__ void cl_finish_kernel(uint32_t* __restrict__ state) {
-    if (threadIdx.x == 0) state[2] = state[3] == 0u ? 1u : 0u;
+    if (threadIdx.x != 0) return;
+    state[1] = state[kClClaim + 1] ? 0xffffffffu : state[kClClaim];
+    state[2] = state[3] == 0u ? 1u : 0u;
 }
 
 ClArgs cl_args(insta_ctx* ctx, uint32_t slot) {

@@ -318,10 +318,11 @@ INSTA_DEV Hit bvh_closest(const MeshView& m, V3 p, uint32_t* stack, uint32_t str
 //          rest ascending
 //   state  [kClState] occupied cells, entries used, valid (1: lists answer
 //          queries), occupied cells beyond the cap, sub-cells without a list,
-//          (build) cells left by the first and the second pass over the cells
+//          (build) cells left by the first and the second pass over the cells,
+//          at kClClaim the entries claimed, as 64 bits
 // ---------------------------------------------------------------------------
 constexpr uint32_t kNoList = 0xffffffffu;
-constexpr uint32_t kClState = 8;
+constexpr uint32_t kClState = 16, kClClaim = 8;
 constexpr float kCellEps = 1e-5f;
 
 struct CellListView {

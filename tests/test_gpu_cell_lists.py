@@ -259,3 +259,32 @@ def test_cells_that_overflow_both_passes(head_avatar, room):
         rid, rd2 = orc.closest_brute(0, pts)
         assert np.array_equal(ids.cpu().numpy(), rid), k
         assert np.array_equal(dist.cpu().numpy(), np.sqrt(rd2)), k
+
+
+def test_more_entries_than_32_bits_count():
+    """A 64^3 grid occupied almost everywhere around a mesh of 16,185 triangles: the lists of its sub-cells take
+    more than 2^32 entries, of which the first 2^25 are kept.  Ids and distances against brute force."""
+    torch = _torch()
+    from insta_amd.capi import Context
+    ensure_oracle()
+    from oracle.oracle import Oracle
+    verts, faces = synth.head_ellipsoid(129, 63)
+    verts = (0.1 * verts + 0.5).astype(np.float32)
+    masks = np.ones(len(faces), np.uint32)
+    G, thr = 64, 2.0
+    cfg = full_config(max_frames=1, grid_size=G, cell_split=4, cell_list_cells=G ** 3)
+    ctx, orc = Context(cfg), Oracle(cfg)
+    for s in (ctx, orc):
+        s.set_canonical_mesh(verts, faces, masks)
+    ctx.set_frames(0, torch.from_numpy(verts[None]).cuda())
+    orc.set_frame(0, verts)
+    cells = _occupied_cells(ctx.build_occupancy(0, thr).cpu().numpy())
+    info = ctx.cell_list_info(0)
+    assert info["valid"] == 1 and info["entries"] == 0xFFFFFFFF, info
+    assert 0 < info["subcells_without_list"] < 64 * len(cells), info
+    pts = _probe_points(cells, G, 4, np.random.default_rng(12), 20000)
+    pts = pts[np.random.default_rng(13).choice(len(pts), 24000, replace=False)]
+    ids, dist = ctx.closest(0, torch.from_numpy(pts).cuda())
+    rid, rd2 = orc.closest_brute(0, pts)
+    assert np.array_equal(ids.cpu().numpy(), rid)
+    assert np.array_equal(dist.cpu().numpy(), np.sqrt(rd2))
