@@ -492,6 +492,14 @@ INSTA_DEV uint32_t group_ballot(bool b) {
     return (uint32_t)(w >> (threadIdx.x & 63u & ~(kGroup - 1u))) & ((1u << kGroup) - 1u);
 }
 
+// LDS words that one lane of a wave writes and others read (or the reverse):
+// a wave's LDS accesses complete in order, so this only keeps the compiler
+// from moving them past each other
+INSTA_DEV void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 struct GroupBest {
     uint32_t dist = 0x7f7fffffu;    // bits of the squared distance (starts at the largest float)
     uint32_t key = 0xffffffffu;     // original id << 16 | BVH-order index (both < 2^14)
@@ -577,7 +585,9 @@ INSTA_DEV Hit group_bvh_closest(const MeshView& m, V3 p, uint32_t* stack) {
             rank += o3 < bits || (o3 == bits && (c ^ 3u) < c) ? 1u : 0u;
             const uint32_t n_live = (uint32_t)__popc(group_ballot(live));
             const uint32_t nearest = group_ballot(live && rank == 0u);
+            wave_lds_order();  // (every lane has popped what these replace)
             if (live && rank) stack[sp + n_live - 1u - rank] = (bits & 0xffff0000u) | (first + c);
+            wave_lds_order();
             if (nearest) {
                 sp += n_live - 1u;
                 node = first + (uint32_t)__builtin_ctz(nearest);
