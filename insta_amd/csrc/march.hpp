@@ -4,6 +4,8 @@
 // random_val.cuh:159-288).
 #pragma once
 
+#include <cmath>
+
 #include "context.hpp"
 
 namespace insta {
@@ -59,14 +61,19 @@ INSTA_DEV bool occupied(const uint8_t* __restrict__ grid, uint32_t G, V3 pos) {
     return (grid[idx >> 3] >> (idx & 7u)) & 1u;
 }
 
-INSTA_DEV float advance_to_next_voxel(float t, float dt, V3 pos, V3 dir, V3 idir, uint32_t res) {
+// where a ray at t leaves the voxel of pos
+INSTA_DEV float next_voxel(float t, V3 pos, V3 dir, V3 idir, uint32_t res) {
     const float r = (float)res;
     const V3 p = v3(r * pos.x, r * pos.y, r * pos.z);
     const float tx = (floorf(p.x + 0.5f + 0.5f * signf(dir.x)) - p.x) * idir.x;
     const float ty = (floorf(p.y + 0.5f + 0.5f * signf(dir.y)) - p.y) * idir.y;
     const float tz = (floorf(p.z + 0.5f + 0.5f * signf(dir.z)) - p.z) * idir.z;
     const float tn = fminf(fminf(tx, ty), tz);
-    const float t_target = t + fmaxf(tn / r, 0.0f);
+    return t + fmaxf(tn / r, 0.0f);
+}
+
+INSTA_DEV float advance_to_next_voxel(float t, float dt, V3 pos, V3 dir, V3 idir, uint32_t res) {
+    const float t_target = next_voxel(t, pos, dir, idir, res);
     do {
         t += dt;
     } while (t < t_target);
@@ -102,9 +109,51 @@ struct Ahead {
     }
 };
 
+// Far cameras, some 10^5 away: a step may be below the last bit of t somewhere
+// in the box, where advance_to_next_voxel would never end (and the walks form
+// it ahead also for a ray all of whose cells are occupied).  The host tells
+// (far_camera) and launches kernels of their own, so that the others' stay as
+// they are (64 x 64 frame of the small sphere 370 us; with the test in every
+// step, or once per ray, 385 us).
+inline bool far_camera(const float origin[3], float dt) {
+    // no ray's t in the box is larger: the box lies within [0, 1]^3, voxels end within one of it
+    const float end = std::fabs(origin[0]) + std::fabs(origin[1]) + std::fabs(origin[2]) + 8.0f;
+    return !(end + 0.5f * dt > end);
+}
+
+// The walk of a far ray, a position at a time (walk_samples; with no samples
+// wanted, `most` 0, skip_empty).  One that stands still in an empty cell ends
+// there, exited.
+template <class Sample>
+INSTA_DEV uint32_t walk_far(const RenderArgs& a, V3 o, V3 d, V3 idir, float& t, uint32_t most, bool& exited,
+                            Sample&& sample) {
+    uint32_t count = 0;
+    exited = false;
+    do {
+        const V3 pos = o + d * t;
+        const bool occ = occupied(a.grid, a.G, pos);
+        exited = !box_contains(a, pos);
+        if (exited || (occ && most == 0)) break;
+        const float target = occ ? t : next_voxel(t, pos, d, idir, a.G);
+        if (occ) sample(count++, t);
+        do {
+            const float next = t + a.dt;
+            exited = !occ && !(next > t);
+            t = next;
+        } while (!exited && t < target);
+    } while (!exited && (most == 0 || count < most));
+    return count;
+}
+
 // Walk from t to the next occupied position inside the box.  Returns false
 // if the ray leaves the box first.
+template <bool kFar>
 INSTA_DEV bool skip_empty(const RenderArgs& a, V3 o, V3 d, V3 idir, float& t) {
+    if constexpr (kFar) {
+        bool exited;
+        walk_far(a, o, d, idir, t, 0u, exited, [](uint32_t, float) {});
+        return !exited;
+    }
     while (true) {
         const Ahead w(a, o, d, idir, t, false);
 #pragma unroll
@@ -119,12 +168,13 @@ INSTA_DEV bool skip_empty(const RenderArgs& a, V3 o, V3 d, V3 idir, float& t) {
 
 // Up to `most` samples from t: sample(j, t) for each, in order; t ends at the
 // next unvisited position.  exited: the ray left the box.
-template <class Sample>
+template <bool kFar, class Sample>
 INSTA_DEV uint32_t walk_samples(const RenderArgs& a, V3 o, V3 d, V3 idir, float& t, uint32_t most, bool& exited,
                                 Sample&& sample) {
+    exited = false;
+    if constexpr (kFar) return most ? walk_far(a, o, d, idir, t, most, exited, sample) : 0u;
     uint32_t count = 0;
     bool through = true;  // the last position seen was occupied
-    exited = false;
     while (count < most && !exited) {
         const Ahead w(a, o, d, idir, t, through);
         bool go = true;

@@ -82,6 +82,7 @@ INSTA_HD uint32_t tiled_threads(uint32_t w, uint32_t h) {
     return ((w + kTile - 1) / kTile) * ((h + kTile - 1) / kTile) * kTile * kTile;
 }
 
+template <bool kFar>
 __global__ __launch_bounds__(kInitThreads) void init_rays_kernel(RenderArgs a, float4* __restrict__ r_o,
                                                                 float4* __restrict__ r_d, float4* __restrict__ r_rgba,
                                                                 float* __restrict__ r_depth,
@@ -109,7 +110,7 @@ __global__ __launch_bounds__(kInitThreads) void init_rays_kernel(RenderArgs a, f
         if (box_contains(a, o + d * t)) {
             const V3 idir = v3(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
             t += ld_random_val0(a.spp, i * 786433u) * a.dt;  // advance_pos_nerf (testbed_nerf.cu:663-664)
-            live = skip_empty(a, o, d, idir, t);
+            live = skip_empty<kFar>(a, o, d, idir, t);
         }
         r_o[i] = make_float4(o.x, o.y, o.z, t);
         r_d[i] = make_float4(d.x, d.y, d.z, 0.0f);
@@ -127,6 +128,7 @@ __global__ __launch_bounds__(kInitThreads) void init_rays_kernel(RenderArgs a, f
 // sample buffer), then the wave reserves contiguous output space and each
 // lane writes its samples from the stored t values (pos = o + d t exactly as
 // during the walk).
+template <bool kFar>
 __global__ __launch_bounds__(kRayThreads) void march_kernel(RenderArgs a, const uint32_t* __restrict__ alive,
                                                             const uint32_t* __restrict__ n_alive_dev,
                                                             uint64_t sample_cap, float4* __restrict__ r_o,
@@ -160,8 +162,8 @@ __global__ __launch_bounds__(kRayThreads) void march_kernel(RenderArgs a, const 
         const uint32_t done = r_steps[r];
         const uint32_t budget = a.max_steps > done ? a.max_steps - done : 0u;
         const uint32_t kmax = K < budget ? K : budget;
-        count = walk_samples(a, o, d, idir, t, kmax, exited,
-                             [&](uint32_t j, float tj) { t_buf[(size_t)j * n_alive + k] = tj; });
+        count = walk_samples<kFar>(a, o, d, idir, t, kmax, exited,
+                                   [&](uint32_t j, float tj) { t_buf[(size_t)j * n_alive + k] = tj; });
     }
     // the wave's samples are one contiguous range, written step-major
     const uint32_t wave_base = __shfl(block_reserve<kRayWaves>(&counters[kCntSamples], count), 0);
@@ -623,6 +625,11 @@ RenderArgs render_args(const insta_ctx* ctx, const insta_camera* cam, uint32_t w
     return a;
 }
 
+bool far_frame(const RenderArgs& a) {
+    const float origin[3] = {a.M[3], a.M[7], a.M[11]};
+    return far_camera(origin, a.dt);
+}
+
 // One march/deform/network/composite round over live list `cur`, with the
 // live count read on the device.  `max_alive` bounds the live count (it
 // sizes the ray grids).
@@ -636,7 +643,8 @@ insta_status enqueue_round(insta_ctx* ctx, RenderWS& ws, const RenderArgs& a, in
                        window);
     const dim3 rgrid((max_alive + kRayThreads - 1) / kRayThreads);
     prof_begin(ctx, prof, INSTA_KERNEL_MARCH, stream);
-    hipLaunchKernelGGL(march_kernel, rgrid, dim3(kRayThreads), 0, stream, a, ws.alive[cur], cnt + cur_slot,
+    hipLaunchKernelGGL(far_frame(a) ? march_kernel<true> : march_kernel<false>, rgrid, dim3(kRayThreads), 0, stream, a,
+                       ws.alive[cur], cnt + cur_slot,
                        (uint64_t)ws.samples, ws.r_o, ws.r_d, ws.r_steps, ws.r_flags, ws.r_off, ws.r_cnt,
                        reinterpret_cast<float*>(ws.s_hit), ws.s_pos, cnt);
     INSTA_HIP(hipGetLastError());
@@ -694,8 +702,9 @@ insta_status enqueue_render(insta_ctx* ctx, RenderWS& ws, const insta_camera* ca
     uint32_t* cnt = ws.d_counters;
     hipLaunchKernelGGL(clear_counters_kernel, dim3(1), dim3(64), 0, stream, cnt, 0u, (uint32_t)kNumCounters);
     prof_begin(ctx, prof, INSTA_KERNEL_INIT, stream);
-    hipLaunchKernelGGL(init_rays_kernel, dim3((tiled_threads(width, height) + kInitThreads - 1) / kInitThreads),
-                       dim3(kInitThreads), 0, stream, a,
+    hipLaunchKernelGGL(far_frame(a) ? init_rays_kernel<true> : init_rays_kernel<false>,
+                       dim3((tiled_threads(width, height) + kInitThreads - 1) / kInitThreads), dim3(kInitThreads), 0,
+                       stream, a,
                        ws.r_o, ws.r_d, ws.r_rgba, ws.r_depth, ws.r_steps, ws.alive[0], cnt);
     INSTA_HIP(hipGetLastError());
     prof_end(ctx, prof, INSTA_KERNEL_INIT, n_pix, stream);

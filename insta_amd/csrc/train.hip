@@ -133,6 +133,7 @@ constexpr uint32_t kXcds = 8;
 
 struct TrainState {
     uint32_t n_images = 0, width = 0, height = 0;
+    bool far = false;              // an image's camera is far_camera
     float4* images = nullptr;
     TrainImage* meta = nullptr;
     // supervision of the training set (nullptr: none): mask id and
@@ -248,6 +249,7 @@ INSTA_DEV bool train_ray(const RayArgs& a, uint32_t i, uint32_t n_rays, uint64_t
     return true;
 }
 
+template <bool kFar>
 __global__ __launch_bounds__(kRayThreads) void train_rays_kernel(RayArgs a, uint32_t n_rays, uint64_t rays_total,
                                                          Pcg32 rng, float4* __restrict__ ray_d,
                                                          float4* __restrict__ ray_o,
@@ -270,8 +272,8 @@ __global__ __launch_bounds__(kRayThreads) void train_rays_kernel(RayArgs a, uint
         idir = v3(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
         // sample t values to step-major scratch (t_buf[j * n_rays + i])
         bool exited;
-        count = walk_samples(ra, o, d, idir, t0, a.box.max_steps, exited,
-                             [&](uint32_t j, float tj) { t_buf[(size_t)j * n_rays + i] = tj; });
+        count = walk_samples<kFar>(ra, o, d, idir, t0, a.box.max_steps, exited,
+                                   [&](uint32_t j, float tj) { t_buf[(size_t)j * n_rays + i] = tj; });
     }
     const uint32_t base = block_reserve<kRayWaves>(&counters[kTSamples], count);
     const bool fits = base + count <= a.max_samples;
@@ -1967,6 +1969,7 @@ insta_status set_training_set(insta_ctx* ctx, uint32_t n_images, uint32_t width,
         return INSTA_ERR_OOM;
     }
     std::vector<TrainImage> meta(n_images);
+    bool far = false;
     for (uint32_t i = 0; i < n_images; ++i) {
         TrainImage& m = meta[i];
         for (int k = 0; k < 12; ++k) m.M[k] = cams[i].matrix[k];
@@ -1976,12 +1979,15 @@ insta_status set_training_set(insta_ctx* ctx, uint32_t n_images, uint32_t width,
         m.cy = cams[i].screen_center[1];
         m.frame = frames[i];
         m.pad[0] = m.pad[1] = m.pad[2] = 0;
+        const float origin[3] = {m.M[3], m.M[7], m.M[11]};
+        far |= far_camera(origin, ctx->cfg.dt);
     }
     INSTA_HIP(hipMemcpyAsync(ts->images, rgba, px * sizeof(float4), hipMemcpyDeviceToDevice, stream));
     INSTA_HIP(hipMemcpyAsync(ts->meta, meta.data(), n_images * sizeof(TrainImage), hipMemcpyHostToDevice, stream));
     INSTA_HIP(hipStreamSynchronize(stream));  // `meta` is pageable host memory
     ts->frames.assign(frames, frames + n_images);
     ts->n_images = n_images;
+    ts->far = far;
     ts->width = width;
     ts->height = height;
     ts->rays_total = 0;
@@ -2042,8 +2048,8 @@ insta_status train_step(insta_ctx* ctx, const insta_train_config& tc, insta_trai
     ra.height = ts->height;
     ra.max_samples = cap;
     ra.fixed_slot = tc.occupancy_slot;
-    hipLaunchKernelGGL(train_rays_kernel, dim3((n_rays + kRayThreads - 1) / kRayThreads), dim3(kRayThreads), 0, stream,
-                       ra, n_rays, ts->rays_total, rng, ts->ray_d, ts->ray_o, ts->ray_frame, ts->ray_img, ts->ray_pix, ts->ray_src, ts->ray_base,
+    hipLaunchKernelGGL(ts->far ? train_rays_kernel<true> : train_rays_kernel<false>,
+                       dim3((n_rays + kRayThreads - 1) / kRayThreads), dim3(kRayThreads), 0, stream, ra, n_rays, ts->rays_total, rng, ts->ray_d, ts->ray_o, ts->ray_frame, ts->ray_img, ts->ray_pix, ts->ray_src, ts->ray_base,
                        ts->ray_cnt, ts->t_buf, ts->ray_T, ts->ray_alive, ts->counters);
     INSTA_HIP(hipGetLastError());
     hipLaunchKernelGGL(train_count_kernel, dim3(1), dim3(64), 0, stream, ts->counters);
