@@ -269,11 +269,25 @@ struct XcdTiles {
 // four column blocks of 16 a wave; or a quarter, a quarter of the levels and
 // one column block a wave, which brings a quarter of the latency where the
 // samples fill few CUs.
-// The line is 131,072 samples: network rounds of a training step of 8,192 rays
-// 204 us with whole tiles, 175 us; above it the whole tiles win (BF16
-// inference of 1,048,576 positions 362 us, with quarter tiles 435 us; FP32
-// render at 512 x 512 1,262 / 1,316 us).
-constexpr uint32_t kSmallTileMax = 256u * 512u;
+// Whole tiles take rounds of 65,536 samples (a workgroup on each of the 256
+// CUs), a round of them the same time however few it has, so quarter tiles take
+// the calls that would end in a short round: up to kFirstRound samples, and up
+// to kSecondRound beyond one round; the BF16 / FP16 kernel, whose whole tiles
+// overlap better, a shorter second.  us, quarter / whole tiles:
+//                20,000   40,000   50,000   65,536   73,000   81,920   98,304  114,688
+//   head FP32  41 /  59  52 / 59  63 / 60  65 / 63  73 / 88  75 / 89  86 / 91  97 / 91
+//   small FP32 29 /  38  36 / 38  41 / 39  43 / 40  47 / 53  48 / 54  54 / 56  59 / 57
+//   head FP16  33 /  46  40 / 44  48 / 44  49 / 46  55 / 63  57 / 65  64 / 67  72 / 67
+//   small FP16 24 /  27  27 / 26  29 / 27  30 / 28  32 / 32  33 / 33  36 / 34  39 / 35
+// (whole tiles at 20,000: as they were before there were quarter tiles.)
+// Beyond two rounds whole tiles win throughout (BF16 inference of 1,048,576
+// positions 362 us, with quarter tiles 435; FP32 render at 512 x 512 1,262 /
+// 1,316 us).
+constexpr uint32_t kRoundSamples = 256u * kTile;
+constexpr uint32_t kFirstRound = 40960u, kSecondRoundF32 = 40960u, kSecondRoundX32 = 16384u;
+INSTA_DEV bool quarter_tiles(uint32_t n, uint32_t second) {
+    return n <= kFirstRound || (n > kRoundSamples && n <= kRoundSamples + second);
+}
 
 template <int L, int X, int NB, class Src>
 INSTA_DEV void f32_tiles(float* s_x, const float* __restrict__ table, const GridParams& gp,
@@ -391,7 +405,7 @@ __global__ __launch_bounds__(256) void network_f32_kernel(const float* __restric
                                                           Src src) {
     __shared__ float s_x[kTile * kF32Stride];
     const uint32_t n = src.count();
-    if (n <= kSmallTileMax) f32_tiles<L, X, 1>(s_x, table, gp, frag, xbias, xrows, n, src);
+    if (quarter_tiles(n, kSecondRoundF32)) f32_tiles<L, X, 1>(s_x, table, gp, frag, xbias, xrows, n, src);
     else f32_tiles<L, X, 4>(s_x, table, gp, frag, xbias, xrows, n, src);
 }
 
@@ -532,7 +546,7 @@ __global__ __launch_bounds__(256, 4) void network_x32_kernel(const _Float16* __r
 #pragma unroll
     for (uint32_t f = 0; f < kFragX32; ++f) A[f] = *reinterpret_cast<const V8*>(frag + ((size_t)f * 64 + lane) * 8);
     const uint32_t n = src.count();
-    if (n <= kSmallTileMax) x32_tiles<L, X, 1>(s_x, A, table, gp, xbias, xrows, n, src);
+    if (quarter_tiles(n, kSecondRoundX32)) x32_tiles<L, X, 1>(s_x, A, table, gp, xbias, xrows, n, src);
     else x32_tiles<L, X, 4>(s_x, A, table, gp, xbias, xrows, n, src);
 }
 

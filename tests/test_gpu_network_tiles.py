@@ -1,7 +1,8 @@
-"""The matrix-core network takes up to 2^17 samples in tiles of 64 and more in
-tiles of 256: an output depends on its own sample alone, so a call of any size
+"""The matrix-core network takes calls that would end in a short round of
+256-sample tiles on the CUs (up to 40,960 samples, and some beyond 65,536) in
+tiles of 64: an output depends on its own sample alone, so a call of any size
 returns, bit for bit, what the same samples return within a larger call.  Sizes
-at the edges of both tiles and on both sides of the line, with positions inside
+at the edges of both tiles and on both sides of the lines, with positions inside
 and outside the unit cube (where dense levels wrap)."""
 import numpy as np
 import pytest
@@ -31,5 +32,6 @@ def test_outputs_do_not_depend_on_the_tile(config, precision):
     c = torch.from_numpy(c).cuda()
     whole = ctx.network_inference(c)
     assert torch.isfinite(whole).all()
-    for n in (1, 15, 17, 63, 64, 65, 255, 257, 4097, 1 << 17):
+    for n in (1, 15, 17, 63, 64, 65, 255, 257, 4097, 40960, 40961, 1 << 16, (1 << 16) + 1, 81920, 81921, 106496, 106497,
+              1 << 17):
         assert torch.equal(ctx.network_inference(c[:n].contiguous()), whole[:n]), n
