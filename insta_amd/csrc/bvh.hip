@@ -394,10 +394,13 @@ __global__ void blend_expression_kernel(const float* __restrict__ canon, const f
 }
 
 constexpr uint32_t kQueryThreads = 256;
-// Points of one call go to groups of lanes up to here: on the 9,976-triangle
-// head 1,000 / 200,000 / 1,000,000 points anywhere in the unit cube take 165 /
-// 582 / 2,093 us in groups and 670 / 956 / 2,234 us one lane each; 3,000,000
-// take 5,610 and 4,949 us.
+// Points of one call go to groups of lanes up to here.  us on the 9,976-triangle
+// head, groups / one lane each, for random points anywhere in the unit cube and
+// (in brackets) near the skin, from its candidate lists:
+//   1,000  196 / 714 (47 / 138)     200,000  878 / 1,214 (124 / 265)
+//   700,000  2,720 / 2,690 (237 / 441)     1,048,576  4,000 / 3,610 (316 / 546)
+// The far points alone would set the line at 700,000; above it they lose up to a
+// tenth, and the near ones, which gain two fifths, decide.
 constexpr uint32_t kGroupedPoints = 1u << 20;
 
 // nearest triangle per point, one group of lanes per point: the frame's

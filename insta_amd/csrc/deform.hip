@@ -15,12 +15,15 @@ namespace insta {
 namespace {
 
 constexpr uint32_t kDeformThreads = 256;
-// Coordinates of one call go to groups of lanes up to here: 200,000 random
-// points near a skin take 121 us in groups and 252 us one lane each (the
-// 9,976-triangle head; 89 and 101 us, the 2,048-triangle sphere), 1,000,000
-// take 432 and 477 us (352 and 270 us): beyond, the chip is full either way
-// and the groups' idle lanes cost more on the smaller mesh.
-constexpr uint32_t kGroupedCoords = 1u << 18;
+// Coordinates of one call go to groups of lanes up to a line that depends on
+// the mesh: beyond it the chip is full either way, and the groups' idle lanes
+// cost more the fewer triangles a query meets.  us for random points near a
+// skin, groups / one lane each, with candidate lists and (in brackets) without:
+//                             131,072              200,000              262,144
+//   9,976-triangle head   125 / 226 (173 / 264)  151 / 290 (229 / 309)  175 / 301 (271 / 325)
+//   2,048-triangle sphere  80 /  93 (102 /  98)  100 / 104 (133 / 125)  120 / 116 (162 / 129)
+constexpr uint32_t kGroupedCoords = 1u << 18, kGroupedCoordsFew = 1u << 17;
+constexpr uint32_t kFewTriangles = 4096;
 
 struct MeshSet {
     const float4* nodes;
@@ -473,7 +476,7 @@ insta_status launch_deform_aos(insta_ctx* ctx, float* coords, uint32_t n, uint32
     if (n == 0) return INSTA_OK;
     const size_t shmem = (size_t)stack_depth(ctx->bvh_k) * kDeformThreads * sizeof(uint32_t);
     const MeshSet ms = mesh_set(ctx, ctx->d_built);
-    if (n <= kGroupedCoords)
+    if (n <= (ctx->nf <= kFewTriangles ? kGroupedCoordsFew : kGroupedCoords))
         hipLaunchKernelGGL(deform_aos_kernel<true>, dim3((n * kGroup + kDeformThreads - 1) / kDeformThreads),
                            dim3(kDeformThreads), shmem / kGroup, stream, ms, coords, n, stride, frame,
                            ctx->cfg.n_extra_dims, ctx->d_misses);

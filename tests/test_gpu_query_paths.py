@@ -111,3 +111,25 @@ def test_second_pass_equals_unbudgeted_queries(scenes, split):
     got = ctx.render(cam, 203, 200, 0, 0)
     for g, r in zip(got, ref):
         assert np.array_equal(g.cpu().numpy(), r.cpu().numpy())
+
+
+@pytest.mark.parametrize("n", [1 << 17, (1 << 17) + 1])
+def test_coords_on_a_small_mesh(n):
+    """The line lies lower for meshes of few triangles: both sides of it against calls far below it."""
+    import torch
+    from insta_amd.capi import Context, small_config
+    av = synth.small_sphere_avatar(seed=0, n_frames=N_FRAMES)
+    ctx = Context(small_config(max_frames=N_FRAMES, cell_split=0))
+    ctx.set_canonical_mesh(av.canonical, av.faces, av.masks)
+    ctx.set_frames(0, torch.from_numpy(np.stack(av.frames)).cuda())
+    c = np.zeros((n, 11), np.float32)
+    c[:, 0:3] = _points(av, n, 8)
+    c[:, 4] = np.arange(n) % N_FRAMES
+    c[:, 8:11] = np.random.default_rng(9).uniform(0.2, 0.8, (n, 3))
+    whole, part = torch.from_numpy(c).cuda(), torch.from_numpy(c).cuda()
+    ctx.deform_samples(whole)
+    for s in (slice(0, 40000), slice(40000, 80000), slice(80000, n)):
+        p = part[s].contiguous()
+        ctx.deform_samples(p)
+        part[s] = p
+    assert torch.equal(whole, part)
