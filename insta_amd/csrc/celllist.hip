@@ -20,7 +20,7 @@
 //             (nearest triangle at the centre), bound U^2 (from the 8
 //             corners), count and entries from those; it claims its entries
 //             with one atomic (layout order varies, contents do not)
-//   5. count, fill: (other splits, and cells whose candidates overflow LDS)
+//   5. count, fill: (other splits, and cells with too many candidates for LDS)
 //             one lane per sub-cell: nearest triangle at the centre
 //             (BVH), the bound U^2 from the 8 corners, a bounded BVH range walk
 //             counting the triangles whose box is within U; the same walk
@@ -119,9 +119,9 @@ __global__ void cl_cells_kernel(const uint64_t* __restrict__ bits, const uint32_
 struct ClArgs {
     MeshView m;
     const uint32_t* cells;
-    uint32_t* left;       // [2][cap] ranks of the cells cl_cell_kernel left over: by its first launch
-                          // (state[5] of them), and in words of their own, since the second launch
-                          // reads those while it writes these, by its second (state[6])
+    uint32_t* left;       // [cap] ranks of the cells cl_cell_kernel's first launch left to its second
+                          // (state[5] of them)
+    uint32_t* walk;       // [cap] by rank: 1 where it left the cell to the per-lane kernels
     uint32_t all;         // the per-lane kernels take every cell
     uint2* head;
     uint32_t* ent;
@@ -238,7 +238,8 @@ INSTA_DEV void bvh_range(const MeshView& m, float4 lo, float4 hi, float U2, uint
 // cells (17 M entries) take 382 + 86 us (second launch); one lane per sub-cell,
 // counting and filling walks, 1,029 + 444 us.
 // A second launch (kSecond) takes the cells with more than kCellCand candidates
-// with larger workgroups and lists.
+// with larger workgroups and lists, up to kCellCand2 of them; cells with more go
+// to the per-lane kernels.
 constexpr uint32_t kCellThreads = 256, kCellCand = 1024;
 constexpr uint32_t kCellThreads2 = 1024, kCellCand2 = 3072;
 
@@ -376,16 +377,16 @@ __global__ __launch_bounds__(kSecond ? kCellThreads2 : kCellThreads) void cl_cel
             __syncthreads();
             overflow = s_cand > kCand || s_cand == 0u;
         }
-        if (overflow) {  // left to the second launch, then to the per-lane kernels
+        if (overflow) {  // left to the second launch, or (too many for it as well) to the per-lane kernels
             if (tid == 0) {
-                if (kSecond)
-                    a.left[(size_t)a.cap + atomicAdd(&a.state[6], 1u)] = rank;
-                else
-                    a.left[atomicAdd(&a.state[5], 1u)] = rank;
+                const bool walk = kSecond || s_cand > kCellCand2;  // (s_cand: all of them where the tree's levels fit)
+                a.walk[rank] = walk ? 1u : 0u;
+                if (!walk) a.left[atomicAdd(&a.state[5], 1u)] = rank;
             }
             __syncthreads();
             continue;
         }
+        if (tid == 0) a.walk[rank] = 0u;
         const uint32_t n_cand = s_cand;
         // the seed: nearest to the sub-cell's centre (the order and prune margin of bvh_closest)
         const V3 ctr = v3((lo.x + hi.x) * 0.5f, (lo.y + hi.y) * 0.5f, (lo.z + hi.z) * 0.5f);
@@ -478,16 +479,21 @@ __global__ __launch_bounds__(kSecond ? kCellThreads2 : kCellThreads) void cl_cel
     }
 }
 
-// cells the per-lane kernels walk, and the i-th one's rank
-INSTA_DEV uint32_t walk_cells(const ClArgs& a) { return a.all ? min(a.state[0], a.cap) : a.state[6]; }
-INSTA_DEV uint32_t walk_rank(const ClArgs& a, uint32_t i) { return a.all ? i : a.left[(size_t)a.cap + i]; }
+// Whether the per-lane kernels walk the cell of this rank.  They visit the cells
+// in rank order and pass over the others: neighbouring waves then walk
+// neighbouring cells, whose nodes and triangles the CU's cache still holds (in
+// the order the cells were left in, a 32^3 grid of 1,109 cells took 7,700 us
+// to build, 7,080 in rank order; all cells one lane per sub-cell, 6,600: the
+// cells left here, of over 3,072 candidates, set the time either way).
+INSTA_DEV bool walked(const ClArgs& a, uint32_t rank) { return a.all || a.walk[rank]; }
 
 __global__ __launch_bounds__(kClThreads) void cl_count_kernel(ClArgs a) {
     extern __shared__ uint32_t stack[];  // [stack_depth(k)][kClThreads]
     const uint32_t S3 = a.S * a.S * a.S;
-    const uint32_t n_sub = walk_cells(a) * S3;
+    const uint32_t n_sub = min(a.state[0], a.cap) * S3;
     for (uint32_t i = blockIdx.x * kClThreads + threadIdx.x; i < n_sub; i += gridDim.x * kClThreads) {
-        const uint32_t rank = walk_rank(a, i / S3);
+        const uint32_t rank = i / S3;
+        if (!walked(a, rank)) continue;
         float4 lo, hi;
         sub_box(a, a.cells[rank], i % S3, lo, hi);
         const V3 ctr = v3((lo.x + hi.x) * 0.5f, (lo.y + hi.y) * 0.5f, (lo.z + hi.z) * 0.5f);
@@ -504,17 +510,18 @@ __global__ __launch_bounds__(kClThreads) void cl_count_kernel(ClArgs a) {
                 hd = make_uint2((uint32_t)off, count | ((uint32_t)h.idx << 16));
         }
         if (hd.y == kNoList) atomicAdd(&a.state[4], 1u);
-        a.head[(size_t)rank * S3 + i % S3] = hd;
+        a.head[i] = hd;
     }
 }
 
 __global__ __launch_bounds__(kClThreads) void cl_fill_kernel(ClArgs a) {
     extern __shared__ uint32_t stack[];  // [stack_depth(k)][kClThreads]
     const uint32_t S3 = a.S * a.S * a.S;
-    const uint32_t n_sub = walk_cells(a) * S3;
+    const uint32_t n_sub = min(a.state[0], a.cap) * S3;
     for (uint32_t i = blockIdx.x * kClThreads + threadIdx.x; i < n_sub; i += gridDim.x * kClThreads) {
-        const uint32_t rank = walk_rank(a, i / S3);
-        const uint2 hd = a.head[(size_t)rank * S3 + i % S3];
+        const uint32_t rank = i / S3;
+        if (!walked(a, rank)) continue;
+        const uint2 hd = a.head[i];
         if (hd.y == kNoList) continue;
         const uint32_t count = hd.y & 0xffffu, seed = hd.y >> 16;
         float4 lo, hi;
@@ -603,6 +610,7 @@ ClArgs cl_args(insta_ctx* ctx, uint32_t slot) {
     a.ent = ctx->d_cl_ent + slot * (size_t)ctx->cfg.cell_list_entries;
     a.state = ctx->d_cl_state + kClState * (size_t)slot;
     a.left = ctx->d_cl_left + 2 * slot * (size_t)ctx->cfg.cell_list_cells;
+    a.walk = a.left + ctx->cfg.cell_list_cells;
     // a workgroup per cell pays for 64 sub-cells, not for 8 or 1: the small
     // sphere at S = 2 takes 230 + 150 us one lane per sub-cell, 920 us so
     a.all = S == 4 ? 0u : 1u;
@@ -678,11 +686,10 @@ insta_status launch_cell_lists(insta_ctx* ctx, uint32_t slot, hipStream_t stream
                        ctx->d_cl_cells + slot * (size_t)ctx->cfg.cell_list_cells);
     const size_t shmem = (size_t)stack_depth(ctx->bvh_k) * kClThreads * sizeof(uint32_t);
     const uint64_t max_sub = (uint64_t)a.cap * a.S * a.S * a.S;
-    uint32_t blocks = (uint32_t)std::min<uint64_t>((max_sub + kClThreads - 1) / kClThreads, kClMaxBlocks);
+    const uint32_t blocks = (uint32_t)std::min<uint64_t>((max_sub + kClThreads - 1) / kClThreads, kClMaxBlocks);
     if (!a.all) {
         hipLaunchKernelGGL(cl_cell_kernel<false>, dim3(std::min(a.cap, kClMaxBlocks)), dim3(kCellThreads), 0, stream, a);
         hipLaunchKernelGGL(cl_cell_kernel<true>, dim3(std::min(a.cap, 512u)), dim3(kCellThreads2), 0, stream, a);
-        blocks = std::min(blocks, 256u);  // hardly any cell is left over
     }
     hipLaunchKernelGGL(cl_count_kernel, dim3(blocks), dim3(kClThreads), shmem, stream, a);
     hipLaunchKernelGGL(cl_fill_kernel, dim3(blocks), dim3(kClThreads), shmem, stream, a);

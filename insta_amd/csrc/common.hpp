@@ -318,8 +318,8 @@ INSTA_DEV Hit bvh_closest(const MeshView& m, V3 p, uint32_t* stack, uint32_t str
 //          rest ascending
 //   state  [kClState] occupied cells, entries used, valid (1: lists answer
 //          queries), occupied cells beyond the cap, sub-cells without a list,
-//          (build) cells left by the first and the second pass over the cells,
-//          at kClClaim the entries claimed, as 64 bits
+//          (build) cells the first pass over them left to the second, at
+//          kClClaim the entries claimed, as 64 bits
 // ---------------------------------------------------------------------------
 constexpr uint32_t kNoList = 0xffffffffu;
 constexpr uint32_t kClState = 16, kClClaim = 8;

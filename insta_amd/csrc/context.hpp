@@ -88,7 +88,7 @@ struct insta_ctx {
     uint64_t* d_cl_bits = nullptr;  // [n_slots][G^3/64]
     uint32_t* d_cl_rank = nullptr;  // [n_slots][G^3/64]
     uint32_t* d_cl_cells = nullptr; // [n_slots][cell_list_cells] occupied cells (linear index)
-    uint32_t* d_cl_left = nullptr;  // [n_slots][2][cell_list_cells] build scratch: cells left by either pass over them
+    uint32_t* d_cl_left = nullptr;  // [n_slots][2][cell_list_cells] build scratch: cells left to the second pass, and to the per-lane walks
     uint2* d_cl_head = nullptr;     // [n_slots][cell_list_cells * S^3]
     uint32_t* d_cl_ent = nullptr;   // [n_slots][cell_list_entries]
     uint32_t* d_cl_state = nullptr; // [n_slots][kClState]
