@@ -198,7 +198,12 @@ constexpr int kTravCounters = 6;
 // budgets, 244 + 36 us (second pass) with; its 512^2 frame 702 -> 572 + 30.
 // Giving up earlier (24 or 12 entries) or with more lanes left costs more in
 // the second pass (410 us, 51 us) than it saves; later, the tail returns.
-constexpr uint32_t kLeafFewLanes = 16, kLeafFew = 8, kLeafMost = 64;
+// The density grid's samples (kMostBudget), sorted, leave whole waves of long
+// queries, and the second pass costs a query one round per 64 leaves: they give
+// up after a sixteenth of the tree's leaves (16 of the 2,048-triangle sphere's
+// 256: an update of 262,144 samples 412 us, with 64 953 us; the head's 1,024
+// leaves: 64, with 32 one of 1,048,576 samples 6,770 us instead of 3,300).
+constexpr uint32_t kLeafFewLanes = 16, kLeafFew = 8, kLeafLeast = 16, kLeafMost = 64;
 constexpr uint32_t kListFewLanes = 4, kListFew = 72, kListMost = 192;
 
 INSTA_DEV bool few_lanes_left(uint32_t few) { return (uint32_t)__popcll(__ballot(true)) <= few; }
@@ -214,6 +219,8 @@ INSTA_DEV Hit bvh_closest_impl(const MeshView& m, V3 p, uint32_t* stack, uint32_
     uint32_t best_orig = 0xffffffffu;
     float bound = prune_bound(best);
     const uint32_t shift = 2u * m.k;
+    [[maybe_unused]] const uint32_t most =
+        kBudget == kMostBudget ? max(kLeafLeast, min(kLeafMost, (1u << shift) / 16u)) : kLeafMost;
     int sp = 0;
     uint32_t node = 0, leaves = 0;
     for (;;) {
@@ -282,7 +289,7 @@ INSTA_DEV Hit bvh_closest_impl(const MeshView& m, V3 p, uint32_t* stack, uint32_
         if (node == kNoNode) break;
         if constexpr (kBudget != kNoBudget) {
             ++leaves;
-            if (leaves >= kLeafMost || (kBudget == kFewBudget && leaves >= kLeafFew && few_lanes_left(kLeafFewLanes))) {
+            if (leaves >= most || (kBudget == kFewBudget && leaves >= kLeafFew && few_lanes_left(kLeafFewLanes))) {
                 *unfinished = true;
                 break;
             }

@@ -223,9 +223,8 @@ def _least_candidates(orc, verts, faces, cells, G, S):
 
 @pytest.mark.parametrize("room", ["all", "exact", "few_more", "too_few"])
 def test_cells_that_overflow_both_passes(head_avatar, room):
-    """A coarse grid, most of whose cells have more candidates than either per-cell pass holds: what the first
-    pass leaves over and what the second does together exceed the cells' capacity where that is the occupied
-    cells' number or little more.  Ids and distances against brute force, also after the slot got another
+    """A coarse grid, most of whose cells have more candidates than either per-cell pass holds and go on to the
+    per-lane kernels, with room for all cells, for exactly the occupied ones, for a few more, and for too few.  Ids and distances against brute force, also after the slot got another
     expression (the heads of a cell that is left out would be the first one's)."""
     torch = _torch()
     from insta_amd.capi import Context
