@@ -686,7 +686,9 @@ insta_status launch_cell_lists(insta_ctx* ctx, uint32_t slot, hipStream_t stream
                        ctx->d_cl_cells + slot * (size_t)ctx->cfg.cell_list_cells);
     const size_t shmem = (size_t)stack_depth(ctx->bvh_k) * kClThreads * sizeof(uint32_t);
     const uint64_t max_sub = (uint64_t)a.cap * a.S * a.S * a.S;
-    const uint32_t blocks = (uint32_t)std::min<uint64_t>((max_sub + kClThreads - 1) / kClThreads, kClMaxBlocks);
+    // (after the per-cell kernels most lanes pass over their cell)
+    const uint32_t blocks =
+        (uint32_t)std::min<uint64_t>((max_sub + kClThreads - 1) / kClThreads, a.all ? kClMaxBlocks : 1024u);
     if (!a.all) {
         hipLaunchKernelGGL(cl_cell_kernel<false>, dim3(std::min(a.cap, kClMaxBlocks)), dim3(kCellThreads), 0, stream, a);
         hipLaunchKernelGGL(cl_cell_kernel<true>, dim3(std::min(a.cap, 512u)), dim3(kCellThreads2), 0, stream, a);
