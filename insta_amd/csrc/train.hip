@@ -26,9 +26,9 @@
 //             every level and then scattered into the hash tables: levels
 //             that fit in LDS by a workgroup per level, feature and chunk
 //             (FP64 LDS atomics; packed FP16 ones with FP16 gradients), larger
-//             ones by global atomics, one level per XCD at a time, or, for
-//             batches above kPartMinBatch, partitioned by table slice and
-//             accumulated slice by slice in LDS
+//             ones partitioned by table slice and accumulated slice by slice in
+//             LDS the same way, or, where a table exceeds kPartMaxEntries, by
+//             global atomics (FP64; packed FP16), one level per XCD at a time
 //   wgrad     weight gradients dW = sum_n delta_n x_n^T as per-chunk partial
 //             products on FP32 MFMA (samples as the K dimension, operands
 //             staged through LDS), then a fixed-order sum over chunks:
@@ -160,10 +160,12 @@ struct TrainState {
     float* t_buf = nullptr;        // march t values, step-major [max_steps][rays of the step]: the rounds and the loss read them
     // optimizer
     float *grad = nullptr, *adam_m = nullptr, *adam_v = nullptr;
-    // hash-table gradients under FP16 accumulation: kHalfCopies partial tables
-    // of the levels beyond the LDS-scattered ones, summed into grad afterwards
-    __half2* grad_h = nullptr;
-    // partitioned scatter: its levels (0: the batch is not partitioned), the
+    // hash-table gradients added to by global atomics (a table above
+    // kPartMaxEntries only): FP64, or under FP16 accumulation kHalfCopies
+    // partial tables; summed into grad afterwards
+    double2* grad_d = nullptr;
+    __half2* grad_h = nullptr;      // (the same memory)
+    // partitioned scatter: its levels (0: none, or tables too large for it), the
     // records of one pass and their directory
     uint32_t part_levels = 0;
     void* recs = nullptr;
@@ -956,23 +958,25 @@ __global__ __launch_bounds__(kScatterThreads) void scatter_lds_kernel(GridParams
 // L2s and HBM.  On the levels of run_mask the corner gradients of consecutive
 // samples that land on one entry (coarse levels along one ray) are summed
 // across the wave first and added by one lane.
-// FP32: atomics straight into the gradients; neighbouring lanes first pair
-// up, so that an entry's two adds are neighbours in one memory request.
+// FP32: FP64 atomics, so that the sums are exact but for one rounding however
+// many samples share an entry; neighbouring lanes first pair up, so that an
+// entry's two adds are neighbours in one memory request.
 // H16: one packed FP16 atomic per corner, into one of kHalfCopies partial
 // tables (by block of kLevelThreads samples; a level's first copy before its
 // second), which keep the rounding of many small adds in check and are summed
 // in a fixed order afterwards.
-// Bound by the L2's atomics, about one request per clock and XCD: 100,003
-// random samples at full size (14 levels of up to 2^19 entries) take 698 us,
-// added per sample into one copy of the tables per XCD they took 1,300.
+// Bound by the L2's atomics, about one request per clock and XCD: a plugin pass
+// of 100,000 samples near the skin at T = 2^20 takes 1,305 us; with one FP32
+// copy of the tables per XCD 2,220, with FP32 atomics straight into the
+// gradients 1,118, but sums of 8,192 crowded samples were off by 1.2e-6 of
+// themselves (now below 2^-22).
 constexpr uint32_t kLevelThreads = 256;
 constexpr uint32_t kHalfCopies = 8;
-// Batches above kPartMinBatch, with no table above kPartMaxEntries (the
-// partition's directory), are partitioned, kPartPass samples at a time (352 MB
-// of records at full size).  Below, the atomics are cheaper than the fixed
-// work of walking every slice and storing every entry: about 7 us per 1,000
-// samples against 60 us.
-constexpr uint32_t kPartMinBatch = 8192;
+// Where no table exceeds kPartMaxEntries (the partition's directory) the levels
+// are partitioned instead, kPartPass samples at a time (352 MB of records at
+// full size), batches of any size: a plugin pass at full size takes 157 / 172 /
+// 191 us for 300 / 4,000 / 8,192 samples; with FP32 atomics for these batches
+// 152 / 183 / 232 us, and sums off by up to 9e-7 of themselves.
 constexpr uint32_t kPartMaxEntries = 1u << 19;
 constexpr uint32_t kPartPass = 1u << 18;
 constexpr uint32_t kPartSlices = 64;  // one wave scans a chunk's slice counts
@@ -983,7 +987,7 @@ __global__ __launch_bounds__(kLevelThreads) void scatter_levels_kernel(GridParam
                                                                        const uint32_t* __restrict__ c_idx,
                                                                        const float4* __restrict__ cpos,
                                                                        const float* __restrict__ denc_g, uint32_t ld,
-                                                                       float* __restrict__ grad_tab,
+                                                                       double* __restrict__ grad_d,
                                                                        __half2* __restrict__ grad_h,
                                                                        uint64_t entries) {
     // blocks: sample blocks per level, a multiple of kHalfCopies
@@ -1031,15 +1035,15 @@ __global__ __launch_bounds__(kLevelThreads) void scatter_levels_kernel(GridParam
             const float ye = __uint_as_float(dpp<0xA0>(__float_as_uint(v.y)));
             const float xo = __uint_as_float(dpp<0xF5>(__float_as_uint(v.x)));
             const float ve = odd ? ye : v.x, vo = odd ? v.y : xo;
-            if (ie != ~0u) atomicAdd(grad_tab + 2u * (size_t)ie + (odd ? 1u : 0u), ve);
-            if (io != ~0u) atomicAdd(grad_tab + 2u * (size_t)io + (odd ? 1u : 0u), vo);
+            if (ie != ~0u) unsafeAtomicAdd(grad_d + 2u * (size_t)ie + (odd ? 1u : 0u), (double)ve);
+            if (io != ~0u) unsafeAtomicAdd(grad_d + 2u * (size_t)io + (odd ? 1u : 0u), (double)vo);
         }
     }
 }
 
-// The same levels for large batches, in two kernels without global atomics
-// (an XCD's L2 retires about one request of them per clock, 5.6 ms per 10^6
-// samples at full size).  partition_kernel writes each chunk's corner
+// The same levels in two kernels without global atomics (an XCD's L2 retires
+// about one request of them per clock, 5.6 ms per 10^6 samples at full size).
+// partition_kernel writes each chunk's corner
 // gradients as records (entry, value), sorted by slice of the level's table;
 // accumulate_kernel, one workgroup per (slice, level), adds its slice's records
 // of every chunk into an LDS copy of the slice and stores it: every entry of
@@ -1240,8 +1244,18 @@ __global__ __launch_bounds__(kAccThreads) void accumulate_kernel(GridParams gp, 
     }
 }
 
-// Gradients of the entries [first, entries) into grad_tab: the sum of the
-// FP16 copies in copy order.
+// Gradients of the entries [first, entries) into grad_tab: the FP64 sums,
+// rounded.
+__global__ void grad_doubles_store_kernel(const double2* __restrict__ grad_d, uint64_t first, uint64_t entries,
+                                          float* __restrict__ grad_tab) {
+    for (uint64_t e = first + blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; e < entries;
+         e += (uint64_t)gridDim.x * blockDim.x) {
+        const double2 v = grad_d[e];
+        *reinterpret_cast<float2*>(grad_tab + 2 * e) = make_float2((float)v.x, (float)v.y);
+    }
+}
+
+// The same of the FP16 copies, summed in copy order.
 __global__ void grad_copies_reduce_kernel(const __half2* __restrict__ grad_h, uint64_t first, uint64_t entries,
                                           float* __restrict__ grad_tab) {
     for (uint64_t e = first + blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; e < entries;
@@ -1587,6 +1601,11 @@ void free_workspace_train(TrainState* ts) {
     ts->ray_cap = ts->sample_cap = ts->compact_cap = 0;
 }
 
+uint32_t largest_table(const insta_ctx* ctx) {
+    const GridParams gp = grid_params(ctx);
+    return *std::max_element(gp.size, gp.size + ctx->cfg.n_levels);
+}
+
 // rays, marched samples and the compacted batch grow independently to the
 // largest request seen
 // grow the training workspace to hold n_rays rays, n_samples marched samples
@@ -1617,11 +1636,8 @@ insta_status grow_train_workspace(insta_ctx* ctx, TrainState* ts, uint32_t n_ray
     ok = ok && train_alloc(ts->part, (size_t)wgrad_chunks(cc) * n_mlp * sizeof(float));
     ok = ok && train_alloc(ts->t_buf, (size_t)rc * ctx->cfg.max_steps * sizeof(float));
     ok = ok && train_alloc(ts->denc, (size_t)2 * INSTA_MAX_LEVELS * cc * sizeof(float));
-    const GridParams gp = grid_params(ctx);
-    uint32_t largest = 0;
-    for (uint32_t l = 0; l < ctx->cfg.n_levels; ++l) largest = std::max(largest, gp.size[l]);
     const uint32_t big = ctx->cfg.n_levels - (uint32_t)__builtin_popcount(ts->lds_levels);
-    if (big && cc > kPartMinBatch && largest <= kPartMaxEntries) {
+    if (big && largest_table(ctx) <= kPartMaxEntries) {
         const size_t pass = std::min(cc, kPartPass);
         const size_t c32 = (pass + Part<false>::kChunkSamples - 1) / Part<false>::kChunkSamples;
         const size_t c16 = (pass + Part<true>::kChunkSamples - 1) / Part<true>::kChunkSamples;
@@ -1692,8 +1708,9 @@ insta_status launch_train_backward(insta_ctx* ctx, TrainState* ts, const insta_t
     const uint32_t n_mlp = (uint32_t)ctx->layout.n_mlp_params;
     const dim3 sgrid(mlp_blocks(cap));
     float* grad_tab = ts->grad + n_mlp;
-    // levels whose tables fit in LDS are scattered by scatter_lds_kernel (FP32
-    // or packed FP16), the others by scatter_levels_kernel (FP32)
+    // levels whose tables fit in LDS are scattered by scatter_lds64_kernel
+    // (FP16: scatter_lds_kernel), the others partitioned or, with tables too
+    // large for that, by scatter_levels_kernel
     const uint32_t lds_mask = ts->lds_levels, lds_end = ts->lds_end;
     const uint32_t big_mask = ((1u << L) - 1u) & ~lds_mask;
     // levels whose cells span at least 1 / kRunMaxStepCells marching steps
@@ -1732,22 +1749,22 @@ insta_status launch_train_backward(insta_ctx* ctx, TrainState* ts, const insta_t
         const uint32_t slots = (__builtin_popcount(big_mask) + kXcds - 1) / kXcds;
         const dim3 grid(kXcds * slots * blocks);
         if (tc.grid_grad_fp16) {
-            // clear this backward's copies (a fill kernel: capturable)
+            // clear this backward's copies (fill kernels: capturable)
             hipLaunchKernelGGL(fill_zero_kernel, dim3(2048), dim3(256), 0, stream,
                                reinterpret_cast<uint32_t*>(ts->grad_h), kHalfCopies * entries);
             hipLaunchKernelGGL(scatter_levels_kernel<true>, grid, dim3(kLevelThreads), 0, stream, gp, big_mask,
-                               run_mask, blocks, n_dev, ts->c_idx, ts->s_cpos, ts->denc, cap, grad_tab, ts->grad_h,
-                               entries);
+                               run_mask, blocks, n_dev, ts->c_idx, ts->s_cpos, ts->denc, cap,
+                               reinterpret_cast<double*>(ts->grad_d), ts->grad_h, entries);
             hipLaunchKernelGGL(grad_copies_reduce_kernel, dim3(2048), dim3(256), 0, stream, ts->grad_h,
                                (uint64_t)lds_end, entries, grad_tab);
         } else {
-            // the added-to gradients start at zero (a fill kernel: capturable);
-            // every other path writes all of its gradients
-            hipLaunchKernelGGL(fill_zero_kernel, dim3(1024), dim3(256), 0, stream,
-                               reinterpret_cast<uint32_t*>(grad_tab + 2 * (size_t)lds_end), 2 * (entries - lds_end));
+            hipLaunchKernelGGL(fill_zero_kernel, dim3(2048), dim3(256), 0, stream,
+                               reinterpret_cast<uint32_t*>(ts->grad_d + lds_end), 4 * (entries - lds_end));
             hipLaunchKernelGGL(scatter_levels_kernel<false>, grid, dim3(kLevelThreads), 0, stream, gp, big_mask,
-                               run_mask, blocks, n_dev, ts->c_idx, ts->s_cpos, ts->denc, cap, grad_tab, ts->grad_h,
-                               entries);
+                               run_mask, blocks, n_dev, ts->c_idx, ts->s_cpos, ts->denc, cap,
+                               reinterpret_cast<double*>(ts->grad_d), ts->grad_h, entries);
+            hipLaunchKernelGGL(grad_doubles_store_kernel, dim3(2048), dim3(256), 0, stream, ts->grad_d,
+                               (uint64_t)lds_end, entries, grad_tab);
         }
         INSTA_HIP(hipGetLastError());
     }
@@ -1914,7 +1931,7 @@ void free_train(insta_ctx* ctx) {
     if (!ts) return;
     free_workspace_train(ts);
     dev_free(ts->images); dev_free(ts->meta); dev_free(ts->seg); dev_free(ts->depth);
-    dev_free(ts->grad); dev_free(ts->grad_h); dev_free(ts->grad_p);
+    dev_free(ts->grad); dev_free(ts->grad_d); dev_free(ts->grad_p);
     dev_free(ts->adam_m); dev_free(ts->adam_v); dev_free(ts->counters); dev_free(ts->net_extra);
     if (ctx->net_src == ts->ema_infer) ctx->net_src = nullptr;
     dev_free(ts->ema); dev_free(ts->ema_infer);
@@ -1937,7 +1954,8 @@ static insta_status ensure_train_state(insta_ctx* ctx, hipStream_t stream) {
         bool ok = train_alloc(ts->grad, np * sizeof(float)) && train_alloc(ts->adam_m, np * sizeof(float)) &&
                   train_alloc(ts->adam_v, np * sizeof(float)) && train_alloc(ts->ema, np * sizeof(float)) &&
                   train_alloc(ts->ema_infer, np * sizeof(float)) &&
-                  train_alloc(ts->grad_h, kHalfCopies * (ctx->layout.n_grid_params / 2) * sizeof(__half2)) &&
+                  (largest_table(ctx) <= kPartMaxEntries ||
+                   train_alloc(ts->grad_d, kHalfCopies * (ctx->layout.n_grid_params / 2) * sizeof(__half2))) &&
                   (ts->lds_end == 0 ||
                    train_alloc(ts->grad_p, (size_t)kScatterMaxChunks * 2 * ts->lds_end * sizeof(float))) &&
                   train_alloc(ts->counters, kTCounters * sizeof(uint32_t)) &&
@@ -1948,6 +1966,7 @@ static insta_status ensure_train_state(insta_ctx* ctx, hipStream_t stream) {
             set_error("training state allocation failed");
             return INSTA_ERR_OOM;
         }
+        ts->grad_h = reinterpret_cast<__half2*>(ts->grad_d);
         INSTA_HIP(hipMemsetAsync(ts->adam_m, 0, np * sizeof(float), stream));
         INSTA_HIP(hipMemsetAsync(ts->adam_v, 0, np * sizeof(float), stream));
     }
