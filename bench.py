@@ -102,9 +102,11 @@ def timed_renders(ctx, cams, res, steps, warmup, out):
     """Render `steps` frames (after `warmup`), cycling the 16 posed frames.
     The timed pass runs with profiling off and reads nothing back between
     frames (each insta_render still waits for its own frame's counters, as
-    the API returns a finished image).  A second, untimed pass over the same
+    the API returns a finished image).  Two more, untimed passes over the same
     frames (renders are deterministic: same camera, frame and sample index)
-    collects the sample counts and the per-kernel HIP-event breakdown.
+    collect the sample and round counts, again with profiling off, and the
+    per-kernel HIP-event breakdown: a profiled frame takes all its samples in
+    one round, so its kernels' times and items are those of that schedule.
     Returns (seconds, samples composited, samples emitted, kernel profile)."""
     import torch
     for s in range(warmup):
@@ -116,7 +118,6 @@ def timed_renders(ctx, cams, res, steps, warmup, out):
         ctx.render(cams[f], res, res, f, f, 0, out)
     torch.cuda.synchronize()
     elapsed = time.perf_counter() - t0
-    ctx.set_profiling(True)
     samples = emitted = rounds = rays0 = 0
     for s in range(steps):
         f = s % 16
@@ -126,6 +127,10 @@ def timed_renders(ctx, cams, res, steps, warmup, out):
         emitted += st.n_samples_emitted
         rounds += st.n_iterations
         rays0 += st.n_rays_alive0
+    ctx.set_profiling(True)
+    for s in range(steps):
+        f = s % 16
+        ctx.render(cams[f], res, res, f, f, 0, out)
     torch.cuda.synchronize()
     prof = ctx.profile()
     prof["_rounds_per_frame"] = rounds / steps
@@ -620,7 +625,8 @@ def main():
     per_launch_items = p["items"] / p["launches"]
     c = costs.get(dom, dict(bytes=0, flops=0))
     # HBM bytes per launch of the same kernels from the committed rocprofv3
-    # FETCH_SIZE / WRITE_SIZE summary of this workload (scaled by a 256 MiB copy)
+    # FETCH_SIZE / WRITE_SIZE summary of this workload's one-round frames
+    # (scaled by a 256 MiB copy)
     traffic = None
     prof_json = ROOT / "profiles" / "render_full_512.json"
     if prof_json.exists():

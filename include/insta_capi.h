@@ -478,8 +478,9 @@ typedef struct insta_train_config {
     uint32_t grid_grad_fp16;  /* 1: hash-grid gradients accumulated in FP16 (packed atomics): per
                                  chunk of 8192 batch entries in LDS for levels of at most 16384
                                  entries (the chunks then summed in FP32), in eight copies by batch
-                                 block (then summed in FP32) for larger levels; 0: FP32
-                                 throughout */
+                                 block (then summed in FP32) for larger levels; 0: FP32 products
+                                 summed in FP64 and rounded to FP32 (per such chunk; per 2^18
+                                 entries for larger levels) */
     uint32_t apply_update;    /* 0: gradients only, parameters unchanged */
     uint32_t seed;            /* PCG32 seed of the ray/background stream */
     int32_t  occupancy_slot;  /* grid the rays march: INSTA_OCCUPANCY_PER_FRAME (each image's
@@ -699,8 +700,11 @@ typedef struct insta_profile {
      * entries they scanned (their exact distances are in bvh_triangles) */
     uint64_t list_queries, list_entries;
 } insta_profile;
-/* enable != 0 starts (and zeroes) accumulation; 0 stops it.  enable == 2 also
- * counts traversal work, with a counting build of the deformation kernel
+/* enable != 0 starts (and zeroes) accumulation; 0 stops it.  A profiled frame
+ * evaluates each ray's samples in one round (all that fit the workspace), so
+ * that a kernel class has one time per frame; other frames of 2^15 pixels or
+ * more take them in windows while the rays live: the same image, and where
+ * rays end early fewer samples.  enable == 2 also counts traversal work, with a counting build of the deformation kernel
  * (slower: for a separate, untimed render). */
 insta_status insta_set_profiling(insta_ctx* ctx, int enable);
 insta_status insta_get_profile(insta_ctx* ctx, insta_profile* out);
