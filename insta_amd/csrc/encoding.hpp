@@ -84,16 +84,22 @@ INSTA_DEV void cell_corners(const GridParams& gp, uint32_t l, V3 x, uint32_t idx
 // (renders) are bound by the instructions of this function, scattered ones by
 // cache lookups, one per lane and load.  So the corners of an x pair come with
 // one load: neighbours on dense levels; on hashed ones the two hashes of an
-// even x differ in bit 0 only, and lanes with an odd x load the upper corner
-// by itself.  Offsets are computed in bytes (the hash's factors times the
-// entry's size), dense rows lie at four scalar bases, and which half of its
-// aligned pair a corner is follows from the cell's parity, the factors being
-// odd.
-// On the 16-level head, 8 loads one after another / 8 together / pairs: FP32
-// render at 512 x 512 (two rounds) 1,355 / 1,294 / 1,255 us; 1,048,576 BF16
-// positions 433 / 412 / 362 us; training forward of 100,000 positions 156 us
-// with 8 loads together, 144 us with pairs.
-template <class E>
+// even x differ in bit 0 only.  Of an odd x, the lower corner comes with its
+// pair all the same and the upper one by itself (kPairs: no lane waits for the
+// others' way), or lanes with an odd x load all corners by themselves
+// (kEvenPairs: two ways, but no bytes for nothing), or all lanes do (kSingle).
+// Offsets are computed in bytes (the hash's factors times the entry's size),
+// dense rows lie at four scalar bases, and which half of its aligned pair a
+// corner is follows from the cell's parity, the factors being odd.
+// 16-level head, us, corners one after another / kSingle / kPairs / kEvenPairs:
+//   FP32 render at 512 x 512              1,355 / 1,294 / 1,255 / 1,330
+//   1,048,576 positions near the skin, FP32 617 / 623 / 560 / 504, BF16 458 / 387 / 383 / 331
+//   anywhere,                          FP32 817 / 892 / 853 / 830, BF16 628 / 587 / 616 / 525
+//   on a lattice,                      FP32 679 / 703 / 706 / 695, BF16 505 / 500 / 589 / 527
+// so renders, training and the density grid take kPairs, inference calls, whose
+// positions may come in any order, kEvenPairs.
+enum Corners { kPairs, kEvenPairs, kSingle };
+template <class E, Corners kMode = kPairs>
 INSTA_DEV void cell_fetch(const GridParams& gp, uint32_t l, V3 x, const char* __restrict__ base, E v[8], float frac[3],
                           float w[8]) {
     struct Two {  // aligned as one entry: half of the pairs start at an odd one
@@ -129,12 +135,20 @@ INSTA_DEV void cell_fetch(const GridParams& gp, uint32_t l, V3 x, const char* __
         const uint32_t hy1 = hy + kPrimeY * S, hz1 = hz + kPrimeZ * S;
         const uint32_t yz[4] = {hy ^ hz, hy1 ^ hz, hy ^ hz1, hy1 ^ hz1};
         const uint32_t x0 = g[0] * S, x1 = x0 + S;
+        const bool apart = g[0] & 1u;
+        if (kMode == kSingle || (kMode == kEvenPairs && apart)) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                v[2 * j] = *reinterpret_cast<const E*>(base + ((x0 ^ yz[j]) & mask));
+                v[2 * j + 1] = *reinterpret_cast<const E*>(base + ((x1 ^ yz[j]) & mask));
+            }
+            return;
+        }
         Two t[4];  // level tables hold an even number of entries
 #pragma unroll
         for (int j = 0; j < 4; ++j) t[j] = *reinterpret_cast<const Two*>(base + ((x0 ^ yz[j]) & (mask & ~S)));
-        const bool apart = g[0] & 1u;
         E up[4];
-        if (apart) {
+        if (kMode == kPairs && apart) {
 #pragma unroll
             for (int j = 0; j < 4; ++j) up[j] = *reinterpret_cast<const E*>(base + ((x1 ^ yz[j]) & mask));
         }
@@ -144,12 +158,13 @@ INSTA_DEV void cell_fetch(const GridParams& gp, uint32_t l, V3 x, const char* __
             const bool odd = (j == 0 || j == 3) ? upper : !upper;
             v[2 * j] = odd ? t[j].b : t[j].a;
             const E other = odd ? t[j].a : t[j].b;
-            v[2 * j + 1] = apart ? up[j] : other;
+            v[2 * j + 1] = kMode == kPairs && apart ? up[j] : other;
         }
     }
 }
 
-template <int F>
+// Features of position x on level l; kMode as in cell_fetch (F = 2).
+template <int F, Corners kMode = kPairs>
 INSTA_DEV void encode_level(const float* __restrict__ table, const GridParams& gp, uint32_t l, V3 x, float acc[F]) {
     float w[8];
     const char* base = reinterpret_cast<const char*>(table + (size_t)gp.offset[l] * F);
@@ -158,7 +173,7 @@ INSTA_DEV void encode_level(const float* __restrict__ table, const GridParams& g
     if constexpr (F == 2) {
         float2 v[8];
         float frac[3];
-        cell_fetch(gp, l, x, base, v, frac, w);
+        cell_fetch<float2, kMode>(gp, l, x, base, v, frac, w);
 #pragma unroll
         for (uint32_t c = 0; c < 8; ++c) {
             acc[0] = acc[0] + w[c] * v[c].x;

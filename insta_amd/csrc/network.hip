@@ -17,7 +17,16 @@ namespace {
 constexpr uint32_t kNetThreads = 128;
 constexpr uint32_t kEncThreads = 256;
 
-template <int F>
+// Calls up to here fetch pairs of corners, larger ones every corner by itself:
+// where a call's lookups exceed the caches, the wider loads of more positions at
+// once only push each other's lines out.  16-level head, us, pairs / by
+// themselves (and one after another), positions anywhere / near the skin:
+//     100,000    110 / 112 (113)    79 /  85 ( 84)
+//     300,000    311 / 291 (291)   189 / 192 (201)
+//   1,048,576  1,067 / 997 (946)   603 / 594 (640)
+constexpr uint32_t kEncPairs = 1u << 18;
+
+template <int F, Corners kMode>
 __global__ __launch_bounds__(kEncThreads) void encode_kernel(const float* __restrict__ table, GridParams gp,
                                                              uint32_t n_levels, const float* __restrict__ pos,
                                                              uint32_t n, float* __restrict__ out) {
@@ -27,7 +36,7 @@ __global__ __launch_bounds__(kEncThreads) void encode_kernel(const float* __rest
     float* o = out + (size_t)i * n_levels * F;
     for (uint32_t l = 0; l < n_levels; ++l) {
         float acc[F];
-        encode_level<F>(table, gp, l, x, acc);
+        encode_level<F, kMode>(table, gp, l, x, acc);
 #pragma unroll
         for (int f = 0; f < F; ++f) o[l * F + f] = acc[f];
     }
@@ -277,10 +286,10 @@ insta_status launch_encode(insta_ctx* ctx, const float* pos, uint32_t n, float* 
     const GridParams gp = grid_params(ctx);
     const dim3 grid((n + kEncThreads - 1) / kEncThreads), block(kEncThreads);
     switch (ctx->cfg.n_features_per_level) {
-        case 1: hipLaunchKernelGGL(encode_kernel<1>, grid, block, 0, stream, table, gp, ctx->cfg.n_levels, pos, n, out); break;
-        case 2: hipLaunchKernelGGL(encode_kernel<2>, grid, block, 0, stream, table, gp, ctx->cfg.n_levels, pos, n, out); break;
-        case 4: hipLaunchKernelGGL(encode_kernel<4>, grid, block, 0, stream, table, gp, ctx->cfg.n_levels, pos, n, out); break;
-        case 8: hipLaunchKernelGGL(encode_kernel<8>, grid, block, 0, stream, table, gp, ctx->cfg.n_levels, pos, n, out); break;
+        case 1: hipLaunchKernelGGL((encode_kernel<1, kPairs>), grid, block, 0, stream, table, gp, ctx->cfg.n_levels, pos, n, out); break;
+        case 2: hipLaunchKernelGGL((n <= kEncPairs ? encode_kernel<2, kPairs> : encode_kernel<2, kSingle>), grid, block, 0, stream, table, gp, ctx->cfg.n_levels, pos, n, out); break;
+        case 4: hipLaunchKernelGGL((encode_kernel<4, kPairs>), grid, block, 0, stream, table, gp, ctx->cfg.n_levels, pos, n, out); break;
+        case 8: hipLaunchKernelGGL((encode_kernel<8, kPairs>), grid, block, 0, stream, table, gp, ctx->cfg.n_levels, pos, n, out); break;
         default: set_error("encode: n_features_per_level must be 1, 2, 4 or 8"); return INSTA_ERR_UNSUPPORTED;
     }
     INSTA_HIP(hipGetLastError());

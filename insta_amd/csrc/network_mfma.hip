@@ -163,6 +163,7 @@ __global__ void table_to_half_kernel(const float* __restrict__ src, _Float16* __
 // sample sources
 // ---------------------------------------------------------------------------
 struct SoaSrc {
+    static constexpr Corners kCorners = kPairs;      // samples of neighbouring rays
     const float4* cpos;
     const float4* cdir;
     float4* out;
@@ -176,6 +177,7 @@ struct SoaSrc {
     INSTA_DEV uint32_t sel(uint32_t i) const { return __float_as_uint(cdir[i].w); }
 };
 struct AosSrc {
+    static constexpr Corners kCorners = kEvenPairs;  // positions in any order
     const float* coords;
     uint32_t stride, n;
     float4* out;
@@ -210,17 +212,17 @@ INSTA_DEV void sh16_dev(float x, float y, float z, float* o) {
 
 // one level of the hash grid, FP32 or FP16 table, FP32 interpolation (the
 // same operation order as the scalar encode)
-template <typename TT>
+template <typename TT, Corners kMode>
 INSTA_DEV float2 encode_level2(const TT* __restrict__ table, const GridParams& gp, uint32_t l, V3 x) {
     if constexpr (sizeof(TT) == 4) {
         float acc[2];
-        encode_level<2>(table, gp, l, x, acc);
+        encode_level<2, kMode>(table, gp, l, x, acc);
         return make_float2(acc[0], acc[1]);
     } else {
         typedef _Float16 h2 __attribute__((ext_vector_type(2)));
         float w[8], frac[3];
         h2 v[8];
-        cell_fetch(gp, l, x, reinterpret_cast<const char*>(table + (size_t)gp.offset[l] * 2), v, frac, w);
+        cell_fetch<h2, kMode>(gp, l, x, reinterpret_cast<const char*>(table + (size_t)gp.offset[l] * 2), v, frac, w);
         // fma(w, v, 0) rounds as w * v and takes the FP16 value as it is (one
         // v_fma_mix_f32 for a conversion and a product)
         float a0 = __builtin_fmaf(w[0], (float)v[0].x, 0.0f);
@@ -313,7 +315,7 @@ INSTA_DEV void f32_tiles(float* s_x, const float* __restrict__ table, const Grid
                 src.load(i, p, d);
 #pragma unroll 2
                 for (int l = l0; l < l0 + L / kSplit; ++l) {
-                    const float2 e = encode_level2<float>(table, gp, (uint32_t)l, p);
+                    const float2 e = encode_level2<float, Src::kCorners>(table, gp, (uint32_t)l, p);
                     row[2 * l] = e.x;
                     row[2 * l + 1] = e.y;
                 }
@@ -462,7 +464,7 @@ INSTA_DEV void x32_tiles(T* s_x, const typename Vec8<T>::type* A, const _Float16
 // one level at a time: two spill, and four waves a SIMD cover the latency
 #pragma unroll 1
                 for (int l = l0; l < l0 + L / kSplit; ++l) {
-                    const float2 e = encode_level2<_Float16>(table, gp, (uint32_t)l, p);
+                    const float2 e = encode_level2<_Float16, Src::kCorners>(table, gp, (uint32_t)l, p);
                     row[2 * l] = (T)e.x;
                     row[2 * l + 1] = (T)e.y;
                 }
