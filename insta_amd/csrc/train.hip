@@ -1543,21 +1543,12 @@ __global__ void wgrad_reduce_kernel(const float* __restrict__ part, const uint32
 }
 
 // Unscale, optionally step Adam.  grad[] receives dL/dparam (unscaled).
-__global__ void adam_kernel(float* __restrict__ params, float* __restrict__ grad, const __half2* __restrict__ grad_h,
-                            float* __restrict__ m, float* __restrict__ v, uint64_t n_params, uint64_t n_mlp,
-                            float inv_scale, float lr, float b1, float b2, float eps, float bc1, float bc2,
-                            float l2_reg, uint32_t apply) {
+__global__ void adam_kernel(float* __restrict__ params, float* __restrict__ grad, float* __restrict__ m,
+                            float* __restrict__ v, uint64_t n_params, float inv_scale, float lr, float b1, float b2,
+                            float eps, float bc1, float bc2, float l2_reg, uint32_t apply) {
     for (uint64_t p = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; p < n_params;
          p += (uint64_t)gridDim.x * blockDim.x) {
-        float g;
-        if (grad_h && p >= n_mlp) {
-            const uint64_t q = p - n_mlp;
-            const __half2 h = grad_h[q >> 1];
-            g = (q & 1u) ? __high2float(h) : __low2float(h);
-        } else {
-            g = grad[p];
-        }
-        g = g * inv_scale;
+        float g = grad[p] * inv_scale;
         grad[p] = g;
         if (apply) {
             g = g + l2_reg * params[p];
@@ -2043,7 +2034,7 @@ insta_status train_step(insta_ctx* ctx, const insta_train_config& tc, insta_trai
         st = prepare_network(ctx, stream);
         if (st != INSTA_OK) return st;
     }
-    const uint64_t np = ctx->layout.n_params, n_mlp = ctx->layout.n_mlp_params;
+    const uint64_t np = ctx->layout.n_params;
     // the marched-sample cap is the step's (a larger reservation changes nothing)
     const uint32_t cap = tc.max_samples;
     hipLaunchKernelGGL(train_clear_kernel, dim3(1), dim3(64), 0, stream, ts->counters, cap);
@@ -2127,9 +2118,8 @@ insta_status train_step(insta_ctx* ctx, const insta_train_config& tc, insta_trai
     const uint32_t t = ts->adam_step + (tc.apply_update ? 1u : 0u);
     const float bc1 = tc.apply_update ? 1.0f - (float)std::pow((double)tc.beta1, (double)t) : 1.0f;
     const float bc2 = tc.apply_update ? 1.0f - (float)std::pow((double)tc.beta2, (double)t) : 1.0f;
-    hipLaunchKernelGGL(adam_kernel, dim3(2048), dim3(256), 0, stream, ctx->d_params, ts->grad,
-                       nullptr, ts->adam_m, ts->adam_v, np, n_mlp,
-                       1.0f / tc.loss_scale, tc.learning_rate, tc.beta1, tc.beta2, tc.epsilon, bc1, bc2,
+    hipLaunchKernelGGL(adam_kernel, dim3(2048), dim3(256), 0, stream, ctx->d_params, ts->grad, ts->adam_m, ts->adam_v,
+                       np, 1.0f / tc.loss_scale, tc.learning_rate, tc.beta1, tc.beta2, tc.epsilon, bc1, bc2,
                        tc.l2_reg, tc.apply_update);
     INSTA_HIP(hipGetLastError());
     if (tc.apply_update) {
