@@ -192,8 +192,13 @@ constexpr int kTravCounters = 6;
 // wave are still at it: a wave runs as long as its longest query, and a few long ones
 // (sub-cells around a mesh pole, whose lists hold hundreds of entries or
 // overflow to the BVH; points near the medial axis, which visit most leaves)
-// would otherwise set the kernel's time.  Waves whose lanes all walk the BVH
-// keep walking: their coherent walk is cheaper than a wave per query.  A
+// would otherwise set the kernel's time.  Waves of which more than kLeafWalkers
+// lanes walk the BVH (no lists: split 0, or before the occupancy is built) keep
+// walking to the last: their coherent walk is cheaper than a wave per query
+// (512 x 512 frame of the head at split 0: 2.96 ms without budgets, 3.06 so,
+// 5.9 with the few-lanes rule for them too), and lists of a coarser split are
+// longer by themselves: twice the entries per halving (split 1: 2.6 ms without
+// budgets, 2.8 so, 3.5 with the entries of split 4).  A
 // 301 x 257 frame of the 9,976-triangle head (1.2 M samples): 928 us without
 // budgets, 244 + 36 us (second pass) with; its 512^2 frame 702 -> 572 + 30.
 // Giving up earlier (24 or 12 entries) or with more lanes left costs more in
@@ -203,7 +208,7 @@ constexpr int kTravCounters = 6;
 // up after a sixteenth of the tree's leaves (16 of the 2,048-triangle sphere's
 // 256: an update of 262,144 samples 412 us, with 64 953 us; the head's 1,024
 // leaves: 64, with 32 one of 1,048,576 samples 6,770 us instead of 3,300).
-constexpr uint32_t kLeafFewLanes = 16, kLeafFew = 8, kLeafLeast = 16, kLeafMost = 64;
+constexpr uint32_t kLeafFewLanes = 16, kLeafFew = 8, kLeafLeast = 16, kLeafMost = 64, kLeafWalkers = 48;
 constexpr uint32_t kListFewLanes = 4, kListFew = 72, kListMost = 192;
 
 INSTA_DEV bool few_lanes_left(uint32_t few) { return (uint32_t)__popcll(__ballot(true)) <= few; }
@@ -221,6 +226,7 @@ INSTA_DEV Hit bvh_closest_impl(const MeshView& m, V3 p, uint32_t* stack, uint32_
     const uint32_t shift = 2u * m.k;
     [[maybe_unused]] const uint32_t most =
         kBudget == kMostBudget ? max(kLeafLeast, min(kLeafMost, (1u << shift) / 16u)) : kLeafMost;
+    [[maybe_unused]] const bool few = kBudget == kFewBudget && few_lanes_left(kLeafWalkers);
     int sp = 0;
     uint32_t node = 0, leaves = 0;
     for (;;) {
@@ -289,7 +295,7 @@ INSTA_DEV Hit bvh_closest_impl(const MeshView& m, V3 p, uint32_t* stack, uint32_
         if (node == kNoNode) break;
         if constexpr (kBudget != kNoBudget) {
             ++leaves;
-            if (leaves >= most || (kBudget == kFewBudget && leaves >= kLeafFew && few_lanes_left(kLeafFewLanes))) {
+            if (leaves >= most || (few && leaves >= kLeafFew && few_lanes_left(kLeafFewLanes))) {
                 *unfinished = true;
                 break;
             }
@@ -382,7 +388,7 @@ INSTA_DEV bool cell_list_find(const CellListView& cl, V3 p, uint2& hd) {
 constexpr uint32_t kListBatch = 2;
 
 template <bool kCount, Budget kBudget = kNoBudget>
-INSTA_DEV Hit list_closest_impl(const MeshView& m, const uint32_t* __restrict__ ent, uint2 hd, V3 p,
+INSTA_DEV Hit list_closest_impl(const MeshView& m, const uint32_t* __restrict__ ent, uint2 hd, V3 p, uint32_t split,
                                 TraversalCount* tc, bool* unfinished = nullptr) {
     float best = 3.40282347e38f;
     int32_t best_idx = -1;
@@ -391,13 +397,15 @@ INSTA_DEV Hit list_closest_impl(const MeshView& m, const uint32_t* __restrict__ 
     const uint32_t n = hd.y & 0xffffu;
     const uint32_t* e = ent + hd.x;
     if constexpr (kCount) ++tc->lists;
+    // twice the entries per halving of the split (4, 2, 1)
+    [[maybe_unused]] const uint32_t more = 2u - split / 2u, list_few = kListFew << more, list_most = kListMost << more;
     bool done = false;
     uint32_t wn[kListBatch];
 #pragma unroll
     for (uint32_t j = 0; j < kListBatch; ++j) wn[j] = e[min(j, n - 1u)];
     for (uint32_t k = 0; k < n && !done; k += kListBatch) {
         if constexpr (kBudget != kNoBudget) {
-            if (k >= kListMost || (kBudget == kFewBudget && k >= kListFew && few_lanes_left(kListFewLanes))) {
+            if (k >= list_most || (kBudget == kFewBudget && k >= list_few && few_lanes_left(kListFewLanes))) {
                 *unfinished = true;
                 break;
             }
@@ -458,7 +466,7 @@ INSTA_DEV Hit closest_impl(const MeshView& m, const CellListView& cl, V3 p, uint
                            TraversalCount* tc, bool* unfinished = nullptr) {
     uint2 hd;
     const bool in_box = p.x >= 0.0f && p.x <= 1.0f && p.y >= 0.0f && p.y <= 1.0f && p.z >= 0.0f && p.z <= 1.0f;
-    if (in_box && cell_list_find(cl, p, hd)) return list_closest_impl<kCount, kBudget>(m, cl.ent, hd, p, tc, unfinished);
+    if (in_box && cell_list_find(cl, p, hd)) return list_closest_impl<kCount, kBudget>(m, cl.ent, hd, p, cl.S, tc, unfinished);
     return bvh_closest_impl<kCount, kBudget>(m, p, stack, stride, 3.40282347e38f, tc, unfinished);
 }
 
