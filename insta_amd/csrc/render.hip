@@ -40,13 +40,20 @@ constexpr uint32_t kInitThreads = 256;   // (1,024: fewer reservations, slower s
 
 // Windows: a trained avatar's rays end within a few samples of the skin, so a
 // frame of at least kWindowPixels evaluates its rays' samples in rounds of
-// kWindow, kWindow, 2 kWindow, 4 kWindow, ... and only while the rays live; a
-// smaller frame, where a round's launches cost more than its samples, takes
-// them all in one.  A 1024 x 1024 FP16 frame of a head with an opaque skin
-// (50 samples marched per live ray, 25 composited) takes 3.41 ms, in one round
-// 4.35 ms (first windows of 8 and 16: 3.64 and 3.57 ms); a 512 x 512 frame of a
-// translucent volume, whose rays end nowhere, takes one more round, 50 us of
-// 2.4 ms, and one in which there is nothing to see two more (round_begin_kernel).
+// kWindow, kWindow, 2 kWindow, 4 kWindow, ... and only while the rays live.  A
+// round's launches and the latency of its walks cost some 130 us whatever it
+// has to do, so frames of less work take all samples in one: below 2^15 pixels,
+// and where the live rays could not meet kWindowSamples samples between them if
+// every step across the box were occupied (the device knows how many live).
+// A 1024 x 1024 FP16 frame of a head with an opaque skin (50 samples marched per
+// live ray, 25 composited) takes 3.41 ms, in one round 4.35 ms (first windows of
+// 8 and 16: 3.64 and 3.57 ms); a 512 x 512 frame of a translucent volume, whose
+// rays end nowhere, takes one more round, and one in which there is nothing to
+// see two more (round_begin_kernel).  us, windows / one round, FP32 and FP16:
+//   head, opaque skin   256^2 (7 M) 1,083 /  818  952 / 633   362^2 (15 M) 1,384 / 1,246  1,119 /   882
+//                       430^2 (21 M) 1,613 / 1,622  1,260 / 1,097   512^2 (30 M) 1,919 / 2,111  1,416 / 1,358
+//   small sphere, opaque 182^2 (14 M)   953 / 1,023  723 / 622   256^2 (27 M) 1,274 / 1,739    861 /   915
+constexpr float kWindowSamples = 13e6f;
 constexpr uint32_t kWindow = 12;
 constexpr uint32_t kWindowPixels = 1u << 15;
 constexpr uint32_t kAllSamples = 0xffffffffu;
@@ -382,7 +389,8 @@ __global__ void clear_counters_kernel(uint32_t* counters, uint32_t first, uint32
 
 // Before a round: clear the next live list's count and the round's sample and
 // queue counts, and set how many samples a ray may emit in it; the first round
-// also keeps the initial live count.  Rounds after the first stay at their
+// also keeps the initial live count, and opens the window where those rays'
+// steps across the box (ray_steps each) are few.  Rounds after the first stay at their
 // window only while at least a quarter of the rays ended by opacity; before the
 // second, those that have met next to none yet count too (the surface is still
 // ahead).  In a translucent volume, where rays will not end early, or in an
@@ -390,11 +398,14 @@ __global__ void clear_counters_kernel(uint32_t* counters, uint32_t first, uint32
 // before every round an empty frame went through five: the head at 512 x 512
 // (FP32, 50 samples a ray) 2,790 us, 2,410 now and 2,380 in a single round; at
 // 182 x 181 1,240, 890 and 900 us.  Frames of surfaces stay as they were.
-__global__ void round_begin_kernel(uint32_t* counters, uint32_t next_slot, uint32_t round, uint32_t window) {
+__global__ void round_begin_kernel(uint32_t* counters, uint32_t next_slot, uint32_t round, uint32_t window,
+                                   float ray_steps) {
     if (threadIdx.x != 0) return;
     if (round == 0) counters[kCntAlive0] = counters[kCntAliveA];
     const uint32_t seen = counters[kCntOpaque] + (round < 2 ? counters[kCntClear] : 0u);
-    counters[kCntLimit] = round == 0 || 4u * seen >= counters[kCntAlive0] ? window : kAllSamples;
+    const bool keep = round == 0 ? (float)counters[kCntAlive0] * ray_steps >= kWindowSamples
+                                 : 4u * seen >= counters[kCntAlive0];
+    counters[kCntLimit] = keep ? window : kAllSamples;
     counters[kCntClear] = 0;
     counters[next_slot] = 0;
     counters[kCntSamples] = 0;
@@ -643,7 +654,9 @@ insta_status enqueue_round(insta_ctx* ctx, RenderWS& ws, const RenderArgs& a, in
     const uint32_t next = 1u - cur;
     const uint32_t cur_slot = cur == 0 ? kCntAliveA : kCntAliveB;
     const uint32_t next_slot = next == 0 ? kCntAliveA : kCntAliveB;
-    hipLaunchKernelGGL(round_begin_kernel, dim3(1), dim3(64), 0, stream, cnt, next_slot, round, window);
+    const float dx = a.hi[0] - a.lo[0], dy = a.hi[1] - a.lo[1], dz = a.hi[2] - a.lo[2];
+    const float ray_steps = std::sqrt(dx * dx + dy * dy + dz * dz) / a.dt;
+    hipLaunchKernelGGL(round_begin_kernel, dim3(1), dim3(64), 0, stream, cnt, next_slot, round, window, ray_steps);
     const dim3 rgrid((max_alive + kRayThreads - 1) / kRayThreads);
     prof_begin(ctx, prof, INSTA_KERNEL_MARCH, stream);
     hipLaunchKernelGGL(far_frame(a) ? march_kernel<true> : march_kernel<false>, rgrid, dim3(kRayThreads), 0, stream, a,
@@ -652,10 +665,9 @@ insta_status enqueue_round(insta_ctx* ctx, RenderWS& ws, const RenderArgs& a, in
                        reinterpret_cast<float*>(ws.s_hit), ws.s_pos, cnt);
     INSTA_HIP(hipGetLastError());
     prof_end(ctx, prof, INSTA_KERNEL_MARCH, 0, stream);
-    // at most max_alive * K <= sample capacity samples this round (a later
-    // round's window may have been opened on the device)
-    const uint32_t n_max =
-        (uint32_t)(round == 0 ? std::min<uint64_t>(ws.samples, (uint64_t)max_alive * window) : ws.samples);
+    // at most max_alive * K <= sample capacity samples this round (windows may
+    // be opened on the device)
+    const uint32_t n_max = (uint32_t)ws.samples;
     prof_begin(ctx, prof, INSTA_KERNEL_DEFORM, stream);
     insta_status st = launch_deform_soa(ctx, ws, frame, cnt + kCntSamples, n_max, cnt + kCntMisses, cnt + kCntQueue, stream);
     if (st != INSTA_OK) return st;
