@@ -192,13 +192,15 @@ constexpr int kTravCounters = 6;
 // wave are still at it: a wave runs as long as its longest query, and a few long ones
 // (sub-cells around a mesh pole, whose lists hold hundreds of entries or
 // overflow to the BVH; points near the medial axis, which visit most leaves)
-// would otherwise set the kernel's time.  Waves of which more than kLeafWalkers
-// lanes walk the BVH (no lists: split 0, or before the occupancy is built) keep
-// walking to the last: their coherent walk is cheaper than a wave per query
-// (512 x 512 frame of the head at split 0: 2.96 ms without budgets, 3.06 so,
-// 5.9 with the few-lanes rule for them too), and lists of a coarser split are
-// longer by themselves: twice the entries per halving (split 1: 2.6 ms without
-// budgets, 2.8 so, 3.5 with the entries of split 4).  A
+// would otherwise set the kernel's time.  The leaves of few lanes count only for
+// a sub-cell whose list was too long.  Samples outside the cells that have lists
+// (split 0; an occupancy wider than the one the lists were built for, as a
+// trained density grid's) are ordinary tree walks: the second pass's wave per
+// query costs more than their tail (the head at 512 x 512, split 0: 2.96 ms
+// without budgets, 3.06 so, 5.9 with the rule for them too; marching a shell
+// twice as thick as the lists' 6.1, 6.5 and 11.3 ms).  Lists of a coarser split
+// are longer by themselves: twice the entries per halving (split 1: 2.6 ms
+// without budgets, 2.8 so, 3.5 with the entries of split 4).  A
 // 301 x 257 frame of the 9,976-triangle head (1.2 M samples): 928 us without
 // budgets, 244 + 36 us (second pass) with; its 512^2 frame 702 -> 572 + 30.
 // Giving up earlier (24 or 12 entries) or with more lanes left costs more in
@@ -208,7 +210,7 @@ constexpr int kTravCounters = 6;
 // up after a sixteenth of the tree's leaves (16 of the 2,048-triangle sphere's
 // 256: an update of 262,144 samples 412 us, with 64 953 us; the head's 1,024
 // leaves: 64, with 32 one of 1,048,576 samples 6,770 us instead of 3,300).
-constexpr uint32_t kLeafFewLanes = 16, kLeafFew = 8, kLeafLeast = 16, kLeafMost = 64, kLeafWalkers = 48;
+constexpr uint32_t kLeafFewLanes = 16, kLeafFew = 8, kLeafLeast = 16, kLeafMost = 64;
 constexpr uint32_t kListFewLanes = 4, kListFew = 72, kListMost = 192;
 
 INSTA_DEV bool few_lanes_left(uint32_t few) { return (uint32_t)__popcll(__ballot(true)) <= few; }
@@ -217,7 +219,7 @@ enum Budget { kNoBudget, kMostBudget, kFewBudget };  // kMostBudget: without the
 
 template <bool kCount, Budget kBudget = kNoBudget>
 INSTA_DEV Hit bvh_closest_impl(const MeshView& m, V3 p, uint32_t* stack, uint32_t stride, float max_dist_sq,
-                               TraversalCount* tc, bool* unfinished = nullptr) {
+                               TraversalCount* tc, bool* unfinished = nullptr, bool few = false) {
     // max_dist_sq (bvh.cuh:48): only triangles closer than this are reported
     float best = max_dist_sq;
     int32_t best_idx = -1;
@@ -226,7 +228,6 @@ INSTA_DEV Hit bvh_closest_impl(const MeshView& m, V3 p, uint32_t* stack, uint32_
     const uint32_t shift = 2u * m.k;
     [[maybe_unused]] const uint32_t most =
         kBudget == kMostBudget ? max(kLeafLeast, min(kLeafMost, (1u << shift) / 16u)) : kLeafMost;
-    [[maybe_unused]] const bool few = kBudget == kFewBudget && few_lanes_left(kLeafWalkers);
     int sp = 0;
     uint32_t node = 0, leaves = 0;
     for (;;) {
@@ -295,7 +296,7 @@ INSTA_DEV Hit bvh_closest_impl(const MeshView& m, V3 p, uint32_t* stack, uint32_
         if (node == kNoNode) break;
         if constexpr (kBudget != kNoBudget) {
             ++leaves;
-            if (leaves >= most || (few && leaves >= kLeafFew && few_lanes_left(kLeafFewLanes))) {
+            if (leaves >= most || (kBudget == kFewBudget && few && leaves >= kLeafFew && few_lanes_left(kLeafFewLanes))) {
                 *unfinished = true;
                 break;
             }
@@ -464,10 +465,11 @@ INSTA_DEV Hit list_closest_impl(const MeshView& m, const uint32_t* __restrict__ 
 template <bool kCount, Budget kBudget = kNoBudget>
 INSTA_DEV Hit closest_impl(const MeshView& m, const CellListView& cl, V3 p, uint32_t* stack, uint32_t stride,
                            TraversalCount* tc, bool* unfinished = nullptr) {
-    uint2 hd;
+    uint2 hd = make_uint2(0u, 0u);
     const bool in_box = p.x >= 0.0f && p.x <= 1.0f && p.y >= 0.0f && p.y <= 1.0f && p.z >= 0.0f && p.z <= 1.0f;
     if (in_box && cell_list_find(cl, p, hd)) return list_closest_impl<kCount, kBudget>(m, cl.ent, hd, p, cl.S, tc, unfinished);
-    return bvh_closest_impl<kCount, kBudget>(m, p, stack, stride, 3.40282347e38f, tc, unfinished);
+    // (hd.y is kNoList where the cell has lists, but this sub-cell's was too long)
+    return bvh_closest_impl<kCount, kBudget>(m, p, stack, stride, 3.40282347e38f, tc, unfinished, hd.y == kNoList);
 }
 
 INSTA_DEV Hit closest(const MeshView& m, const CellListView& cl, V3 p, uint32_t* stack, uint32_t stride) {

@@ -133,3 +133,31 @@ def test_coords_on_a_small_mesh(n):
         ctx.deform_samples(p)
         part[s] = p
     assert torch.equal(whole, part)
+
+
+@pytest.mark.parametrize("split", [0, 1, 4])
+def test_wider_occupancy_than_the_lists(split):
+    """Samples inside and outside the cells that have lists, side by side in a wave: the budgeted render against the
+    counting build's."""
+    torch = pytest.importorskip("torch")
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from insta_amd.capi import Context
+    av = synth.head_avatar(seed=1, n_frames=1)
+    cfg = full_config(max_frames=1, cell_split=split)
+    ctx = Context(cfg)
+    ctx.set_canonical_mesh(av.canonical, av.faces, av.masks)
+    ctx.set_frames(0, torch.from_numpy(np.stack(av.frames)).cuda())
+    ctx.set_params(torch.from_numpy(synth.network_params(7, ctx.layout, cfg)).cuda())
+    wide = ctx.build_occupancy(0, 0.04).clone()
+    ctx.build_occupancy(0, 0.015)
+    ctx.set_occupancy(-1, wide)
+    cam = make_camera(synth.look_at_camera(np.array([0.4, 0.7, 0.6]), 0.4), synth.focal_from_fov(200, 30.0))
+    ctx.set_profiling(True, count_traversal=True)
+    ref = [t.clone() for t in ctx.render(cam, 203, 200, 0, -1)]
+    tc = ctx.traversal_counts()
+    ctx.set_profiling(False)
+    assert tc["queries"] > tc["list_queries"] >= (1000 if split else 0)
+    got = ctx.render(cam, 203, 200, 0, -1)
+    for g, r in zip(got, ref):
+        assert np.array_equal(g.cpu().numpy(), r.cpu().numpy())
