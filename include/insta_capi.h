@@ -92,10 +92,11 @@ typedef struct insta_config {
      * largest possible nearest distance), sorted by box distance.  Queries in
      * such a sub-cell scan the list; all others traverse the BVH.  The result
      * is the same either way.  0 = BVH only, else 1, 2 or 4 (default 4).  The
-     * lists cost set-up per posed frame (512^2 head: 2.3 ms at 4, 1.4 at 2,
-     * against 0.24 for the occupancy grid alone) and repay it when a frame is
-     * rendered about three times or more; one render per pose is fastest at
-     * 0, a served request's frame at 2 */
+     * lists cost set-up per posed frame (the head: 1.0 ms at 4, 1.3 at 2,
+     * against 0.24 for the occupancy grid alone).  At 4 one 512^2 render of
+     * the pose about repays it (3.9 ms in all against 4.0 without, 3.5 against
+     * 3.3 with an opaque skin), one of 1024^2 clearly (8.8 against 10.6);
+     * smaller frames rendered once are fastest at 0 */
     uint32_t cell_split;
     uint32_t cell_list_cells;        /* occupied cells per frame that get lists (cap) */
     uint32_t cell_list_entries;      /* list entries per frame (cap; sub-cells past it use the BVH) */
